@@ -75,14 +75,11 @@ __device__ inline void load_dom(const float* dom, int model, Dom& d) {
 // reciprocal: five instructions, branch-free, exact limits (e^{2z} -> inf
 // gives 1, -> 0 gives -1).  Absolute error <= 2.5e-7; the rounding of
 // 1 - 2r near z = 0 costs relative, not absolute, accuracy.
-__device__ inline float tanh_f(float z) {
+// z s is the argument, s a power of two.
+__device__ inline float tanh_f(float z, float s = 1.f) {
   constexpr float k2log2e = 2.8853900817779268f;   // 2 / ln 2
-  const float e = __builtin_amdgcn_exp2f(z * k2log2e);
+  const float e = __builtin_amdgcn_exp2f(z * (k2log2e * s));
   return fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f);
-}
-
-__device__ inline f4 mfma16(float a, float b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 // cos and sin of a half angle |phi| <= pi/2 (no range reduction): even and

@@ -5,12 +5,28 @@
 // each wave processes 16 pairs at a time ("sub-tile").
 // Lane l handles pair (l & 15) of the sub-tile and hidden units
 //   u = 16*rb + 4*(l >> 4) + r,   rb < H/16, r < 4,
-// which is exactly the row set that lane holds in the D layout of
-// v_mfma_f32_16x16x4f32 (D[i][j]: lane = j + 16*(i/4), reg = i%4).  Because
-// the contraction index of an MFMA may be permuted freely, K-step (kb, ks)
-// feeds the B operand from register [kb][ks] (unit 16kb + 4g + ks for lane
-// group g) and the A operand with the matching weight column, so a layer's
-// output registers are directly the next layer's input registers.
+// which is exactly the row set that lane holds in the D layout of the 16x16
+// matrix instructions (D[i][j]: lane = j + 16*(i/4), reg = i%4).  Because the
+// contraction index of an MFMA may be permuted freely, a K-step of 32 takes
+// the B operand's eight values of lane group g from registers [2q][0..3] and
+// [2q + 1][0..3] (units 32q + 16b + 4g + ks) and the A operand with the
+// matching weight columns, so a layer's output registers are directly the
+// next layer's input registers.
+//
+// Hidden-layer products run on the f16 matrix cores at float32 accuracy: each
+// float32 operand is carried as x = hi + lo with hi = f16(x), lo = f16(x - hi)
+// (22 bits and the sign of the rest), and a product is hi hi + hi lo + lo hi
+// with float32 accumulation.  v_mfma_f32_16x16x32_f16 does 32 contraction
+// steps in the time the float32 instruction does two, so the three products
+// cost 3/16 of the float32 matrix time, and they leave the vector ALU free
+// (a float32 MFMA does not overlap it).  Measured on [16 x 64] x [64 x 16]
+// products of uniform weights and tanh values against float64: relative
+// 2-norm error 8.7e-8, against 1.44e-7 for the float32 instruction's chain of
+// fused multiply-adds.  f16 has a narrow exponent range, so everything that is
+// not bounded by 1 is scaled by powers of two chosen per chunk (Scales):
+// weights by their largest value, tangents by theirs, gradients by a bound
+// formed from the chunk's upstream gradients; the inverse factors are exact
+// and ride on per-pair scalars.
 //
 // Reference math (per pair, trainers.py:113-118 with the tangents that the
 // nested jvp of trainers.py:213-247 pushes through):
@@ -24,8 +40,7 @@
 // zt_i = W1[:, i] / sd_i (per subdomain), a1_0 = h, a1_i = d1 zt_i and
 // a1_ii = d2 zt_i^2, so the B operand of every layer-2 MFMA is rebuilt from h
 // with one or two multiplies.  Layer 2 is evaluated one axis at a time (Z_0,
-// then Z_i and Z_ii per axis), which keeps 3 x H/4 accumulators live instead
-// of J x H/4.
+// then Z_i per axis).
 #pragma once
 
 #include "fbpx_common.hpp"
@@ -99,62 +114,140 @@ __device__ inline void stage_small(const float* th, float* ss) {
     ss[i] = th[i < SM::B2 ? i : (i < SM::WL ? L::B2 + (i - SM::B2) : L::WL + (i - SM::WL))];
 }
 
-// Lane-major LDS fragments of W2: the MFMA A operands of one K-step for all
-// 64 lanes, NRB = H/16 contiguous floats per lane (one ds_read_b128 at
-// H = 64).  With lane l = 16g + pl and K-step q:
-//   wt[(q*64 + l)*NRB + ob] = W2[16ob + pl][16kb + 4g + ks],        q = 4kb + ks
-//     (A of W2 . b: rows o = 16ob + pl, contraction units 16kb + 4g + ks)
-//   wr[(q*64 + l)*NRB + ib] = c_o W2[o][16ib + pl], o = 16ob + 4g + ks, q = 4ob + ks
-//     (A of (diag(c) W2)^T . g), c = WL (the backward carries G / WL, see
-//     bwd_two) or 1 when wl is null.
-// Consecutive lanes read consecutive 16-byte slots: conflict-free.
-template <int H>
-__device__ inline void stage_w2(const float* w2, const float* wl, float* wt, float* wr) {
-  constexpr int NRB = H / 16;
-  for (int t = threadIdx.x; t < 4 * NRB * 64; t += blockDim.x) {
-    const int q = t >> 6, l = t & 63, g = l >> 4, pl = l & 15;
-    const int kb = q >> 2, ks = q & 3;
-    const int k = 16 * kb + 4 * g + ks;   // contraction unit (wt) / row o (wr)
-    float a[NRB], c[NRB];
-    const float cw = (wr && wl) ? wl[k] : 1.f;
-#pragma unroll
-    for (int j = 0; j < NRB; ++j) {
-      if (wt) a[j] = w2[(16 * j + pl) * H + k];
-      if (wr) c[j] = w2[k * H + 16 * j + pl] * cw;
-    }
-#pragma unroll
-    for (int j = 0; j < NRB; ++j) {
-      if (wt) wt[t * NRB + j] = a[j];
-      if (wr) wr[t * NRB + j] = c[j];
-    }
-  }
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+
+// x0, x1 -> packed (hi, hi) and (lo, lo), x = hi + lo (both rounded to
+// nearest).  one: 1.f in a scalar register the optimiser cannot see through,
+// so that x - hi is one v_fma_mix_f32 on the packed half; the empty asm keeps
+// the packed conversion from being redone per element.
+__device__ inline void split2(float x0, float x1, float one, uint32_t& hi, uint32_t& lo) {
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2v{x0, x1}, h2v));
+  asm("" : "+v"(hi));
+  const h2v h = __builtin_bit_cast(h2v, hi);
+  const f2v r = {fmaf(x0, one, -(float)h[0]), fmaf(x1, one, -(float)h[1])};
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, h2v));
 }
 
-// One K-step of lane-major fragments (see stage_w2).
-template <int NRB>
-struct Frag {
-  float v[NRB];
+__device__ inline float opaque_one() {
+  float one = 1.f;
+  asm("" : "+s"(one));
+  return one;
+}
+
+// A lane's H/16 x 4 values of one pair as two f16 halves: hi[2 rb + c] packs
+// units 16 rb + 4 g + 2c and + 2c + 1.  b(q): the B operand of K-step q
+// (H >= 32: blocks 2q and 2q + 1; H = 16: one block, hi twice).
+template <int H>
+struct Split {
+  static constexpr int NRB = H / 16;
+  uint32_t hi[2 * NRB], lo[2 * NRB];
+  template <class V>
+  __device__ void set(const V& v, float one) {
+#pragma unroll
+    for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) split2(v[rb][2 * c], v[rb][2 * c + 1], one, hi[2 * rb + c], lo[2 * rb + c]);
+  }
+  __device__ h8v b(const uint32_t* p, int q) const {
+    return __builtin_bit_cast(h8v, u4v{p[(4 * q) % (2 * NRB)], p[(4 * q + 1) % (2 * NRB)],
+                                       p[(4 * q + 2) % (2 * NRB)], p[(4 * q + 3) % (2 * NRB)]});
+  }
 };
 
-template <int NRB>
-__device__ inline Frag<NRB> ld_frag(const float* p) {
-  Frag<NRB> f;
-  if constexpr (NRB == 4) {
-    const f4 t = *reinterpret_cast<const f4*>(p);
-    f.v[0] = t[0];
-    f.v[1] = t[1];
-    f.v[2] = t[2];
-    f.v[3] = t[3];
-  } else if constexpr (NRB == 2) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    const f2 t = *reinterpret_cast<const f2*>(p);
-    f.v[0] = t[0];
-    f.v[1] = t[1];
-  } else {
-    f.v[0] = p[0];
-  }
-  return f;
+__device__ inline f4 mfma_k32(h8v a, h8v b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+// 2^e with m 2^e <= 2^top (within a factor of two below it), e within
+// [-100, lim]: the clamp keeps the inverse and products of factors finite and
+// is what m = 0 and m = inf take.
+__device__ inline float pow2_scale(float m, int top, int lim) {
+  int e = top + 126 - (int)((__builtin_bit_cast(uint32_t, m) >> 23) & 255u);
+  e = e < -100 ? -100 : (e > lim ? lim : e);
+  return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
 }
+__device__ inline float pow2_inv(float s) {   // 1 / s for s = 2^e, |e| < 127
+  return __builtin_bit_cast(float, (uint32_t)(254u << 23) - __builtin_bit_cast(uint32_t, s));
+}
+// the same value in every lane, as a scalar
+__device__ inline float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+// Powers of two of one chunk (all exact):
+//   W2 2^w and (diag(WL) W2) 2^r are at most 2^14 in LDS,
+//   zt_i 2^e[i] is at most 4 (table ztS),
+//   the upstream gradients are carried times 2^k (backward).
+template <int XD>
+struct Scales {
+  float w, iw, r, ir, e[XD], ie[XD], k, ik;
+};
+
+// Lane-major LDS fragments of W2 (f16 hi / lo): the MFMA A operands of one
+// K-step q and 16-row block ob for all 64 lanes.  With lane l = 16g + pl,
+// H >= 32: fragment f = (q NRB + ob) 2 + piece holds 8 halves per lane,
+//   wt: W2[16ob + pl][k] 2^w, k = 32q + 16b + 4g + ks at 4b + ks
+//   wr: (WL_k W2[k][16ob + pl]) 2^r, same k         (A of (diag(WL) W2)^T . g)
+// H = 16: one fragment, 4 hi then 4 lo halves per lane (k = 4g + ks).
+// Consecutive lanes read consecutive 16-byte slots: conflict-free.
+template <int H>
+struct W2Frags {
+  static constexpr int NRB = H / 16;
+  static constexpr int NQ = H >= 32 ? H / 32 : 1;
+  static constexpr int NEL = H >= 32 ? 8 : 4;         // weights per item
+  static constexpr int ITEMS = NQ * NRB * 64;
+  static constexpr int IT = (ITEMS + 255) / 256;      // items per thread of a 256-thread workgroup
+  static constexpr int WORDS = H * H;                 // 32-bit words of one set (hi and lo)
+  float a[IT][NEL], c[IT][NEL];
+  __device__ static int unit(int q, int g, int j) { return 32 * q + 16 * (j >> 2) + 4 * g + (j & 3); }
+  template <bool WT, bool WR>
+  __device__ void load(const float* w2, const float* wl) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = (int)threadIdx.x + 256 * it, l = t & 63, g = l >> 4, pl = l & 15, f = t >> 6;
+      const int q = f / NRB, ob = f % NRB;
+      if (t >= ITEMS) continue;
+#pragma unroll
+      for (int j = 0; j < NEL; ++j) {
+        const int k = unit(q, g, j);
+        if (WT) a[it][j] = w2[(16 * ob + pl) * H + k];
+        if (WR) c[it][j] = w2[k * H + 16 * ob + pl] * wl[k];
+      }
+    }
+  }
+  // this thread's largest |value|.  (An infinite or NaN weight makes its
+  // subdomain's values NaN: hi + lo of an infinity is inf - inf.)
+  __device__ static float largest(const float (*v)[NEL]) {
+    float m = 0.f;
+#pragma unroll
+    for (int it = 0; it < IT; ++it)
+      if ((int)threadIdx.x + 256 * it < ITEMS) {
+#pragma unroll
+        for (int j = 0; j < NEL; ++j) m = fmaxf(m, fabsf(v[it][j]));
+      }
+    return m;
+  }
+  __device__ static void store(const float (*v)[NEL], float scale, float one, float* dst) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = (int)threadIdx.x + 256 * it, l = t & 63, f = t >> 6;
+      if (t >= ITEMS) continue;
+      uint32_t hi[NEL / 2], lo[NEL / 2];
+#pragma unroll
+      for (int c = 0; c < NEL / 2; ++c) split2(v[it][2 * c] * scale, v[it][2 * c + 1] * scale, one, hi[c], lo[c]);
+      uint32_t* w = reinterpret_cast<uint32_t*>(dst);
+      if constexpr (H >= 32) {
+        *reinterpret_cast<u4v*>(w + (2 * f * 64 + l) * 4) = u4v{hi[0], hi[1], hi[2], hi[3]};
+        *reinterpret_cast<u4v*>(w + ((2 * f + 1) * 64 + l) * 4) = u4v{lo[0], lo[1], lo[2], lo[3]};
+      } else {
+        *reinterpret_cast<u4v*>(w + l * 4) = u4v{hi[0], hi[1], lo[0], lo[1]};
+      }
+    }
+  }
+};
 
 // Sum over the four 16-lane rows (lane groups g) for every pl, in registers:
 // v_permlane32_swap exchanges the upper half of its first operand with the
@@ -176,6 +269,16 @@ __device__ inline float sum_groups(float v) {
 template <int CTRL>
 __device__ inline float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
+// Largest of v over the wave, in every lane (v >= 0).
+__device__ inline float max_wave(float v) {
+  v = fmaxf(v, dpp<0x140>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  v = fmaxf(v, dpp<0x1B>(v));
+  v = fmaxf(v, dpp<0xB1>(v));
+  v = fmaxf(v, __shfl_xor(v, 16));
+  return fmaxf(v, __shfl_xor(v, 32));
 }
 
 // One reduce-scatter stage over a DPP row: lanes whose stage bit is set keep
@@ -296,10 +399,9 @@ __device__ inline float tanh_d3(float h) {
   return -2.f * (d1 * d1 - 2.f * h * h * d1);
 }
 
-// Per-subdomain layer-1 tangent tables in LDS (4 * XD * H floats): with
-// zt_i[u] = W1[u][i] / sd_i,
-//   zt[i*H + u] = zt_i[u],  zt[XD*H + i*H + u] = -2 zt_i[u],
-//   zt[2*XD*H + i*H + u] = -2 zt_i[u]^2,  zt[3*XD*H + i*H + u] = zt_i[u]^2.
+// Per-subdomain layer-1 tangent tables in LDS: with zt_i[u] = W1[u][i] / sd_i,
+//   zt[i*H + u] = zt_i[u],  zt[XD*H + i*H + u] = zt_i[u]^2;
+// a third table zt_i[u] 2^e[i] follows them with two hidden layers (stage_two).
 template <int XD, int H, class SM, bool WAVE = false>
 __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
   for (int t = Team<WAVE>::tid(); t < XD * H; t += Team<WAVE>::size()) {
@@ -310,9 +412,7 @@ __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
       if (i == j) s = isd[j];
     const float z = ss[SM::W1 + u * XD + i] * s;
     zt[t] = z;
-    zt[XD * H + t] = -2.f * z;
-    zt[2 * XD * H + t] = -2.f * z * z;
-    zt[3 * XD * H + t] = z * z;
+    zt[XD * H + t] = z * z;
   }
 }
 
@@ -323,16 +423,15 @@ __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
 //   w1  = ss + W1 + 4g*XD      W1[16rb + 4g + r][i]        at [(16rb + r)*XD + i]
 //   vec = ss + 4g              B1/B2/WL[16rb + 4g + r]     at [off + 16rb + r]
 //   zt  = szt + 4g             zt[i][16rb + 4g + r]        at [i*H + 16rb + r]
-//   zm, zq, z2: the -2 zt, -2 zt^2 and zt^2 tables, same indexing
-//   wt  = swt + lane*NRB       K-step q of the W2 fragments at [q*64*NRB]
-//   wr  = swr + lane*NRB       K-step q of the transposed fragments, same
+//   z2, zs: the zt^2 and zt 2^e tables, same indexing
+//   wt  = swt + lane*4         fragment f of W2 (W2Frags) at [f*256]
+//   wr  = swr + lane*4         fragment f of the transposed set, same
 struct LaneLds {
   const float* w1;
   const float* vec;
   const float* zt;
-  const float* zm;
-  const float* zq;
   const float* z2;
+  const float* zs;
   const float* wt;
   const float* wr;
 };
@@ -344,37 +443,67 @@ __device__ inline LaneLds lane_lds(const float* ss, const float* szt, const floa
   v.w1 = ss + SM::W1 + 4 * g * XD;
   v.vec = ss + 4 * g;
   v.zt = szt + 4 * g;
-  v.zm = szt + XD * H + 4 * g;
-  v.zq = szt + 2 * XD * H + 4 * g;
-  v.z2 = szt + 3 * XD * H + 4 * g;
-  v.wt = swt + (16 * g + pl) * (H / 16);
-  v.wr = swr + (16 * g + pl) * (H / 16);
+  v.z2 = szt + XD * H + 4 * g;
+  v.zs = szt + 2 * XD * H + 4 * g;
+  v.wt = swt + (16 * g + pl) * 4;
+  v.wr = swr + (16 * g + pl) * 4;
   return v;
 }
 
-// Z[ob] += sum over K-steps q of the fragment A operands (LDS, lane-major,
-// K-step q at frag + q*64*NRB) times B[q >> 2][q & 3] (registers).  A
-// scheduling region of its own in which each fragment is read two K-steps
-// ahead of the MFMAs that use it (group barriers: two reads, then per
-// K-step its NRB MFMAs and the next read), so the LDS latency is hidden
-// behind MFMAs instead of stalling each K-step.
-template <int H, class BOp>
-__device__ inline void frag_pass(const float* frag, BOp b, f4* Z) {
-  constexpr int NRB = H / 16, NQ = 4 * NRB;
-  __builtin_amdgcn_sched_barrier(0);
+// Z[ob] += fragments (LDS, see W2Frags) times the split B operand.  The two
+// small products of every K-step are accumulated before the large ones, whose
+// rounding then happens once per K-step: 8.7e-8 relative error at H = 64
+// where one K-step after the other gives about 1e-7.
+template <int H>
+__device__ inline void frag_pass(const float* frag, const Split<H>& b, f4* Z) {
+  using F = W2Frags<H>;
+  constexpr int NRB = H / 16;
+  if constexpr (H >= 32) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const Frag<NRB> w = ld_frag<NRB>(frag + q * 64 * NRB);
+    for (int ob = 0; ob < NRB; ++ob) {
+      h8v hi[F::NQ], lo[F::NQ];
 #pragma unroll
-    for (int ob = 0; ob < NRB; ++ob) Z[ob] = mfma16(w.v[ob], b[q >> 2][q & 3], Z[ob]);
+      for (int q = 0; q < F::NQ; ++q) {
+        hi[q] = *reinterpret_cast<const h8v*>(frag + (q * NRB + ob) * 512);
+        lo[q] = *reinterpret_cast<const h8v*>(frag + (q * NRB + ob) * 512 + 256);
+      }
+#pragma unroll
+      for (int q = 0; q < F::NQ; ++q) {
+        Z[ob] = mfma_k32(lo[q], b.b(b.hi, q), Z[ob]);
+        Z[ob] = mfma_k32(hi[q], b.b(b.lo, q), Z[ob]);
+      }
+#pragma unroll
+      for (int q = 0; q < F::NQ; ++q) Z[ob] = mfma_k32(hi[q], b.b(b.hi, q), Z[ob]);
+    }
+    // the reads of the next row block go between this block's MFMAs
+    constexpr int NR = 2 * F::NQ, NM = 3 * F::NQ;
+    __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
+#pragma unroll
+    for (int ob = 0; ob + 1 < NRB; ++ob) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+    // one K-step of 16: hi and lo weights side by side in a K of 32 against
+    // lo twice (which adds the lo lo product) and hi twice
+    const h8v w = *reinterpret_cast<const h8v*>(frag);
+    Z[0] = mfma_k32(w, b.b(b.lo, 0), Z[0]);
+    Z[0] = mfma_k32(w, b.b(b.hi, 0), Z[0]);
   }
-  __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+}
+
+template <int H>
+__device__ inline void frag_mul(const float* frag, const Split<H>& b, f4* Z) {
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    __builtin_amdgcn_sched_group_barrier(0x008, NRB, 0);
-    if (q + 2 < NQ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-  }
-  __builtin_amdgcn_sched_barrier(0);
+  for (int ob = 0; ob < H / 16; ++ob) Z[ob] = f4{0.f, 0.f, 0.f, 0.f};
+  frag_pass<H>(frag, b, Z);
 }
 
 // Layer 1 for this lane's units (rows 16rb + 4g + r): h = tanh(W1 xh + b1).
@@ -392,56 +521,37 @@ __device__ inline void layer1_stream(const LaneLds& v, const float* xh, float (*
   }
 }
 
-// One layer-2 MFMA pass: Z[ob] (+)= W2 . B with B[kb][ks] = base * scale.
-// kind 0: B = h (Z initialised with b2), 1: B = d1 zt_i, 2: B = d2 zt_i^2,
-// 3: B = base zt_i with base = d1 supplied in place of h;
-// zrow = i * H selects the zt row of axis i.
+// Z_0 2^w = (W2 h1 + b2) 2^w.
 template <int H, class SM>
-__device__ inline void layer2_pass(const LaneLds& v, const float (*h1)[4], int zrow, int kind, f4* Z) {
-  constexpr int NRB = H / 16;
-  float bv[NRB][4];
+__device__ inline void layer2_value(const LaneLds& v, const float (*h1)[4], float sw, float one, f4* Z) {
 #pragma unroll
-  for (int kb = 0; kb < NRB; ++kb)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float h = h1[kb][ks];
-      float b = h;
-      if (kind == 1) {
-        b = fmaf(-h, h, 1.f) * v.zt[zrow + 16 * kb + ks];            // d1 zt
-      } else if (kind == 2) {
-        b = (h * fmaf(-h, h, 1.f)) * v.zq[zrow + 16 * kb + ks];      // d2 zt^2 = h d1 (-2 zt^2)
-      } else if (kind == 3) {
-        b = h * v.zt[zrow + 16 * kb + ks];                           // (given d1) zt
-      }
-      bv[kb][ks] = b;
-    }
-#pragma unroll
-  for (int ob = 0; ob < NRB; ++ob) {
-    if (kind == 0) {
-      const float* b2 = v.vec + SM::B2 + 16 * ob;
-      Z[ob] = f4{b2[0], b2[1], b2[2], b2[3]};
-    } else {
-      Z[ob] = f4{0.f, 0.f, 0.f, 0.f};
-    }
+  for (int ob = 0; ob < H / 16; ++ob) {
+    const float* b2 = v.vec + SM::B2 + 16 * ob;
+    Z[ob] = f4{b2[0] * sw, b2[1] * sw, b2[2] * sw, b2[3] * sw};
   }
-  frag_pass<H>(v.wt, bv, Z);
+  Split<H> b;
+  b.set(h1, one);
+  frag_pass<H>(v.wt, b, Z);
 }
 
-// One layer-2 MFMA pass with the B operand given in registers (no bias):
-// Z[ob] = W2 . b, b[kb][ks] the value for unit 16kb + 4g + ks of this lane's pair.
+// a[rb][r] zs[zrow + ...]: the B operand e1 zt_i 2^e[i] of axis i (zrow = i H).
 template <int H>
-__device__ inline void layer2_pass_raw(const LaneLds& v, const float (*b)[4], f4* Z) {
+__device__ inline void tangent_split(const LaneLds& v, const float (*e1)[4], int zrow, float one, Split<H>& b) {
+  float t[H / 16][4];
 #pragma unroll
-  for (int ob = 0; ob < H / 16; ++ob) Z[ob] = f4{0.f, 0.f, 0.f, 0.f};
-  frag_pass<H>(v.wt, b, Z);
+  for (int rb = 0; rb < H / 16; ++rb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[rb][r] = e1[rb][r] * v.zs[zrow + 16 * rb + r];
+  b.set(t, one);
 }
 
 // The pair's layer-1 combination of every tangent the upstream gradient
 // asks for, s = sum_i (gur_i a1_i + gur_ii a1_ii) with a1_i = e1 zt_i and
 // a1_ii = e2 zt_i^2 (e1 = 1 - h1^2, e2 = -2 h1 e1, e3 = e1 (4 - 6 e1)):
 //   s = e1 (A - 2 h1 B),  A = sum_i gur_i zt_i,  B = sum_i gur_ii zt_i^2,
-// and the factor that the W2^T vector vt multiplies in the layer-1 gradient,
-//   rv = e2 A + e3 B = e1 (-2 h1 A + (4 - 6 e1) B).
+// and -1/2 times the factor that the W2^T vector vt multiplies in the layer-1
+// gradient,
+//   e2 A + e3 B = -2 rv,  rv = e1 (h1 A + (3 e1 - 2) B).
 template <class S, int H>
 __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const float* gur, float (*sv)[4],
                               float (*rv)[4]) {
@@ -458,8 +568,114 @@ __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const floa
       const float h = h1[rb][r];
       const float e1 = fmaf(-h, h, 1.f);
       sv[rb][r] = e1 * fmaf(-2.f * h, B, A);
-      rv[rb][r] = e1 * fmaf(h * A, -2.f, fmaf(-6.f, e1, 4.f) * B);
+      rv[rb][r] = e1 * fmaf(h, A, fmaf(3.f, e1, -2.f) * B);
     }
+}
+
+// Stages one subdomain of a two-hidden-layer network in LDS: the small
+// parameters, the tangent tables and the f16 fragments of W2 (and with WR of
+// diag(WL) W2), and forms the chunk's scales.  With BWD, gm[c] is this
+// thread's largest |upstream gradient| of jet column c over its share of the
+// chunk's pairs, and the gradients' scale k is chosen from a bound on every
+// gradient value that enters a product: with R the largest absolute row sum
+// of W2, ZB_i = max_o sum_u |W2[o][u] zt_i[u]| >= |Z_i|, ZT_i = max |zt_i| and
+// g the bound on gur (window jets |w| <= 1, |w_i| <= 0.65 k_i, |w_ii| <= k_i^2
+// with k_i = pi / sd_i; |2 h e1|, |f2| <= 0.77, |f3| <= 2):
+//   |s| <= bS = sum_i g_i ZT_i + 0.77 g_ii ZT_i^2,
+//   |G_i| 2^-e[i] <= 0.77 g_ii ZB_i ZT_i,  |G_0| <= g_0 + 0.77 R bS + 2 sum_i g_ii ZB_i^2.
+// Typical values lie 2^-8 to 2^-12 below the bound; the f16 pairs hold 22
+// bits down to 2^-17 below it and 2^-40 of the bound absolutely after that.
+// All threads of the workgroup; ends with a barrier.
+template <class S, int H, class SM, bool WR, bool BWD>
+__device__ inline void stage_two(const float* th, const Dom& d, const float* isd, const float* gm, float one,
+                                 float* ss, float* szt, float* swt, float* swr, float* red, Scales<S::XD>& sc) {
+  constexpr int XD = S::XD, J = S::J;
+  using L = Layout<XD, H, 2>;
+  using F = W2Frags<H>;
+  constexpr int RW = 0, RR = 1, RS = 2, RZ = 3, RG = RZ + XD, NR = BWD ? RG + J : 2;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  F f;
+  stage_small<XD, H, 2>(th, ss);
+  f.template load<true, WR>(th + L::W2, th + L::WL);
+  __syncthreads();
+  stage_zt<XD, H, SM>(ss, isd, szt);
+  __syncthreads();
+  float zmax[XD];
+#pragma unroll
+  for (int i = 0; i < XD; ++i) zmax[i] = max_wave(fabsf(szt[i * H + lane % H]));
+  float m[NR];
+  m[RW] = F::largest(f.a);
+  m[RR] = WR ? F::largest(f.c) : 0.f;
+  if constexpr (BWD) {
+    // row sums: a wave's items are all of one 16-row block, row 16ob + pl of
+    // lane pl, so adding the lane groups completes them
+    float rs = 0.f, zb[XD];
+#pragma unroll
+    for (int i = 0; i < XD; ++i) zb[i] = 0.f;
+#pragma unroll
+    for (int it = 0; it < F::IT; ++it)
+      if ((int)threadIdx.x + 256 * it < F::ITEMS) {
+#pragma unroll
+        for (int j = 0; j < F::NEL; ++j) {
+          const int k = F::unit(it, lane >> 4, j);
+          const float a = fabsf(f.a[it][j]);
+          rs += a;
+#pragma unroll
+          for (int i = 0; i < XD; ++i) zb[i] = fmaf(a, fabsf(szt[i * H + k]), zb[i]);
+        }
+      }
+    m[RS] = sum_groups(rs);
+#pragma unroll
+    for (int i = 0; i < XD; ++i) m[RZ + i] = sum_groups(zb[i]);
+#pragma unroll
+    for (int c = 0; c < J; ++c) m[RG + c] = gm[c];
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const float v = max_wave(m[i]);
+    if (lane == 0) red[wave * 16 + i] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    m[i] = uniform(fmaxf(fmaxf(red[i], red[16 + i]), fmaxf(red[32 + i], red[48 + i])));
+  sc.w = pow2_scale(m[RW], 14, 40);
+  sc.iw = pow2_inv(sc.w);
+  sc.r = WR ? pow2_scale(m[RR], 14, 40) : 1.f;
+  sc.ir = pow2_inv(sc.r);
+#pragma unroll
+  for (int i = 0; i < XD; ++i) {
+    sc.e[i] = uniform(pow2_scale(zmax[i], 2, 40));
+    sc.ie[i] = pow2_inv(sc.e[i]);
+  }
+  sc.k = sc.ik = 1.f;
+  if constexpr (BWD) {
+    const float us = fabsf(d.usd);
+    float g0 = m[RG], bS = 0.f, q = 0.f, b = 0.f;
+#pragma unroll
+    for (int i = 0; i < XD; ++i) {
+      if (!S::has1(i)) continue;
+      const float k = kPi * fabsf(isd[i]);
+      const float ga = m[RG + S::col1(i)], gb = S::has2(i) ? m[RG + S::col2(i)] : 0.f;
+      g0 = fmaf(0.65f * k, ga, fmaf(k * k, gb, g0));
+      bS = fmaf(us * fmaf(1.3f * k, gb, ga), zmax[i], fmaf(0.77f * us * gb, zmax[i] * zmax[i], bS));
+      q = fmaf(2.f * us * gb, m[RZ + i] * m[RZ + i], q);
+      b = fmaxf(b, 0.77f * us * gb * m[RZ + i] * zmax[i]);
+    }
+    b = fmaxf(fmaxf(b, bS), fmaf(us, g0, fmaf(0.77f * m[RS], bS, q)));
+    sc.k = uniform(pow2_scale(b, 15, 100));
+    sc.ik = pow2_inv(sc.k);
+  }
+  for (int t = threadIdx.x; t < XD * H; t += blockDim.x) {
+    float e = sc.e[0];
+#pragma unroll
+    for (int j = 1; j < XD; ++j)
+      if (t / H == j) e = sc.e[j];
+    szt[2 * XD * H + t] = szt[t] * e;
+  }
+  F::store(f.a, sc.w, one, swt);
+  if constexpr (WR) F::store(f.c, sc.r, one, swr);
+  __syncthreads();
 }
 
 // ------------------------------------------------------------------ forward
@@ -476,9 +692,10 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   static_assert(!WAVE || NH == 1, "one wave per chunk: one-hidden-layer networks");
   constexpr int J = S::J, NRB = H / 16, NT = WAVE ? 4 : 1;
   __shared__ float ss_[NT][SM::N];
-  __shared__ float szt_[NT][4 * XD * H];
+  __shared__ float szt_[NT][(NH == 2 ? 3 : 2) * XD * H];
   __shared__ __attribute__((aligned(16))) float swt[NH == 2 ? H * H : 1];
   __shared__ __attribute__((aligned(16))) float swr[NH == 2 && S::N1 > 0 ? H * H : 1];
+  __shared__ float red[64];
   float* const ss = ss_[T::index()];
   float* const szt = szt_[T::index()];
 
@@ -503,9 +720,6 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
 #pragma unroll
     for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
     st.store(ss);
-  } else {
-    stage_small<XD, H, NH, WAVE>(th, ss);
-    stage_w2<H>(th + L::W2, nullptr, swt, S::N1 > 0 ? swr : nullptr);
   }
   Dom d;
   load_dom(dom, model, d);
@@ -515,9 +729,15 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
     mu[i] = (d.xmax[i] + d.xmin[i]) / 2.f;
     isd[i] = 1.f / ((d.xmax[i] - d.xmin[i]) / 2.f);
   }
-  T::sync();
-  stage_zt<XD, H, SM, WAVE>(ss, isd, szt);
-  T::sync();
+  const float one = opaque_one();
+  Scales<XD> sc;
+  if constexpr (NH == 1) {
+    T::sync();
+    stage_zt<XD, H, SM, WAVE>(ss, isd, szt);
+    T::sync();
+  } else {
+    stage_two<S, H, SM, (S::N1 > 0), false>(th, d, isd, nullptr, one, ss, szt, swt, swr, red, sc);
+  }
 
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
   if constexpr (NH == 2) {
@@ -561,37 +781,39 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
         }
     } else {
       f4 Z0[NRB];
-      layer2_pass<H, SM>(v, h1, 0, 0, Z0);
+      layer2_value<H, SM>(v, h1, sc.w, one, Z0);
       // output-layer weights times the layer-2 tanh derivatives, per element:
       // wd1 = WL f1 and wd2 = WL f1 h2 = WL f2 / (-2), so that u_i = sum wd1 Z_i
       // and the Z_i^2 part of u_ii = sum WL (f1 Z_ii + f2 Z_i^2) costs two FMAs;
       // every second-derivative column is accumulated without its factor -2,
       // which is applied once to the pair's totals
-      float wd1[NRB][4], wd2[NRB][4];
+      float f1[NRB][4], wd1[NRB][4], wd2[NRB][4];
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float wlu = v.vec[SM::WL + 16 * ob + r];
-          const float h = tanh_f(Z0[ob][r]);
+          const float h = tanh_f(Z0[ob][r], sc.iw);
           ur[0] = fmaf(wlu, h, ur[0]);
-          wd1[ob][r] = wlu * fmaf(-h, h, 1.f);
+          f1[ob][r] = fmaf(-h, h, 1.f);
+          wd1[ob][r] = wlu * f1[ob][r];
           wd2[ob][r] = wd1[ob][r] * h;
         }
 #pragma unroll
       for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
       __builtin_amdgcn_sched_barrier(0);
-      // sum_o WL f1 Z_c = sum_u vt[u] a1_c[u] with vt = W2^T (WL f1): one
-      // W2^T pass per sub-tile replaces the Z_ii passes of every axis and the
-      // Z_i passes of axes without a second derivative.  With e1 = 1 - h1^2,
+      // sum_o WL f1 Z_c = sum_u vt[u] a1_c[u] with vt = (diag(WL) W2)^T f1: one
+      // transposed pass per sub-tile replaces the Z_ii passes of every axis and
+      // the Z_i passes of axes without a second derivative.  With e1 = 1 - h1^2,
       // a1_i = e1 zt_i and a1_ii = -2 h1 e1 zt_i^2, so the per-axis dot
       // products take ve = vt e1 (first order) and w = vt e1 h1 (second order).
+      // Scales: vt 2^r, Z_i 2^(w + e[i]), taken off the pair's sums.
       float e1[NRB][4], ve[NRB][4], w[NRB][4];
       if constexpr (S::N1 > 0) {
         f4 vt[NRB];
-#pragma unroll
-        for (int ib = 0; ib < NRB; ++ib) vt[ib] = f4{0.f, 0.f, 0.f, 0.f};
-        frag_pass<H>(v.wr, wd1, vt);
+        Split<H> b;
+        b.set(f1, one);
+        frag_mul<H>(v.wr, b, vt);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
@@ -608,27 +830,37 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
         if (!S::has1(i)) continue;
         if (!S::has2(i)) {
           // u_i = sum_u vt[u] e1[u] zt_i[u]
+          float q = 0.f;
 #pragma unroll
           for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) ur[S::col1(i)] = fmaf(ve[rb][r], v.zt[i * H + 16 * rb + r], ur[S::col1(i)]);
+            for (int r = 0; r < 4; ++r) q = fmaf(ve[rb][r], v.zt[i * H + 16 * rb + r], q);
+          ur[S::col1(i)] = q * sc.ir;
           continue;
         }
         f4 Zi[NRB];
-        layer2_pass<H, SM>(v, e1, i * H, 3, Zi);
+        {
+          Split<H> b;
+          tangent_split<H>(v, e1, i * H, one, b);
+          frag_mul<H>(v.wt, b, Zi);
+        }
+        const float iz = sc.iw * sc.ie[i];
+        float q1 = 0.f, q2 = 0.f, q3 = 0.f;
 #pragma unroll
         for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float zi = Zi[ob][r];
-            ur[S::col1(i)] = fmaf(wd1[ob][r], zi, ur[S::col1(i)]);
-            ur[S::col2(i)] = fmaf(wd2[ob][r] * zi, zi, ur[S::col2(i)]);
+            q1 = fmaf(wd1[ob][r], zi, q1);
+            q2 = fmaf(wd2[ob][r] * zi, zi, q2);
           }
         // + sum_u vt[u] h1 e1 zt_i^2 (the a1_ii column, factor -2 deferred)
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) ur[S::col2(i)] = fmaf(w[rb][r], v.z2[i * H + 16 * rb + r], ur[S::col2(i)]);
+          for (int r = 0; r < 4; ++r) q3 = fmaf(w[rb][r], v.z2[i * H + 16 * rb + r], q3);
+        ur[S::col1(i)] = q1 * iz;
+        ur[S::col2(i)] = fmaf(q2 * iz, iz, q3 * sc.ir);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -773,7 +1005,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   __shared__ float sacc_[NT][L::P];
   __shared__ float ssmall_[4 * NS * H];   // per wave (four teams of one wave with WAVE)
   __shared__ float sbl_[64];
-  __shared__ float szt_[NT][4 * XD * H];
+  __shared__ float szt_[NT][2 * XD * H];
   float* const ss = ss_[T::index()];
   float* const sacc = sacc_[T::index()];
   float* const szt = szt_[T::index()];
@@ -816,7 +1048,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   stage_zt<XD, H, SM, WAVE>(ss, isd, szt);
   T::sync();
 
-  const LaneLds v = lane_lds<XD, H, SM>(ss, szt, szt, szt, pl, g);
+  const LaneLds v = lane_lds<XD, H, SM>(ss, szt, ss, ss, pl, g);
   float* mysmall = ssmall + wave * NS * H;
   float dbl = 0.f;
   for (int base = beg + wave * 16; base < end; base += nw * 16) {
@@ -899,31 +1131,17 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   finish_row<XD, H, 1, WAVE, ADAM>(sacc, ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs, af, model, bc);
 }
 
-// W2^T G for one sub-tile: GA[ib] (A operand W2^T[i = 16ib+pl][o = 16ob+4g+ks]
-// from the padded row-major copy wr; B operand = G in D layout).
-template <int H>
-__device__ inline void w2t_pass(const LaneLds& v, const f4* G, f4* GA) {
-#pragma unroll
-  for (int ib = 0; ib < H / 16; ++ib) GA[ib] = f4{0.f, 0.f, 0.f, 0.f};
-  frag_pass<H>(v.wr, G, GA);
-}
-
-// Workgroup-shared dW2 accumulation.  The 4 waves of a workgroup process
-// sub-tiles in lockstep (64 pairs per tile) and write two transposes to LDS:
-//   stb[rb*BS + w*WS + (p >> 2)*PG + (p & 3)*16 + s] = layer-1 h of unit 16rb+s,
-//                                                      pair p of wave w
-//   stg[ob*BS + ...same...]                          = G_c of unit 16ob+s
-// For h <= 32 each group of 4 pairs is padded from 64 to PG = 68 floats, so
-// the 16 lanes of a 128-bit store phase (pairs 0..15, 16 bytes each) start
-// in 16 distinct 4-bank groups instead of sharing 4 of them; a read (one pair
-// group, 64 lanes) stays 64 consecutive floats.  At h = 64 the unpadded
-// offsets (multiples of 64 floats) let the reads pair up as ds_read2st64,
-// and the registers that saves are worth more than the store conflicts.
-// dW2 blocks (16 x 16, rows o, columns u): H = 64: wave w owns column block
-// w (all 4 row blocks) and contracts it over the pairs of all four waves, so
-// each accumulator is held once per workgroup instead of once per wave (the
-// whole 64 x 64 block set would not fit a wave's registers); the waves run
-// their tiles in lockstep, with workgroup barriers around each column.
+// dW2 accumulation.  For each gradient column c the waves write the split
+// G_c and a1_c of their 16 pairs to LDS as [pair][16 units] tiles of f16 (512
+// bytes per wave, 16-unit block and piece; the lanes' 8-byte stores of a tile
+// are 512 consecutive bytes) and read them back transposed, four pairs of one
+// unit per lane (ds_read_b64_tr_b16 on 512 consecutive bytes), as A (rows o)
+// and B (columns u) operands of a contraction over pairs.
+// H = 64: the four waves run their tiles in lockstep and share one set of
+// accumulators; wave w holds the quadrant of row blocks 2 (w >> 1) + {0, 1}
+// and column blocks 2 (w & 1) + {0, 1} and contracts it over the pairs of all
+// four waves (the whole 64 x 64 set would not fit a wave's registers), with
+// workgroup barriers around each column.
 // H <= 32 (PRIV): every wave holds all NRB^2 blocks (16 registers at H = 32)
 // over its own pairs, reading back only what it wrote itself, so the tile
 // loop needs no workgroup barrier: LDS operations of one wavefront are
@@ -934,26 +1152,15 @@ struct DW2Own {
   static constexpr int NRB = H / 16;
   static constexpr bool PRIV = H <= 32;
   static constexpr int NOB = PRIV ? NRB * NRB : 4;  // blocks held by a wave
-  static constexpr int NSRC = PRIV ? 1 : 4;        // waves whose pairs it contracts over
-  static constexpr int PG = H == 64 ? 64 : 68;      // floats per group of 4 pairs
-  static constexpr int WS = 4 * PG;                 // per wave (16 pairs)
-  static constexpr int BS = 4 * WS;                 // per 16-unit block (4 waves)
-  static constexpr int TSZ = NRB * BS;              // floats per transpose buffer
-  // float offset of pair 4 gp + pp, units 4 cu .. 4 cu + 3, in a wave's WS
-  // floats.  SWZ: the 16-byte chunk c = 4 pp + cu is stored at
-  // c ^ (gp ^ (pp & 2)) within its 64-float group, so that the 128-bit
-  // stores of the 16 pairs do not collide in the banks (the unpadded h = 64
-  // groups alias); the reads of a pair group stay 64 distinct floats
-  template <bool SWZ>
-  __device__ static int chunk_off(int gp, int pp, int cu) {
-    const int c = 4 * pp + cu;
-    return gp * PG + 4 * (SWZ ? c ^ (gp ^ (pp & 2)) : c);
-  }
-  __device__ static int col_block(int wave, int j) { return PRIV ? j % NRB : wave; }
-  __device__ static int row_block(int wave, int j) { return PRIV ? j / NRB : j; }
+  static constexpr int TILE = 128;                  // floats of a wave's tile (16 pairs x 16 units, one piece)
+  static constexpr int BS = 4 * TILE;               // of a 16-unit block (four waves)
+  static constexpr int PS = NRB * BS;               // of a piece
+  static constexpr int TSZ = 2 * PS;                // of a buffer
+  __device__ static int row_block(int wave, int j) { return PRIV ? j / NRB : 2 * (wave >> 1) + (j >> 1); }
+  __device__ static int col_block(int wave, int j) { return PRIV ? j % NRB : 2 * (wave & 1) + (j & 1); }
 };
 
-// Orders a wave's LDS transposes around the dW2 reads: a workgroup barrier
+// Orders a wave's LDS tiles around the dW2 reads: a workgroup barrier
 // when the waves share the accumulators, else a wavefront-scope fence.
 template <bool PRIV>
 __device__ inline void tile_sync() {
@@ -963,77 +1170,97 @@ __device__ inline void tile_sync() {
     __syncthreads();
 }
 
-// dW2 += G_c a1_c^T over this wave's own 16 pairs (PRIV), all NRB^2 blocks.
-// stgp, stbp: this wave's G and h transposes at its lane offset (+ 16 g +
-// pl); pair group ks at + ks * PG, 16-unit block b at + b * BS.  a1_c of unit
-// u = 16 ib + pl is rebuilt from h as in dw2_shared, with sc[16 ib] for the
-// column block ib (KIND 1, 2).
-template <int H, int KIND>
-__device__ inline void dw2_private(const float* stgp, const float* stbp, const float* sc, f4* dW2) {
+__device__ inline h4v read_tr(const float* p) {
+  typedef __fp16 hh4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) hh4* lds_h4;
+  return __builtin_bit_cast(h4v, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4)p));
+}
+__device__ inline h8v join(h4v a, h4v b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
+// dW2 += G_c a1_c^T over this wave's own 16 pairs (PRIV), all NRB^2 blocks;
+// gt, at: this wave's tiles at its lane offset.  hi and lo of G side by side
+// in a K of 32 against lo of a1 twice (which adds the lo lo product) and hi
+// of a1 twice.
+template <int H>
+__device__ inline void dw2_private(const float* gt, const float* at, f4* dW2) {
   using O = DW2Own<H>;
   constexpr int NRB = H / 16;
+  h4v ah[NRB], al[NRB], bh[NRB], bl[NRB];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    float a[NRB], b[NRB];
+  for (int b = 0; b < NRB; ++b) {
+    ah[b] = read_tr(gt + b * O::BS);
+    al[b] = read_tr(gt + O::PS + b * O::BS);
+    bh[b] = read_tr(at + b * O::BS);
+    bl[b] = read_tr(at + O::PS + b * O::BS);
+  }
 #pragma unroll
-    for (int ib = 0; ib < NRB; ++ib) {
-      const float h = stbp[ib * O::BS + ks * O::PG];
-      float v = h;
-      if (KIND == 1) v = fmaf(-h, h, 1.f) * sc[16 * ib];
-      if (KIND == 2) v = h * fmaf(-h, h, 1.f) * sc[16 * ib];
-      b[ib] = v;
-    }
-#pragma unroll
-    for (int ob = 0; ob < NRB; ++ob) a[ob] = stgp[ob * O::BS + ks * O::PG];
-#pragma unroll
-    for (int j = 0; j < O::NOB; ++j) dW2[j] = mfma16(a[j / NRB], b[j % NRB], dW2[j]);
+  for (int j = 0; j < O::NOB; ++j) {
+    const h8v a = join(ah[j / NRB], al[j / NRB]);
+    dW2[j] = mfma_k32(a, join(bl[j % NRB], bl[j % NRB]), dW2[j]);
+    dW2[j] = mfma_k32(a, join(bh[j % NRB], bh[j % NRB]), dW2[j]);
   }
 }
 
-// dW2[j] += G_c a1_c^T over the tile.  a1_c of unit u = 16 ibw + pl is
-// rebuilt from h: KIND 0: h, 1: (1 - h^2) sc, 2: h (1 - h^2) sc with sc
-// supplied by the caller (zt_i and -2 zt_i^2 for unit u).
-// stgl[ks] = stg + (NRB == 2 ? row block (wave >> 1) * BS : 0) +
-// chunk_off<SWZ>(ks, g, pl >> 2) + (pl & 3) is this lane's G read base for
-// pair 4 ks + g, unit pl (source wave w at + w * WS, row block ob at
-// + ob * BS); its h read base is stbl + ks * PG with stbl = stb + ibw * BS +
-// 16 g + pl (plain layout) or stgl[ks] + db (swizzled: both buffers share
-// the layout, db = stb - stg + the row-block offsets).
-template <int H, int KIND, bool SWZ>
-__device__ inline void dw2_shared(const float* const* stgl, const float* stbl, int db, float sc, f4* dW2,
-                                  int wave) {
-  using O = DW2Own<H>;
-  // swizzled buffers: the h buffer's read base for pair group ks is
-  // stgl[ks] + db; db is kept opaque so that the four sums are formed at
-  // their reads instead of held in four more registers through the tile
-  if (SWZ) asm volatile("" : "+v"(db));
-#pragma unroll
-  for (int s = 0; s < O::NSRC; ++s) {
-    const int w = O::NSRC == 1 ? wave : s;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float h = SWZ ? stgl[ks][db + w * O::WS] : stbl[w * O::WS + ks * O::PG];
-      float b = h;
-      if (KIND == 1) b = fmaf(-h, h, 1.f) * sc;
-      if (KIND == 2) b = h * fmaf(-h, h, 1.f) * sc;
-#pragma unroll
-      for (int j = 0; j < O::NOB; ++j) {
-        const float a = stgl[ks][(O::NOB == 1 ? 0 : j * O::BS) + w * O::WS];
-        dW2[j] = mfma16(a, b, dW2[j]);
-      }
-    }
-  }
-}
-
-// Write this wave's D-layout tile (units x 16 pairs) into a transpose buffer;
-// tl = t + wave * WS + (pl >> 2) * PG + (pl & 3) * 16 + 4 g.
+// dW2[j] += G_c a1_c^T over the tile's 64 pairs (two K-steps of two waves'
+// pairs), this wave's quadrant; gt, at: the quadrant's first row / column
+// block at the lane offset.
 template <int H>
-__device__ inline void store_tile(float* tl, const f4* v) {
+__device__ inline void dw2_shared(const float* gt, const float* at, f4* dW2) {
+  using O = DW2Own<H>;
 #pragma unroll
-  for (int ob = 0; ob < H / 16; ++ob) *reinterpret_cast<f4*>(tl + ob * DW2Own<H>::BS) = v[ob];
+  for (int ks = 0; ks < 2; ++ks) {
+    h8v a[2][2], b[2][2];   // [block][piece]
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int o = c * O::PS + j * O::BS + 2 * ks * O::TILE;
+        a[j][c] = join(read_tr(gt + o), read_tr(gt + o + O::TILE));
+        b[j][c] = join(read_tr(at + o), read_tr(at + o + O::TILE));
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      dW2[j] = mfma_k32(a[j >> 1][1], b[j & 1][0], dW2[j]);
+      dW2[j] = mfma_k32(a[j >> 1][0], b[j & 1][1], dW2[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dW2[j] = mfma_k32(a[j >> 1][0], b[j & 1][0], dW2[j]);
+  }
+}
+
+// Write this wave's split values (units x 16 pairs) to its tiles of a buffer;
+// tl = buffer + wave TILE + 8 pl + 2 g.
+template <int H>
+__device__ inline void store_tile(float* tl, const Split<H>& v) {
+  using O = DW2Own<H>;
+#pragma unroll
+  for (int b = 0; b < H / 16; ++b) {
+    *reinterpret_cast<u2v*>(tl + b * O::BS) = u2v{v.hi[2 * b], v.hi[2 * b + 1]};
+    *reinterpret_cast<u2v*>(tl + O::PS + b * O::BS) = u2v{v.lo[2 * b], v.lo[2 * b + 1]};
+  }
+}
+
+// This thread's largest |gseg| per jet column over its share of the chunk's
+// pairs (stage_two reduces them over the workgroup).
+template <int J>
+__device__ inline void gradient_max(const fbpx_worklist& wl, const float* gseg, int beg, int end, float* gm) {
+#pragma unroll
+  for (int c = 0; c < J; ++c) gm[c] = 0.f;
+#pragma unroll 4
+  for (int k = beg + (int)threadIdx.x; k < end; k += 256) {
+    const int seg = wl.pair_seg[k];
+#pragma unroll
+    for (int c = 0; c < J; ++c) gm[c] = fmaxf(gm[c], fabsf(gseg[(size_t)seg * J + c]));
+  }
 }
 
 // [xd, h, h, 1]: hidden-to-hidden layer on MFMA, streamed one axis at a time.
+// Scales (all powers of two, Scales): everything linear in the upstream
+// gradient is carried times 2^k; on top of it (marked ' below)
+//   Z_i' = Z_i 2^(w + e[i]),  S' = S 2^w, and with them G_0', dWL', Q' times 2^w;
+//   vt' = vt 2^r and gz1_0' times 2^r (and -1/2 until column 0);  stored G_i times 2^-e[i], so that
+//   G_i (e1 zt_i 2^e[i])^T adds to dW2 like the other columns, and so
+//   GA_i' and gz1_i' carry 2^(r - e[i]).
 template <int XD, int H, int D1M, int D2M>
 __device__ inline void bwd_two(const float* theta, const float* dom, const float* x, const fbpx_worklist& wl,
                                const float* gseg, float* partial, int chunk, float gs, const AdamFold& af,
@@ -1053,21 +1280,20 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   static_assert(H >= 16 && H <= 64, "hidden width 16, 32 or 64");
   static_assert(2 * O::TSZ >= L::P, "the gradient row reuses the transpose buffers");
   __shared__ float ss[SM::N];
-  __shared__ float szt[4 * XD * H];
+  __shared__ float szt[3 * XD * H];
   __shared__ __attribute__((aligned(16))) float swt[H * H];
   __shared__ __attribute__((aligned(16))) float swr[H * H];
   __shared__ __attribute__((aligned(16))) float strans[2 * O::TSZ];
   __shared__ float ssmall[4 * NS * H];
   __shared__ float sbl[64];
-  float* stb = strans;
-  float* stg = strans + O::TSZ;
+  __shared__ float red[64];
+  float* sta = strans;            // a1 columns
+  float* stg = strans + O::TSZ;   // G columns
 
   const int model = wl.chunk_model[chunk];
   const int beg = wl.chunk_start[chunk];
   const int end = wl.chunk_start[chunk + 1];
   const float* th = theta + (size_t)model * L::P;
-  stage_small<XD, H, 2>(th, ss);
-  stage_w2<H>(th + L::W2, th + L::WL, swt, swr);
   for (int i = threadIdx.x; i < 4 * NS * H; i += blockDim.x) ssmall[i] = 0.f;
   if (threadIdx.x < 64) sbl[threadIdx.x] = 0.f;
   Dom d;
@@ -1078,31 +1304,25 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     mu[i] = (d.xmax[i] + d.xmin[i]) / 2.f;
     isd[i] = 1.f / ((d.xmax[i] - d.xmin[i]) / 2.f);
   }
-  __syncthreads();
-  stage_zt<XD, H, SM>(ss, isd, szt);
-  __syncthreads();
+  const float one = opaque_one();
+  Scales<XD> sc;
+  {
+    float gm[J];
+    gradient_max<J>(wl, gseg, beg, end, gm);
+    stage_two<S, H, SM, true, true>(th, d, isd, gm, one, ss, szt, swt, swr, red, sc);
+  }
+  d.usd *= sc.k;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int pl = lane & 15, g = lane >> 4;
-  const int ucol = 16 * O::col_block(wave, 0) + pl;   // this lane's dW2 column unit (shared blocks)
-  const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)];   // WL of the unit a reduction leaves here
+  // WL of the unit a reduction leaves in this lane (for G_0')
+  const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)] * sc.iw;
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
-  // both transpose buffers are swizzled at h = 64 where the four extra read
-  // bases fit the register budget (every first-derivative axis also carries
-  // its second derivative; the h buffer's reads add an offset to them)
-  constexpr bool SWZ = H == 64 && D1M == D2M;
-  float* const stbw = stb + wave * O::WS + O::template chunk_off<SWZ>(pl >> 2, pl & 3, g);   // store bases
-  float* const stgw = stg + wave * O::WS + O::template chunk_off<SWZ>(pl >> 2, pl & 3, g);
-  // dW2 read bases: stgl[ks] for the G buffer; for the h buffer stbl (plain
-  // layout) or stgl[ks] + stb_off (swizzled)
-  const float* const stbl = stb + O::col_block(wave, 0) * O::BS + 16 * g + pl;
-  const int stb_off = (int)(stb - stg) + O::col_block(wave, 0) * O::BS;
-  const float* stgl[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) stgl[ks] = stg + O::template chunk_off<SWZ>(ks, g, pl >> 2) + (pl & 3);
-  // PRIV: this wave's own transposes at its lane offset
-  const float* const stgp = stg + wave * O::WS + 16 * g + pl;
-  const float* const stbp = stb + wave * O::WS + 16 * g + pl;
+  float* const staw = sta + wave * O::TILE + 8 * pl + 2 * g;   // this wave's stores
+  float* const stgw = stg + wave * O::TILE + 8 * pl + 2 * g;
+  // dW2 reads: this wave's own tiles (PRIV) or its quadrant's blocks
+  const float* const star = sta + (O::PRIV ? wave * O::TILE : O::col_block(wave, 0) * O::BS) + 2 * lane;
+  const float* const stgr = stg + (O::PRIV ? wave * O::TILE : O::row_block(wave, 0) * O::BS) + 2 * lane;
   float* mysmall = ssmall + wave * NS * H;
   float aW1[ACC ? XD : 1][NRB][4], aWL[NRB][4], aB1[NRB][4], aB2[NRB][4];
   if constexpr (ACC) {
@@ -1160,17 +1380,15 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     layer1_stream<XD, H, SM>(v, xh, h1);
     float vWL[NRB][4], gz10[NRB][4], vv[NRB][4];
 
-    tile_sync<O::PRIV>();   // the previous tile's transposes have been consumed
-
     // ---- Z_0 = W2 h1 + b2 -> h2
     float h2[NRB][4];
     {
       f4 Z0[NRB];
-      layer2_pass<H, SM>(v, h1, 0, 0, Z0);
+      layer2_value<H, SM>(v, h1, sc.w, one, Z0);
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h2[ob][r] = tanh_f(Z0[ob][r]);
+        for (int r = 0; r < 4; ++r) h2[ob][r] = tanh_f(Z0[ob][r], sc.iw);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -1181,8 +1399,10 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     //      (f1 = 1 - h2^2, f2 = -2 h2 f1, f3 = f1 (4 - 6 f1)).  The layer-1
     //      gradient starts as gz1_0 = vt rv (see pair_s); the axes add
     //      e2 zt_i GA_i and column 0 adds e1 GA_0.
-    f4 G0[NRB], vt[NRB];
+    float G0[NRB][4];
+    f4 vt[NRB];
     float Sx[NRB][4], Q[NRB][4];
+    const float gur0 = gur[0] * sc.w;
     if constexpr (S::N1 == 0) {
       // value only: no tangents, s = 0
 #pragma unroll
@@ -1190,16 +1410,21 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float h = h2[ob][r];
-          G0[ob][r] = fmaf(-h, h, 1.f) * gur[0];
-          vWL[ob][r] = gur[0] * h;
+          G0[ob][r] = fmaf(-h, h, 1.f) * gur0;
+          vWL[ob][r] = gur0 * h;
           gz10[ob][r] = 0.f;
         }
     } else {
-      float sv[NRB][4], rv[NRB][4];
-      pair_s<S, H>(v, h1, gur, sv, rv);
+      float rv[NRB][4];
+      Split<H> ssp, fsp;
+      {
+        float sv[NRB][4];
+        pair_s<S, H>(v, h1, gur, sv, rv);
+        ssp.set(sv, one);
+      }
       {
         f4 Sv[NRB];
-        layer2_pass_raw<H>(v, sv, Sv);
+        frag_mul<H>(v.wt, ssp, Sv);
 #pragma unroll
         for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
@@ -1208,47 +1433,36 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
             Q[ob][r] = 0.f;
           }
       }
-      f4 gs[NRB];
       {
-        f4 sw[NRB];
+        float f1[NRB][4];
 #pragma unroll
-        for (int ob = 0; ob < NRB; ++ob) {
-          sw[ob] = f4{sv[ob][0], sv[ob][1], sv[ob][2], sv[ob][3]};
+        for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) gs[ob][r] = fmaf(-h2[ob][r], h2[ob][r], 1.f);
-        }
-        store_tile<H>(stbw, sw);
-        store_tile<H>(stgw, gs);
+          for (int r = 0; r < 4; ++r) f1[ob][r] = fmaf(-h2[ob][r], h2[ob][r], 1.f);
+        fsp.set(f1, one);
       }
-      w2t_pass<H>(v, gs, vt);
+      tile_sync<O::PRIV>();   // the previous tile's column has been consumed
+      store_tile<H>(staw, ssp);
+      store_tile<H>(stgw, fsp);
+      frag_mul<H>(v.wr, fsp, vt);
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) gz10[rb][r] = vt[rb][r] * rv[rb][r];
       tile_sync<O::PRIV>();
       if constexpr (O::PRIV)
-        dw2_private<H, 0>(stgp, stbp, nullptr, dW2);
+        dw2_private<H>(stgr, star, dW2);
       else
-        dw2_shared<H, 0, SWZ>(stgl, stbl, stb_off, 1.f, dW2, wave);
-      tile_sync<O::PRIV>();
+        dw2_shared<H>(stgr, star, dW2);
     }
-    // layer-1 h for the B operands of the remaining dW2 columns (published
-    // with the first column's G; every column has a barrier before its reads)
-    {
-      f4 hv[NRB];
-#pragma unroll
-      for (int rb = 0; rb < NRB; ++rb) hv[rb] = f4{h1[rb][0], h1[rb][1], h1[rb][2], h1[rb][3]};
-      store_tile<H>(stbw, hv);
-    }
-    // from here on layer 1 enters only through e1 = 1 - h1^2 and h1 e1, and
-    // the axes take layer 2 through p2 = h2 - h2^3 = -f2 / 2
-    float e1[NRB][4], he[NRB][4], p2[NRB][4];
+    // from here on layer 1 enters through h1 and e1 = 1 - h1^2, and the axes
+    // take layer 2 through p2 = h2 - h2^3 = -f2 / 2
+    float e1[NRB][4], p2[NRB][4];
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         e1[rb][r] = fmaf(-h1[rb][r], h1[rb][r], 1.f);
-        he[rb][r] = h1[rb][r] * e1[rb][r];
         p2[rb][r] = fmaf(-h2[rb][r] * h2[rb][r], h2[rb][r], h2[rb][r]);
       }
     __builtin_amdgcn_sched_barrier(0);
@@ -1265,47 +1479,55 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       const bool two = S::has2(i);
       const float gur_a = pick<J>(gur, S::col1(i));
       const float gur_b = two ? pick<J>(gur, S::col2(i)) : 0.f;
-      const float isd_i = pick<XD>(isd, i);
+      const float e_i = pick<XD>(sc.e, i), ie_i = pick<XD>(sc.ie, i);
+      // gz1_i' = gz1_i 2^(r - e[i]) (r alone without a second derivative)
+      const float post = pick<XD>(isd, i) * sc.ir * (two ? e_i : 1.f);
       const int zrow = i * H;
       float gzi[NRB][4];
       if (two) {
-        f4 Gi[NRB];
+        Split<H> gsp, asp;
+        tangent_split<H>(v, e1, zrow, one, asp);
         {
           f4 Zi[NRB];
-          layer2_pass<H, SM>(v, e1, zrow, 3, Zi);
-          const float gm4 = -4.f * gur_b;
+          frag_mul<H>(v.wt, asp, Zi);
+          const float gq = (gur_b * ie_i) * (sc.iw * ie_i);   // Q' += gur_b Z_i^2 2^w
+          const float gm4 = -4.f * gq;                        // 2 gur_b f2 Z_i 2^-e[i]
+          float Gi[NRB][4];
 #pragma unroll
           for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float z = Zi[ob][r];
-              Q[ob][r] = fmaf(gur_b * z, z, Q[ob][r]);
-              Gi[ob][r] = gm4 * (p2[ob][r] * z);   // 2 gur_b f2 z
+              Q[ob][r] = fmaf(gq * z, z, Q[ob][r]);
+              Gi[ob][r] = gm4 * (p2[ob][r] * z);
             }
+          gsp.set(Gi, one);
         }
         __builtin_amdgcn_sched_barrier(0);
-        // column i: publish G_i, then W2~^T G_i while the other waves catch up
-        store_tile<H>(stgw, Gi);
+        // column i: publish G_i and a1_i, then W2~^T G_i while the other waves
+        // catch up
+        tile_sync<O::PRIV>();
+        store_tile<H>(staw, asp);
+        store_tile<H>(stgw, gsp);
         {
           f4 GA[NRB];
-          w2t_pass<H>(v, Gi, GA);
-          const float gb2 = 2.f * gur_b;
+          frag_mul<H>(v.wr, gsp, GA);
+          const float gb4 = -4.f * gur_b * ie_i * ie_i, ga = gur_a * ie_i;
 #pragma unroll
           for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const float p = he[rb][r] * v.zm[zrow + 16 * rb + r];   // e2 zt_i
-              const float q = fmaf(gb2, p, gur_a * e1[rb][r]);
+              const float p = (h1[rb][r] * e1[rb][r]) * v.zs[zrow + 16 * rb + r];   // -e2 zt_i 2^e[i] / 2
+              const float q = fmaf(gb4, p, ga * e1[rb][r]);
               gzi[rb][r] = fmaf(vt[rb][r], q, e1[rb][r] * GA[rb][r]);
               gz10[rb][r] = fmaf(p, GA[rb][r], gz10[rb][r]);
             }
         }
         tile_sync<O::PRIV>();
         if constexpr (O::PRIV)
-          dw2_private<H, 1>(stgp, stbp, szt + zrow + pl, dW2);
+          dw2_private<H>(stgr, star, dW2);
         else
-          dw2_shared<H, 1, SWZ>(stgl, stbl, stb_off, szt[zrow + ucol], dW2, wave);
-        tile_sync<O::PRIV>();
+          dw2_shared<H>(stgr, star, dW2);
       } else {
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
@@ -1317,9 +1539,9 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) aW1[i][rb][r] = fmaf(gzi[rb][r], isd_i, aW1[i][rb][r]);
+          for (int r = 0; r < 4; ++r) aW1[i][rb][r] = fmaf(gzi[rb][r], post, aW1[i][rb][r]);
       } else {
-        reduce_units_to_lds<NRB>(gzi, mysmall + (K_W1 + i) * H, pl, g, isd_i);
+        reduce_units_to_lds<NRB>(gzi, mysmall + (K_W1 + i) * H, pl, g, post);
       }
     }
     if constexpr (S::N1 > 0) {
@@ -1332,8 +1554,8 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
           const float f1 = fmaf(-h, h, 1.f);
           const float f2 = -2.f * p2[ob][r];
           const float f3 = f1 * fmaf(-6.f, f1, 4.f);
-          G0[ob][r] = fmaf(f3, Q[ob][r], fmaf(f2, Sx[ob][r], f1 * gur[0]));
-          vWL[ob][r] = fmaf(f2, Q[ob][r], fmaf(f1, Sx[ob][r], gur[0] * h));
+          G0[ob][r] = fmaf(f3, Q[ob][r], fmaf(f2, Sx[ob][r], f1 * gur0));
+          vWL[ob][r] = fmaf(f2, Q[ob][r], fmaf(f1, Sx[ob][r], gur0 * h));
         }
     }
     // ---- column 0: db2 += G_0, dW2 += G_0 h^T, W2~^T G_0 -> layer 1
@@ -1347,29 +1569,37 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) aB2[ob][r] += G0[ob][r];
     } else {
+      reduce_units_to_lds<NRB>(G0, mysmall + K_B2 * H, pl, g, wl_red);
+    }
+    {
+      Split<H> gsp, hsp;
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vv[ob][r] = G0[ob][r];
-      reduce_units_to_lds<NRB>(vv, mysmall + K_B2 * H, pl, g, wl_red);
-    }
-    store_tile<H>(stgw, G0);
-    {
+        for (int r = 0; r < 4; ++r) G0[ob][r] *= sc.iw;
+      gsp.set(G0, one);
+      hsp.set(h1, one);
+      tile_sync<O::PRIV>();
+      store_tile<H>(staw, hsp);
+      store_tile<H>(stgw, gsp);
       f4 GA[NRB];
-      w2t_pass<H>(v, G0, GA);
+      frag_mul<H>(v.wr, gsp, GA);
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) gz10[rb][r] = fmaf(e1[rb][r], GA[rb][r], gz10[rb][r]);
+        for (int r = 0; r < 4; ++r) gz10[rb][r] = fmaf(-2.f, gz10[rb][r], e1[rb][r] * GA[rb][r]);
     }
     // dW1[:, i] += gz1_0 xh_i (the gz1_i parts were added per axis)
     if constexpr (ACC) {
+      float xr[XD];
+#pragma unroll
+      for (int i = 0; i < XD; ++i) xr[i] = xh[i] * sc.ir;
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
 #pragma unroll
-          for (int i = 0; i < XD; ++i) aW1[i][rb][r] = fmaf(gz10[rb][r], xh[i], aW1[i][rb][r]);
+          for (int i = 0; i < XD; ++i) aW1[i][rb][r] = fmaf(gz10[rb][r], xr[i], aW1[i][rb][r]);
           aWL[rb][r] += vWL[rb][r];
           aB1[rb][r] += gz10[rb][r];
         }
@@ -1380,10 +1610,10 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) vv[rb][r] = gz10[rb][r] * xh[i];
-        reduce_units_to_lds<NRB>(vv, mysmall + (K_W1 + i) * H, pl, g);
+        reduce_units_to_lds<NRB>(vv, mysmall + (K_W1 + i) * H, pl, g, sc.ir);
       }
-      reduce_units_to_lds<NRB>(vWL, mysmall + K_WL * H, pl, g);
-      reduce_units_to_lds<NRB>(gz10, mysmall + K_B1 * H, pl, g);
+      reduce_units_to_lds<NRB>(vWL, mysmall + K_WL * H, pl, g, sc.iw);
+      reduce_units_to_lds<NRB>(gz10, mysmall + K_B1 * H, pl, g, sc.ir);
     }
     // the next tile's point and upstream jets, in flight during the last dW2 column
     __builtin_amdgcn_sched_barrier(0);
@@ -1393,18 +1623,18 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     for (int c = 0; c < J; ++c) gUn[c] = valid_n ? gseg[(size_t)segn * J + c] : 0.f;
     tile_sync<O::PRIV>();
     if constexpr (O::PRIV)
-      dw2_private<H, 0>(stgp, stbp, nullptr, dW2);
+      dw2_private<H>(stgr, star, dW2);
     else
-      dw2_shared<H, 0, SWZ>(stgl, stbl, stb_off, 1.f, dW2, wave);
-    // (the next tile's leading barrier orders these reads before new writes)
+      dw2_shared<H>(stgr, star, dW2);
+    // (the next tile's first column has a barrier before its stores)
   }
 
   // ---- end of chunk: the transpose buffers become the gradient row
   if constexpr (ACC) {
 #pragma unroll
     for (int i = 0; i < XD; ++i) reduce_units_to_lds<NRB>(aW1[i], mysmall + (K_W1 + i) * H, pl, g);
-    reduce_units_to_lds<NRB>(aWL, mysmall + K_WL * H, pl, g);
-    reduce_units_to_lds<NRB>(aB1, mysmall + K_B1 * H, pl, g);
+    reduce_units_to_lds<NRB>(aWL, mysmall + K_WL * H, pl, g, sc.iw);
+    reduce_units_to_lds<NRB>(aB1, mysmall + K_B1 * H, pl, g, sc.ir);
     reduce_units_to_lds<NRB>(aB2, mysmall + K_B2 * H, pl, g, wl_red);
   }
   if (g == 0) sbl[wave * 16 + pl] = dbl;
@@ -1428,7 +1658,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     }
     __syncthreads();
   }
-  finish_row<XD, H, 2>(sacc, ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs, af, model, bc);
+  finish_row<XD, H, 2>(sacc, ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs * sc.ik, af, model, bc);
 }
 
 // g_scale: NULL, or d L / d loss when gseg holds the segment gradients at
