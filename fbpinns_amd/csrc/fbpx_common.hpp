@@ -243,4 +243,10 @@ __device__ inline void adam_elem(float& p, float& m, float& v, float g, float bc
 void set_error(const char* fmt, ...);
 int hip_check(hipError_t e, const char* what);
 
+// fbpx_inside_fill that writes only below min(offsets[p + 1], n_pairs) and
+// sets *bad (device) where a point's boxes do not end exactly there (slots
+// left over are filled with box 0).
+int inside_fill_checked(hipStream_t s, const float* x, int n, int xd, const float* xmin, const float* xmax, int m,
+                        const int64_t* offsets, int64_t n_pairs, int32_t* n_take, int32_t* m_take, int32_t* bad);
+
 }  // namespace fbpx

@@ -19,14 +19,12 @@
 //            order, so its index is jnp.unique's inverse p_take; the pairs
 //            of a segment keep the point-major (reference) order, which
 //            gives each pair its slot.
-//   tiles    pairs grouped by model position, ascending point within: for
-//            every (model position, block of 2048 points) a workgroup
-//            repeats the inside test of the block's points against that one
-//            box (skipped when the block's bounding box misses the box), so
-//            a count pass, one exclusive scan in (model, block) order and a
-//            fill pass place every pair stably without sorting; each tile
-//            pair finds its point-major twin by binary search in the point's
-//            ascending box list.
+//   tiles    pairs grouped by model position, ascending point within: a
+//            stable counting sort of the point-major pairs by model position.
+//            Each workgroup takes the pairs of 1024 points, counts them per
+//            model in LDS, one exclusive scan in (model, block) order gives
+//            every block's place in every model, and a fill pass writes the
+//            pairs there in order (tile_sort_kernel).
 //   chunks   cut flags at every model start, every `chunk` pairs inside a
 //            model and at both kernels' bin edges (round(linspace) over the
 //            pairs, numpy's half-to-even rounding), compacted by a scan.
@@ -42,10 +40,11 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kThreads * kScanItems;   // elements per scan workgroup
-constexpr int kTileItems = 8;
-constexpr int kTilePoints = kThreads * kTileItems;  // points per tile workgroup
+constexpr int kTilePoints = 1024;                   // points per tile workgroup
+constexpr int kSortWaves = 8;                       // waves of a tile workgroup
+constexpr int kSortModels = 1536;                   // models counted at a time (48 KB of LDS counters)
 constexpr int kUsedLds = 32768;                     // models flagged in LDS
-constexpr int64_t kUsedPairs = 16384;               // pairs per "used" workgroup
+constexpr int64_t kUsedPairs = 4096;                // pairs per "used" workgroup
 constexpr int kMaxPou = 32;
 
 // ------------------------------------------------------------------ scan
@@ -61,11 +60,11 @@ __device__ inline T wave_incl_scan(T v) {
   return v;
 }
 
-// Exclusive scan over the 256 threads of the workgroup (thread order); total
+// Exclusive scan over the NT threads of the workgroup (thread order); total
 // is the sum over all threads.  Every thread must call it.
-template <class T>
+template <class T, int NT = kThreads>
 __device__ inline T block_excl_scan(T v, T& total) {
-  __shared__ T wsum[kThreads / 64];
+  __shared__ T wsum[NT / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const T inc = wave_incl_scan(v);
   if (lane == 63) wsum[w] = inc;
@@ -73,7 +72,7 @@ __device__ inline T block_excl_scan(T v, T& total) {
   T base = 0;
   total = 0;
 #pragma unroll
-  for (int i = 0; i < kThreads / 64; ++i) {
+  for (int i = 0; i < NT / 64; ++i) {
     if (i < w) base += wsum[i];
     total += wsum[i];
   }
@@ -192,41 +191,44 @@ __global__ void __launch_bounds__(kThreads) used_kernel(const int32_t* __restric
 }
 
 // info slots (device int32, read back by the host at the end)
-enum { kInfoActive = 0, kInfoUsed, kInfoNpou, kInfoBadActive, kInfoBadPou, kInfoLen = 8 };
+enum { kInfoActive = 0, kInfoUsed, kInfoNpou, kInfoBadActive, kInfoBadPou, kInfoBadOffsets,
+       kInfoSegs, kInfoCuts, kInfoPlaced, kInfoLen = 16 };
 
 // One workgroup: the active remap of trainers.py:347-357 and all_ims.
-__global__ void __launch_bounds__(kThreads) remap_kernel(const int32_t* __restrict__ active,
-                                                         const uint8_t* __restrict__ used,
-                                                         const int32_t* __restrict__ pou, int m,
-                                                         int32_t* __restrict__ act_out, int32_t* __restrict__ all_ims,
-                                                         int32_t* __restrict__ inv, int32_t* __restrict__ info) {
+constexpr int kRemapThreads = 1024;
+__global__ void __launch_bounds__(kRemapThreads) remap_kernel(const int32_t* __restrict__ active,
+                                                              const uint8_t* __restrict__ used,
+                                                              const int32_t* __restrict__ pou, int m,
+                                                              int32_t* __restrict__ act_out,
+                                                              int32_t* __restrict__ all_ims,
+                                                              int32_t* __restrict__ inv, int32_t* __restrict__ info) {
   __shared__ uint32_t pmask;
-  __shared__ int bad_a, bad_p;
+  __shared__ int bad;   // bit 0: active, bit 1: pou
   if (threadIdx.x == 0) {
     pmask = 0;
-    bad_a = 0;
-    bad_p = 0;
+    bad = 0;
   }
-  __syncthreads();
+  uint32_t my_pou = 0;
+  int my_bad = 0;
   int carry = 0;
-  for (int j0 = 0; j0 < m; j0 += kThreads) {
+  for (int j0 = 0; j0 < m; j0 += kRemapThreads) {
     const int j = j0 + threadIdx.x;
     int a = 0;
     if (j < m) {
       a = active[j];
-      if (a < 0 || a > 2) atomicOr(&bad_a, 1);
+      if (a < 0 || a > 2) my_bad |= 1;
       const int pv = pou[j];
       if (pv < 0 || pv >= kMaxPou)
-        atomicOr(&bad_p, 1);
+        my_bad |= 2;
       else
-        atomicOr(&pmask, 1u << pv);
+        my_pou |= 1u << pv;
       if (a == 0) a = 1;
       if (!used[j]) a = 0;
       act_out[j] = a;
       inv[j] = -1;
     }
     int tot;
-    const int ex = block_excl_scan<int>(a == 1, tot);
+    const int ex = block_excl_scan<int, kRemapThreads>(a == 1, tot);
     if (a == 1) {
       all_ims[carry + ex] = j;
       inv[j] = carry + ex;
@@ -234,11 +236,11 @@ __global__ void __launch_bounds__(kThreads) remap_kernel(const int32_t* __restri
     carry += tot;
   }
   const int n_active = carry;
-  for (int j0 = 0; j0 < m; j0 += kThreads) {
+  for (int j0 = 0; j0 < m; j0 += kRemapThreads) {
     const int j = j0 + threadIdx.x;
     const int a = j < m ? act_out[j] : 0;
     int tot;
-    const int ex = block_excl_scan<int>(a == 2, tot);
+    const int ex = block_excl_scan<int, kRemapThreads>(a == 2, tot);
     if (a == 2) {
       all_ims[carry + ex] = j;
       inv[j] = carry + ex;
@@ -246,12 +248,15 @@ __global__ void __launch_bounds__(kThreads) remap_kernel(const int32_t* __restri
     carry += tot;
   }
   __syncthreads();
+  if (my_pou) atomicOr(&pmask, my_pou);
+  if (my_bad) atomicOr(&bad, my_bad);
+  __syncthreads();
   if (threadIdx.x == 0) {
     info[kInfoActive] = n_active;
     info[kInfoUsed] = carry;
     info[kInfoNpou] = __popc(pmask);
-    info[kInfoBadActive] = bad_a;
-    info[kInfoBadPou] = bad_p;
+    info[kInfoBadActive] = bad & 1;
+    info[kInfoBadPou] = bad >> 1;
   }
 }
 
@@ -291,10 +296,12 @@ __global__ void __launch_bounds__(kThreads) seg_size_kernel(int n, const int64_t
   }
 }
 
-// Per point: p_take, the slot of each point-major pair (segment start + its
-// rank among the segment's pairs in point-major order), np_take and the
-// re-indexed m_take.
-__global__ void __launch_bounds__(kThreads) seg_fill_kernel(int n, const int64_t* __restrict__ off,
+// Per pair: p_take, the slot (segment start + its rank among the segment's
+// pairs in point-major order), the re-indexed m_take and, at a segment's first
+// pair, np_take.  A thread per pair keeps the three output streams coalesced
+// (a thread per point took 65 us for 3.6 M pairs).
+__global__ void __launch_bounds__(kThreads) seg_fill_kernel(int64_t s, const int64_t* __restrict__ off,
+                                                            const int32_t* __restrict__ n_take,
                                                             const int32_t* __restrict__ mg,
                                                             const int32_t* __restrict__ pou,
                                                             const uint32_t* __restrict__ pmask,
@@ -304,145 +311,101 @@ __global__ void __launch_bounds__(kThreads) seg_fill_kernel(int n, const int64_t
                                                             int32_t* __restrict__ p_take, int32_t* __restrict__ slot_pm,
                                                             int32_t* __restrict__ np_take,
                                                             int32_t* __restrict__ m_take) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p >= n) return;
-  int seg = point_seg_start[p];
-  const int64_t q0 = off[p], q1 = off[p + 1];
-  for (int64_t q = q0; q < q1; ++q) m_take[q] = inv[mg[q]];
-  for (uint32_t mm = pmask[p]; mm; mm &= mm - 1, ++seg) {
-    const int v = __ffs(mm) - 1;
-    int w = seg_pair_start[seg];
-    np_take[seg] = p;
-    for (int64_t q = q0; q < q1; ++q) {
-      if (pou[mg[q]] == v) {
-        p_take[q] = seg;
-        slot_pm[q] = w++;
-      }
-    }
+  const int64_t q = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (q >= s) return;
+  const int p = n_take[q], j = mg[q];
+  m_take[q] = inv[j];
+  const int v = pou[j];
+  if ((unsigned)v >= (unsigned)kMaxPou) return;   // reported by remap_kernel
+  const uint32_t mm = pmask[p];
+  const int64_t q0 = off[p];
+  const int seg = point_seg_start[p] + __popc(mm & ((1u << v) - 1));
+  int rank = (int)(q - q0);
+  if (mm & (mm - 1)) {   // several levels: count the point's earlier pairs of this one
+    rank = 0;
+    for (int64_t r = q0; r < q; ++r) rank += pou[mg[r]] == v;
   }
+  p_take[q] = seg;
+  slot_pm[q] = seg_pair_start[seg] + rank;
+  if (rank == 0) np_take[seg] = p;
 }
 
-// Bounding box of each block of kTilePoints points: lo[b][i], hi[b][i].
-template <int XD>
-__global__ void __launch_bounds__(kThreads) block_bbox_kernel(const float* __restrict__ x, int n,
-                                                              float* __restrict__ lo, float* __restrict__ hi) {
-  __shared__ float slo[kThreads][XD], shi[kThreads][XD];
-  const int b = blockIdx.x;
-  float l[XD], h[XD];
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    l[i] = INFINITY;
-    h[i] = -INFINITY;
-  }
-  for (int k = 0; k < kTileItems; ++k) {
-    const int p = b * kTilePoints + threadIdx.x * kTileItems + k;
-    if (p < n) {
-#pragma unroll
-      for (int i = 0; i < XD; ++i) {
-        const float v = x[(size_t)p * XD + i];
-        l[i] = fminf(l[i], v);   // a NaN coordinate is never inside a box; fminf skips it
-        h[i] = fmaxf(h[i], v);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    slo[threadIdx.x][i] = l[i];
-    shi[threadIdx.x][i] = h[i];
-  }
-  __syncthreads();
-  if (threadIdx.x < XD) {
-    const int i = threadIdx.x;
-    float a = INFINITY, c = -INFINITY;
-    for (int t = 0; t < kThreads; ++t) {
-      a = fminf(a, slo[t][i]);
-      c = fmaxf(c, shi[t][i]);
-    }
-    lo[b * XD + i] = a;
-    hi[b * XD + i] = c;
-  }
-}
-
-// The inside test of point p against one box (decompositions.py:225-226).
-template <int XD>
-__device__ inline bool inside_box(const float* __restrict__ x, int p, const float* blo, const float* bhi) {
-  bool in = true;
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    const float v = x[(size_t)p * XD + i];
-    in = in && (v >= blo[i]) && (v <= bhi[i]);
-  }
-  return in;
-}
-
-// Workgroup (model position k, point block b), flattened k * nblk + b.
-// FILL = false: blkcnt[k * nblk + b] = the block's points inside box
-// all_ims[k] (0 for k >= n_used).  FILL = true: writes those points' tile
-// pairs at base[k * nblk + b] onwards, in ascending point order.
-template <int XD, bool FILL>
-__global__ void __launch_bounds__(kThreads) tile_kernel(const float* __restrict__ x, int n, int nblk,
-                                                        const float* __restrict__ xmin, const float* __restrict__ xmax,
-                                                        const float* __restrict__ blo, const float* __restrict__ bhi,
-                                                        const int32_t* __restrict__ all_ims,
-                                                        const int32_t* __restrict__ info, int32_t* __restrict__ blkcnt,
-                                                        const int64_t* __restrict__ off, const int32_t* __restrict__ mg,
-                                                        const int32_t* __restrict__ p_take,
-                                                        const int32_t* __restrict__ slot_pm,
-                                                        int32_t* __restrict__ pair_point, int32_t* __restrict__ pair_seg,
-                                                        int32_t* __restrict__ pair_slot) {
-  const int64_t wg = blockIdx.x;
-  const int k = (int)(wg / nblk), b = (int)(wg % nblk);
+// Stable counting sort of the point-major pairs by model position, one
+// workgroup per block of kTilePoints points, wave w over kTilePoints /
+// kSortWaves consecutive points of it, kSortModels models at a time.
+// FILL = false: blkcnt[k * nblk + b] = the block's pairs of model position k
+// (0 for k >= n_used).  FILL = true: blkcnt holds the scanned bases; each
+// wave turns its counts into its own bases and places its pairs 64 at a time,
+// a pair's place being its model's base plus its rank among the 64 lanes
+// (equal models found by one ballot per bit of the position), so pairs of a
+// model stay in point-major order.  LDS and memory latency bound: pairs are
+// read twice and written once.  (Testing every point of a block against
+// every box and searching each pair's twin in its point's list took 1.35 +
+// 1.85 ms on 524,288 points, 864 boxes and 3.6 M pairs; this takes 12 + 131
+// us.)
+template <bool FILL>
+__global__ void __launch_bounds__(64 * kSortWaves) tile_sort_kernel(
+    int n, int nblk, int m, int win, const int64_t* __restrict__ off, const int32_t* __restrict__ info,
+    const int32_t* __restrict__ m_take, const int32_t* __restrict__ n_take, const int32_t* __restrict__ p_take,
+    const int32_t* __restrict__ slot_pm, int32_t* __restrict__ blkcnt, int32_t* __restrict__ pair_point,
+    int32_t* __restrict__ pair_seg, int32_t* __restrict__ pair_slot) {
+  extern __shared__ int32_t sort_cnt[];   // [kSortWaves][win]
+  constexpr int kWavePoints = kTilePoints / kSortWaves;
+  const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int32_t* cnt = sort_cnt + w * win;
   const int n_used = info[kInfoUsed];
-  if (k >= n_used) {
-    if (!FILL && threadIdx.x == 0) blkcnt[wg] = 0;
-    return;
-  }
-  const int j = all_ims[k];
-  float lo[XD], hi[XD];
-  bool miss = false;
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    lo[i] = xmin[(size_t)j * XD + i];
-    hi[i] = xmax[(size_t)j * XD + i];
-    miss = miss || hi[i] < blo[b * XD + i] || lo[i] > bhi[b * XD + i];
-  }
-  if (miss) {   // uniform across the workgroup: no point of the block can be inside
-    if (!FILL && threadIdx.x == 0) blkcnt[wg] = 0;
-    return;
-  }
-  const int p0 = b * kTilePoints + threadIdx.x * kTileItems;
-  uint32_t bits = 0;
-#pragma unroll
-  for (int t = 0; t < kTileItems; ++t) {
-    const int p = p0 + t;
-    if (p < n && inside_box<XD>(x, p, lo, hi)) bits |= 1u << t;
-  }
-  int tot;
-  const int ex = block_excl_scan<int>(__popc(bits), tot);
-  if (!FILL) {
-    if (threadIdx.x == 0) blkcnt[wg] = tot;
-    return;
-  }
-  int t_out = blkcnt[wg] + ex;   // blkcnt holds the scanned bases here
-  for (; bits; bits &= bits - 1) {
-    const int p = p0 + __ffs(bits) - 1;
-    // the pair's point-major twin: box j in the point's ascending box list
-    const int64_t q_end = off[p + 1];
-    int64_t a = off[p], c = q_end;
-    while (a < c) {
-      const int64_t mid = (a + c) >> 1;
-      if (mg[mid] < j)
-        a = mid + 1;
-      else
-        c = mid;
+  const int p0 = min(n, b * kTilePoints + w * kWavePoints), p1 = min(n, p0 + kWavePoints);
+  const int64_t q0 = off[p0], q1 = off[p1];
+  for (int k0 = 0; k0 < (FILL ? n_used : m); k0 += win) {
+    for (int k = lane; k < win; k += 64) cnt[k] = 0;
+    if (k0 < n_used) {
+      for (int64_t q = q0 + lane; q < q1; q += 64) {
+        const int k = m_take[q] - k0;
+        if (k >= 0 && k < win) atomicAdd(&cnt[k], 1);
+      }
     }
-    const bool found = a < q_end && mg[a] == j;   // always, for offsets of these points
-    pair_point[t_out] = p;
-    pair_seg[t_out] = found ? p_take[a] : -1;
-    pair_slot[t_out] = found ? slot_pm[a] : -1;
-    ++t_out;
+    __syncthreads();
+    for (int k = threadIdx.x; k < win && k0 + k < m; k += 64 * kSortWaves) {
+      const int64_t slot = (int64_t)(k0 + k) * nblk + b;
+      int32_t base = FILL ? blkcnt[slot] : 0;
+      for (int v = 0; v < kSortWaves; ++v) {
+        const int32_t c = sort_cnt[v * win + k];
+        if (FILL) sort_cnt[v * win + k] = base;
+        base += c;
+      }
+      if (!FILL) blkcnt[slot] = base;
+    }
+    __syncthreads();
+    if (FILL) {
+      for (int64_t q = q0; q < q1; q += 64) {   // wave-uniform trip count
+        const bool live = q + lane < q1;
+        const int k = live ? m_take[q + lane] - k0 : -1;
+        const bool in = k >= 0 && k < win;
+        uint64_t same = __ballot(in);
+        if (same == 0) continue;
+#pragma unroll
+        for (int bit = 0; bit < 11; ++bit) {
+          const bool one = (k >> bit) & 1;
+          const uint64_t v = __ballot(one);
+          same &= one ? v : ~v;
+        }
+        if (in) {
+          const int64_t t = cnt[k] + __popcll(same & ((1ull << lane) - 1));
+          // the model's highest lane moves its base past the 64 pairs, after
+          // every lane has read it (a wave's LDS operations are in order)
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+          if ((same >> lane) == 1) cnt[k] += __popcll(same);
+          pair_point[t] = n_take[q + lane];
+          pair_seg[t] = p_take[q + lane];
+          pair_slot[t] = slot_pm[q + lane];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      }
+      __syncthreads();
+    }
   }
 }
+static_assert(kSortModels <= 1 << 11, "a model position within a window is matched on 11 bits");
 
 // model_start[k] = base[k * nblk] for k <= n_used (base[n_used * nblk] = s).
 __global__ void __launch_bounds__(kThreads) model_start_kernel(const int32_t* __restrict__ base, int nblk, int m,
@@ -538,6 +501,14 @@ __global__ void __launch_bounds__(kThreads) bins_kernel(int nb, const int32_t* _
   }
 }
 
+// The sizes found on the way, next to the other info slots (one read-back).
+__global__ void sizes_kernel(const int32_t* __restrict__ n_segs, const int32_t* __restrict__ cuts,
+                             const int32_t* __restrict__ placed, int32_t* __restrict__ info) {
+  info[kInfoSegs] = *n_segs;
+  info[kInfoCuts] = *cuts;
+  info[kInfoPlaced] = *placed;
+}
+
 // ------------------------------------------------------------------ work space
 
 size_t align_up(size_t v) { return (v + 255) & ~size_t(255); }
@@ -564,8 +535,6 @@ struct Work {
   int32_t* info;
   uint32_t* pmask;
   int32_t* slot_pm;
-  float* blo;
-  float* bhi;
   int32_t* blkcnt;
   int32_t* model_start;
   uint8_t* flags;
@@ -587,8 +556,6 @@ Work carve(void* base, int n, int xd, int m, int64_t s, int fbins, int bbins, si
   w.info = c.take<int32_t>(kInfoLen);
   w.pmask = c.take<uint32_t>(n);
   w.slot_pm = c.take<int32_t>(s);
-  w.blo = c.take<float>(nb * xd);
-  w.bhi = c.take<float>(nb * xd);
   w.blkcnt = c.take<int32_t>((int64_t)m * nb + 1);
   w.model_start = c.take<int32_t>((int64_t)m + 1);
   w.flags = c.take<uint8_t>(s + 1);
@@ -599,17 +566,13 @@ Work carve(void* base, int n, int xd, int m, int64_t s, int fbins, int bbins, si
   return w;
 }
 
-template <int XD>
-void launch_tiles(hipStream_t st, bool fill_pass, const float* x, int n, int nblk, int m, const float* xmin,
-                  const float* xmax, const Work& w, const int32_t* all_ims, const int64_t* off,
-                  const int32_t* p_take, int32_t* pair_point, int32_t* pair_seg, int32_t* pair_slot) {
-  const dim3 grid((unsigned)((int64_t)m * nblk));
-  if (fill_pass)
-    hipLaunchKernelGGL((tile_kernel<XD, true>), grid, dim3(kThreads), 0, st, x, n, nblk, xmin, xmax, w.blo, w.bhi,
-                       all_ims, w.info, w.blkcnt, off, w.mg, p_take, w.slot_pm, pair_point, pair_seg, pair_slot);
-  else
-    hipLaunchKernelGGL((tile_kernel<XD, false>), grid, dim3(kThreads), 0, st, x, n, nblk, xmin, xmax, w.blo, w.bhi,
-                       all_ims, w.info, w.blkcnt, off, w.mg, p_take, w.slot_pm, pair_point, pair_seg, pair_slot);
+void launch_tiles(hipStream_t st, bool fill_pass, int n, int nblk, int m, const Work& w, const int64_t* off,
+                  const fbpx_takes_out& o) {
+  const int win = std::min(m, kSortModels);
+  const size_t lds = sizeof(int32_t) * kSortWaves * win;
+  hipLaunchKernelGGL(fill_pass ? tile_sort_kernel<true> : tile_sort_kernel<false>, dim3((unsigned)nblk),
+                     dim3(64 * kSortWaves), lds, st, n, nblk, m, win, off, w.info, o.m_take, o.n_take, o.p_take,
+                     w.slot_pm, w.blkcnt, o.pair_point, o.pair_seg, o.pair_slot);
 }
 
 int check_sizes(const char* what, const float* x, int32_t n, int32_t xd, const float* xmin, const float* xmax,
@@ -706,12 +669,14 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
 
   // point-major pairs and the models they use
   fill<uint8_t>(st, w.used, m, 0);
+  fill<int32_t>(st, w.info, kInfoLen, 0);
   if (s > 0) {
-    if ((rc = fbpx_inside_fill(stream, x, n, xd, xmin, xmax, m, nullptr, offsets, o.n_take, w.mg))) return rc;
+    if ((rc = inside_fill_checked(st, x, n, xd, xmin, xmax, m, offsets, s, o.n_take, w.mg, w.info + kInfoBadOffsets)))
+      return rc;
     hipLaunchKernelGGL(used_kernel, dim3((unsigned)((s + kUsedPairs - 1) / kUsedPairs)), dim3(kThreads), 0, st, w.mg,
                        s, m, w.used);
   }
-  hipLaunchKernelGGL(remap_kernel, dim3(1), dim3(kThreads), 0, st, active, w.used, pou, m, o.active, o.all_ims, w.inv,
+  hipLaunchKernelGGL(remap_kernel, dim3(1), dim3(kRemapThreads), 0, st, active, w.used, pou, m, o.active, o.all_ims, w.inv,
                      w.info);
 
   // segments: (point, pou) rows in ascending order and each pair's slot
@@ -725,26 +690,16 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
     hipLaunchKernelGGL(seg_size_kernel, dim3(grid_for(n)), dim3(kThreads), 0, st, n, offsets, w.mg, pou, w.pmask,
                        o.point_seg_start, o.seg_pair_start);
   scan<int32_t, int32_t>(st, o.seg_pair_start, s, o.seg_pair_start, w.tsum);
-  if (n > 0)
-    hipLaunchKernelGGL(seg_fill_kernel, dim3(grid_for(n)), dim3(kThreads), 0, st, n, offsets, w.mg, pou, w.pmask,
-                       o.point_seg_start, o.seg_pair_start, w.inv, o.p_take, w.slot_pm, o.np_take, o.m_take);
+  if (s > 0)
+    hipLaunchKernelGGL(seg_fill_kernel, dim3(grid_for(s)), dim3(kThreads), 0, st, s, offsets, o.n_take, w.mg, pou,
+                       w.pmask, o.point_seg_start, o.seg_pair_start, w.inv, o.p_take, w.slot_pm, o.np_take, o.m_take);
 
   // tile order: count per (model position, point block), scan, fill
   const int64_t nwg = (int64_t)m * nblk;
   if (nwg > 0) {
-    switch (xd) {
-      case 1: hipLaunchKernelGGL(block_bbox_kernel<1>, dim3((unsigned)nblk), dim3(kThreads), 0, st, x, n, w.blo, w.bhi); break;
-      case 2: hipLaunchKernelGGL(block_bbox_kernel<2>, dim3((unsigned)nblk), dim3(kThreads), 0, st, x, n, w.blo, w.bhi); break;
-      default: hipLaunchKernelGGL(block_bbox_kernel<3>, dim3((unsigned)nblk), dim3(kThreads), 0, st, x, n, w.blo, w.bhi); break;
-    }
-    for (int pass = 0; pass < 2; ++pass) {
-      switch (xd) {
-        case 1: launch_tiles<1>(st, pass, x, n, (int)nblk, m, xmin, xmax, w, o.all_ims, offsets, o.p_take, o.pair_point, o.pair_seg, o.pair_slot); break;
-        case 2: launch_tiles<2>(st, pass, x, n, (int)nblk, m, xmin, xmax, w, o.all_ims, offsets, o.p_take, o.pair_point, o.pair_seg, o.pair_slot); break;
-        default: launch_tiles<3>(st, pass, x, n, (int)nblk, m, xmin, xmax, w, o.all_ims, offsets, o.p_take, o.pair_point, o.pair_seg, o.pair_slot); break;
-      }
-      if (pass == 0) scan<int32_t, int32_t>(st, w.blkcnt, nwg, w.blkcnt, w.tsum);
-    }
+    launch_tiles(st, false, n, (int)nblk, m, w, offsets, o);
+    scan<int32_t, int32_t>(st, w.blkcnt, nwg, w.blkcnt, w.tsum);
+    launch_tiles(st, true, n, (int)nblk, m, w, offsets, o);
   } else {
     fill<int32_t>(st, w.blkcnt, 1, 0);
   }
@@ -772,15 +727,12 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
                      w.fedges, w.cut, s, (int)max_chunks, o.fbin_chunk_start);
   hipLaunchKernelGGL(bins_kernel, dim3(grid_for((bbins > 0 ? bbins : max_chunks) + 1)), dim3(kThreads), 0, st, bbins,
                      w.bedges, w.cut, s, (int)max_chunks, o.bbin_chunk_start);
-  if ((rc = hip_check(hipGetLastError(), "build_worklist"))) return rc;
-
   // sizes back to the host
+  hipLaunchKernelGGL(sizes_kernel, dim3(1), dim3(1), 0, st, o.point_seg_start + n, w.cut + s + 1, w.blkcnt + nwg,
+                     w.info);
+  if ((rc = hip_check(hipGetLastError(), "build_worklist"))) return rc;
   int32_t h_info[kInfoLen] = {};
-  int32_t h_tail[3] = {};   // n_segs, cuts, s from the tile scan
   if ((rc = hip_check(hipMemcpyAsync(h_info, w.info, sizeof(h_info), hipMemcpyDeviceToHost, st), "copy info")) ||
-      (rc = hip_check(hipMemcpyAsync(&h_tail[0], o.point_seg_start + n, 4, hipMemcpyDeviceToHost, st), "copy")) ||
-      (rc = hip_check(hipMemcpyAsync(&h_tail[1], w.cut + s + 1, 4, hipMemcpyDeviceToHost, st), "copy")) ||
-      (rc = hip_check(hipMemcpyAsync(&h_tail[2], w.blkcnt + nwg, 4, hipMemcpyDeviceToHost, st), "copy")) ||
       (rc = hip_check(hipStreamSynchronize(st), "build_worklist: sync")))
     return rc;
   if (h_info[kInfoBadActive]) {
@@ -791,18 +743,18 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
     set_error("build_worklist: pou values must lie in [0, %d)", kMaxPou);
     return FBPX_EUNSUPPORTED;
   }
-  if ((int64_t)h_tail[2] != s) {
+  if ((int64_t)h_info[kInfoPlaced] != s || h_info[kInfoBadOffsets]) {
     set_error("build_worklist: tile pass placed %d pairs of %lld (offsets not from fbpx_takes_count on these inputs?)",
-              h_tail[2], (long long)s);
+              h_info[kInfoPlaced], (long long)s);
     return FBPX_EINVAL;
   }
   info->n_pairs = s;
-  info->n_segs = h_tail[0];
+  info->n_segs = h_info[kInfoSegs];
   info->n_used = h_info[kInfoUsed];
   info->n_active = h_info[kInfoActive];
-  info->n_chunks = h_tail[1] - 1;
-  info->n_fbins = fbins > 0 ? fbins : h_tail[1] - 1;
-  info->n_bbins = bbins > 0 ? bbins : h_tail[1] - 1;
+  info->n_chunks = h_info[kInfoCuts] - 1;
+  info->n_fbins = fbins > 0 ? fbins : h_info[kInfoCuts] - 1;
+  info->n_bbins = bbins > 0 ? bbins : h_info[kInfoCuts] - 1;
   info->npou = h_info[kInfoNpou];
   return FBPX_OK;
 }

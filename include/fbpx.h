@@ -184,8 +184,7 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
 /* Window jets summed per segment: wsum[seg][J] = sum over the segment's pairs
  * of the jets of window_fn (decompositions.py:196-199, windows.py:25-35).
  * Parameter-independent; computed once per work list.  pair_scratch:
- * [n_pairs][J] caller-provided work space (e.g. the forward pair buffer),
- * written by slot. */
+ * [n_pairs][J] caller-provided work space (e.g. the forward pair buffer). */
 int fbpx_pou_prepare(void* stream, const fbpx_net* net, const float* dom,
                      const float* x, const fbpx_worklist* wl, float* pair_scratch,
                      float* wsum);
