@@ -35,13 +35,30 @@ their step is launch-bound and the timings would be noise.
 default_spec for a small work list: ("waves", WAVE_CHUNK) for a
 one-hidden-layer network with at least WAVE_MIN_CHUNKS_PER_CU chunks (at
 FBPX_CHUNK pairs) per CU averaging at most WAVE_MAX_CHUNK_PAIRS pairs (the
-short chunks it was measured on), else DEFAULT_SMALL.  Measured on MI355X, batched
+short chunks it was measured on); plan_chunk pairs for a two-hidden-layer
+network whose FBPX_CHUNK-pair list leaves CUs without a second workgroup; else
+DEFAULT_SMALL.  Measured on MI355X, batched
 1D inverse oscillators, [1, 32, 1], 23 pairs per chunk on average, steps/s of
 ("chunks", 512) -> ("waves", 32): 90 chunks 27,100 -> 27,400; 355 chunks
 25,200 -> 25,000; 719 chunks 22,300 -> 22,900; 1,490 chunks 20,700 ->
 22,200; 3,061 chunks 17,800 -> 20,300; 6,078 chunks 12,600 -> 16,000.  With
 few chunks a workgroup's waves shorten each chunk's latency chain by sharing
 its sub-tiles; with many, the waves a short chunk leaves idle cost more.
+
+plan_chunk (the lists that nobody times: inference and FBPINNJets layers, and
+the small lists above): two chunks per CU, of 64 to 384 pairs.  Forward +
+backward us by chunk cap (none = one chunk per subdomain):
+  [2,64,64,1] 180,699 pairs, 56 subdomains: none 221 + 647, 128 40 + 143,
+    384 36 + 111, 512 43 + 136
+  [3,64,64,1] 13,647 pairs, 36 subdomains: none 81 + 245, 64 26 + 47, 128
+    25 + 53, 512 43 + 118
+  [2,32,32,1] 361,229 pairs, 196 subdomains: none 68 + 142, 256 33 + 110, 384
+    31 + 97, 512 37 + 114
+  [3,64,1] 206,094 pairs, 75 subdomains: none 120 + 205, 384 32 + 50
+  [3,64,64,1] values of 685,693 pairs, 864 subdomains: none 61, 256 53, 384
+    51, 512 55
+A few pairs per chunk cost a weight staging each; a whole subdomain per chunk
+leaves most of 256 CUs idle.
 """
 
 import math
@@ -62,8 +79,16 @@ DEFAULT_LARGE = ("bins", 1)
 MIN_PAIRS = 200_000
 WAVE_MIN_CHUNKS_PER_CU = 2
 WAVE_MAX_CHUNK_PAIRS = 64
+PLAN_CHUNKS_PER_CU = 2
+PLAN_CHUNK_MAX = 384
 TIE = 0.02
 _cache = {}
+
+
+def plan_chunk(n_pairs, n_cu):
+    """Chunk cap of a work list that is not timed (see above)."""
+    per = -(-int(n_pairs) // (PLAN_CHUNKS_PER_CU * max(int(n_cu), 1)))
+    return min(max(64, -(-per // 64) * 64), PLAN_CHUNK_MAX)
 
 
 def default_spec(n_pairs, nh=2, n_chunks=0, n_cu=1):
@@ -73,6 +98,8 @@ def default_spec(n_pairs, nh=2, n_chunks=0, n_cu=1):
         return DEFAULT_LARGE
     if nh == 1 and n_chunks >= WAVE_MIN_CHUNKS_PER_CU * n_cu and n_pairs <= WAVE_MAX_CHUNK_PAIRS * n_chunks:
         return ("waves", WAVE_CHUNK)
+    if nh == 2 and n_chunks < PLAN_CHUNKS_PER_CU * n_cu:
+        return ("chunks", plan_chunk(n_pairs, n_cu))
     return DEFAULT_SMALL
 
 

@@ -426,7 +426,8 @@ class FusedEngine:
         `active`) used and every used subdomain trained."""
         x = x.to(self.device, torch.float32).contiguous()
         active = np.ones(self.m, dtype=int) if active is None else np.asarray(active)
-        plan, takes, _, _ = device_plan(x, active, self.all_params)
+        n_cu = torch.cuda.get_device_properties(self.device).multi_processor_count
+        plan, takes, _, _ = device_plan(x, active, self.all_params, chunk=lambda s: autotune.plan_chunk(s, n_cu))
         net = self.net0.with_schema(*schema)
         wsum = torch.empty((max(plan.wl.n_segs, 1), net.J), dtype=torch.float32, device=self.device)
         scratch = torch.empty((max(plan.wl.n_pairs, 1), net.J), dtype=torch.float32, device=self.device)

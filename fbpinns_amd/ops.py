@@ -738,7 +738,8 @@ def device_worklist(x, xmins, xmaxs, active, pou, chunk=0, fbins=0, bbins=0):
     under the scheduler state `active` (m,) with levels `pou` (m,), built on
     the GPU by fbpx_takes_count + fbpx_build_worklist (get_inputs,
     trainers.py:332-419, and the fbpx_worklist layout).  chunk / fbins /
-    bbins: 0 = none (see include/fbpx.h).  Returns (tensors, info): a dict of
+    bbins: 0 = none (see include/fbpx.h); chunk may be a function of the pair
+    count.  Returns (tensors, info): a dict of
     int32 CUDA tensors cut to their exact sizes and the info sizes as a dict."""
     dev = x.device
     x = x.to(torch.float32).contiguous()
@@ -763,6 +764,8 @@ def device_worklist(x, xmins, xmaxs, active, pou, chunk=0, fbins=0, bbins=0):
                              xmaxs.data_ptr(), m, offsets.data_ptr(), work.data_ptr(), w0, ctypes.byref(s_c)),
           "fbpx_takes_count")
     s = int(s_c.value)
+    if callable(chunk):
+        chunk = int(chunk(s))
     max_chunks = int(L.fbpx_takes_max_chunks(m, s, chunk, fbins, bbins))
     wb = L.fbpx_takes_work_bytes(n, xd, m, s, fbins, bbins)
     del work

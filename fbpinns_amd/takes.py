@@ -208,7 +208,8 @@ def device_plan(x, active, all_params, chunk=None, fbins=None, bbins=None):
     ascending point inside a subdomain, so the trained pairs are a prefix.
     Chunks (runs of one subdomain's pairs, one partial gradient row each) end
     at every subdomain boundary, every `chunk` pairs inside a subdomain when
-    `chunk` is set, and at the bin edges.  fbins / bbins: the forward /
+    `chunk` is set (a number, or a function of the pair count), and at the bin
+    edges.  fbins / bbins: the forward /
     backward launch as that many workgroups, each over an equal share of the
     pairs (the backward over the trained prefix only), a contiguous run of
     chunks per workgroup; None = one workgroup per chunk.  Segments are the
@@ -221,7 +222,8 @@ def device_plan(x, active, all_params, chunk=None, fbins=None, bbins=None):
     dec = all_params["static"]["decomposition"]
     p = dec["subdomain"]["params"]
     pou = dec["subdomain"]["pou"].reshape(-1).round().to(torch.int32)
-    t, info = ops.device_worklist(x, p[0], p[1], np.asarray(active, dtype=np.int32), pou, int(chunk or 0),
+    t, info = ops.device_worklist(x, p[0], p[1], np.asarray(active, dtype=np.int32), pou,
+                                  chunk if callable(chunk) else int(chunk or 0),
                                   int(fbins or 0), int(bbins or 0))
     sizes = {"n_pairs": info["n_pairs"], "n_chunks": info["n_chunks"], "n_points": x.shape[0],
              "n_segs": info["n_segs"], "npou": info["npou"], "n_fbins": info["n_fbins"], "n_bbins": info["n_bbins"]}
