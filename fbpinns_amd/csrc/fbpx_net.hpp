@@ -1133,10 +1133,13 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
 
 // dW2 accumulation.  For each gradient column c the waves write the split
 // G_c and a1_c of their 16 pairs to LDS as [pair][16 units] tiles of f16 (512
-// bytes per wave, 16-unit block and piece; the lanes' 8-byte stores of a tile
-// are 512 consecutive bytes) and read them back transposed, four pairs of one
-// unit per lane (ds_read_b64_tr_b16 on 512 consecutive bytes), as A (rows o)
-// and B (columns u) operands of a contraction over pairs.
+// bytes per wave, 16-unit block and piece) and read them back transposed, four
+// pairs of one unit per lane (ds_read_b64_tr_b16), as A (rows o) and B
+// (columns u) operands of a contraction over pairs.  The four 8-byte unit
+// groups of pair p are stored in the order g ^ (p >> 2): in plain order the 16
+// pairs of a store phase share banks (16.3 cycles per ds_write_b64 and CU
+// against 6.9), and a transposed read takes each 128-byte row of four pairs
+// whole in either order (2.2 cycles).
 // H = 64: the four waves run their tiles in lockstep and share one set of
 // accumulators; wave w holds the quadrant of row blocks 2 (w >> 1) + {0, 1}
 // and column blocks 2 (w & 1) + {0, 1} and contracts it over the pairs of all
@@ -1156,6 +1159,11 @@ struct DW2Own {
   static constexpr int BS = 4 * TILE;               // of a 16-unit block (four waves)
   static constexpr int PS = NRB * BS;               // of a piece
   static constexpr int TSZ = 2 * PS;                // of a buffer
+  // float offset in a tile of pair p, units 4 g .. 4 g + 3
+  __device__ static int at(int p, int g) { return 8 * p + 2 * (g ^ (p >> 2)); }
+  // the address lane 16 q + s supplies to a transposed read, which gives it
+  // unit s of pairs 4 q .. 4 q + 3
+  __device__ static int at_tr(int lane) { return at(lane >> 2, lane & 3); }
   __device__ static int row_block(int wave, int j) { return PRIV ? j / NRB : 2 * (wave >> 1) + (j >> 1); }
   __device__ static int col_block(int wave, int j) { return PRIV ? j % NRB : 2 * (wave & 1) + (j & 1); }
 };
@@ -1229,7 +1237,7 @@ __device__ inline void dw2_shared(const float* gt, const float* at, f4* dW2) {
 }
 
 // Write this wave's split values (units x 16 pairs) to its tiles of a buffer;
-// tl = buffer + wave TILE + 8 pl + 2 g.
+// tl = buffer + wave TILE + at(pl, g).
 template <int H>
 __device__ inline void store_tile(float* tl, const Split<H>& v) {
   using O = DW2Own<H>;
@@ -1318,11 +1326,11 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // WL of the unit a reduction leaves in this lane (for G_0')
   const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)] * sc.iw;
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
-  float* const staw = sta + wave * O::TILE + 8 * pl + 2 * g;   // this wave's stores
-  float* const stgw = stg + wave * O::TILE + 8 * pl + 2 * g;
+  float* const staw = sta + wave * O::TILE + O::at(pl, g);   // this wave's stores
+  float* const stgw = stg + wave * O::TILE + O::at(pl, g);
   // dW2 reads: this wave's own tiles (PRIV) or its quadrant's blocks
-  const float* const star = sta + (O::PRIV ? wave * O::TILE : O::col_block(wave, 0) * O::BS) + 2 * lane;
-  const float* const stgr = stg + (O::PRIV ? wave * O::TILE : O::row_block(wave, 0) * O::BS) + 2 * lane;
+  const float* const star = sta + (O::PRIV ? wave * O::TILE : O::col_block(wave, 0) * O::BS) + O::at_tr(lane);
+  const float* const stgr = stg + (O::PRIV ? wave * O::TILE : O::row_block(wave, 0) * O::BS) + O::at_tr(lane);
   float* mysmall = ssmall + wave * NS * H;
   float aW1[ACC ? XD : 1][NRB][4], aWL[NRB][4], aB1[NRB][4], aB2[NRB][4];
   if constexpr (ACC) {
