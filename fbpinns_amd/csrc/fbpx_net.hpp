@@ -400,7 +400,7 @@ __device__ inline float tanh_d3(float h) {
 }
 
 // Per-subdomain layer-1 tangent tables in LDS: with zt_i[u] = W1[u][i] / sd_i,
-//   zt[i*H + u] = zt_i[u],  zt[XD*H + i*H + u] = zt_i[u]^2;
+//   zt[i*H + u] = zt_i[u],  zt[XD*H + i*H + u] = -2 zt_i[u]^2;
 // a third table zt_i[u] 2^e[i] follows them with two hidden layers (stage_two).
 template <int XD, int H, class SM, bool WAVE = false>
 __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
@@ -412,7 +412,7 @@ __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
       if (i == j) s = isd[j];
     const float z = ss[SM::W1 + u * XD + i] * s;
     zt[t] = z;
-    zt[XD * H + t] = z * z;
+    zt[XD * H + t] = -2.f * z * z;
   }
 }
 
@@ -423,7 +423,7 @@ __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
 //   w1  = ss + W1 + 4g*XD      W1[16rb + 4g + r][i]        at [(16rb + r)*XD + i]
 //   vec = ss + 4g              B1/B2/WL[16rb + 4g + r]     at [off + 16rb + r]
 //   zt  = szt + 4g             zt[i][16rb + 4g + r]        at [i*H + 16rb + r]
-//   z2, zs: the zt^2 and zt 2^e tables, same indexing
+//   z2, zs: the -2 zt^2 and zt 2^e tables, same indexing
 //   wt  = swt + lane*4         fragment f of W2 (W2Frags) at [f*256]
 //   wr  = swr + lane*4         fragment f of the transposed set, same
 struct LaneLds {
@@ -521,13 +521,13 @@ __device__ inline void layer1_stream(const LaneLds& v, const float* xh, float (*
   }
 }
 
-// Z_0 2^w = (W2 h1 + b2) 2^w.
+// Z_0 2^w = (W2 h1 + b2) 2^w (b2 is staged times 2^w).
 template <int H, class SM>
-__device__ inline void layer2_value(const LaneLds& v, const float (*h1)[4], float sw, float one, f4* Z) {
+__device__ inline void layer2_value(const LaneLds& v, const float (*h1)[4], float one, f4* Z) {
 #pragma unroll
   for (int ob = 0; ob < H / 16; ++ob) {
     const float* b2 = v.vec + SM::B2 + 16 * ob;
-    Z[ob] = f4{b2[0] * sw, b2[1] * sw, b2[2] * sw, b2[3] * sw};
+    Z[ob] = f4{b2[0], b2[1], b2[2], b2[3]};
   }
   Split<H> b;
   b.set(h1, one);
@@ -548,10 +548,10 @@ __device__ inline void tangent_split(const LaneLds& v, const float (*e1)[4], int
 // The pair's layer-1 combination of every tangent the upstream gradient
 // asks for, s = sum_i (gur_i a1_i + gur_ii a1_ii) with a1_i = e1 zt_i and
 // a1_ii = e2 zt_i^2 (e1 = 1 - h1^2, e2 = -2 h1 e1, e3 = e1 (4 - 6 e1)):
-//   s = e1 (A - 2 h1 B),  A = sum_i gur_i zt_i,  B = sum_i gur_ii zt_i^2,
-// and -1/2 times the factor that the W2^T vector vt multiplies in the layer-1
-// gradient,
-//   e2 A + e3 B = -2 rv,  rv = e1 (h1 A + (3 e1 - 2) B).
+//   s = e1 (A + h1 B),  A = sum_i gur_i zt_i,  B = sum_i gur_ii (-2 zt_i^2),
+// and -1 / (2 e1) times the factor that the W2^T vector vt multiplies in the
+// layer-1 gradient,
+//   e2 A + e3 sum_i gur_ii zt_i^2 = -2 e1 rv,  rv = h1 A + (1 - 1.5 e1) B.
 template <class S, int H>
 __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const float* gur, float (*sv)[4],
                               float (*rv)[4]) {
@@ -560,15 +560,24 @@ __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const floa
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float A = 0.f, B = 0.f;
+      bool a = false, b = false;
 #pragma unroll
       for (int i = 0; i < S::XD; ++i) {
-        if (S::has1(i)) A = fmaf(gur[S::col1(i)], v.zt[i * H + 16 * rb + r], A);
-        if (S::has2(i)) B = fmaf(gur[S::col2(i)], v.z2[i * H + 16 * rb + r], B);
+        if (S::has1(i)) {
+          const float t = v.zt[i * H + 16 * rb + r], g = gur[S::col1(i)];
+          A = a ? fmaf(g, t, A) : g * t;
+          a = true;
+        }
+        if (S::has2(i)) {
+          const float t = v.z2[i * H + 16 * rb + r], g = gur[S::col2(i)];
+          B = b ? fmaf(g, t, B) : g * t;
+          b = true;
+        }
       }
       const float h = h1[rb][r];
       const float e1 = fmaf(-h, h, 1.f);
-      sv[rb][r] = e1 * fmaf(-2.f * h, B, A);
-      rv[rb][r] = e1 * fmaf(h, A, fmaf(3.f, e1, -2.f) * B);
+      sv[rb][r] = e1 * (b ? fmaf(h, B, A) : A);
+      rv[rb][r] = b ? fmaf(h, A, fmaf(-1.5f, e1, 1.f) * B) : h * A;
     }
 }
 
@@ -673,6 +682,7 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
       if (t / H == j) e = sc.e[j];
     szt[2 * XD * H + t] = szt[t] * e;
   }
+  for (int t = threadIdx.x; t < H; t += blockDim.x) ss[SM::B2 + t] *= sc.w;
   F::store(f.a, sc.w, one, swt);
   if constexpr (WR) F::store(f.c, sc.r, one, swr);
   __syncthreads();
@@ -781,12 +791,11 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
         }
     } else {
       f4 Z0[NRB];
-      layer2_value<H, SM>(v, h1, sc.w, one, Z0);
+      layer2_value<H, SM>(v, h1, one, Z0);
       // output-layer weights times the layer-2 tanh derivatives, per element:
       // wd1 = WL f1 and wd2 = WL f1 h2 = WL f2 / (-2), so that u_i = sum wd1 Z_i
-      // and the Z_i^2 part of u_ii = sum WL (f1 Z_ii + f2 Z_i^2) costs two FMAs;
-      // every second-derivative column is accumulated without its factor -2,
-      // which is applied once to the pair's totals
+      // and the Z_i^2 part of u_ii = sum WL (f1 Z_ii + f2 Z_i^2) costs two FMAs
+      // (its factor -2 is applied to the lane's sum)
       float f1[NRB][4], wd1[NRB][4], wd2[NRB][4];
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
@@ -854,13 +863,13 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
             q1 = fmaf(wd1[ob][r], zi, q1);
             q2 = fmaf(wd2[ob][r] * zi, zi, q2);
           }
-        // + sum_u vt[u] h1 e1 zt_i^2 (the a1_ii column, factor -2 deferred)
+        // + sum_u vt[u] h1 e1 (-2 zt_i^2) (the a1_ii column)
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) q3 = fmaf(w[rb][r], v.z2[i * H + 16 * rb + r], q3);
         ur[S::col1(i)] = q1 * iz;
-        ur[S::col2(i)] = fmaf(q2 * iz, iz, q3 * sc.ir);
+        ur[S::col2(i)] = fmaf(q2 * iz, -2.f * iz, q3 * sc.ir);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -869,7 +878,7 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
     for (int c = 0; c < J; ++c) uj[c] = sum_groups(ur[c]);
     uj[0] = (uj[0] + ss[SM::BL]) * d.usd + d.umu;
 #pragma unroll
-    for (int c = 1; c < J; ++c) uj[c] *= (NH == 2 && c > S::N1) ? -2.f * d.usd : d.usd;
+    for (int c = 1; c < J; ++c) uj[c] *= d.usd;
     float wj[J], uw[J];
     window_jets<S>(xv, d, wj);
     jet_mul<S>(uj, wj, uw);
@@ -1266,7 +1275,7 @@ __device__ inline void gradient_max(const fbpx_worklist& wl, const float* gseg, 
 // Scales (all powers of two, Scales): everything linear in the upstream
 // gradient is carried times 2^k; on top of it (marked ' below)
 //   Z_i' = Z_i 2^(w + e[i]),  S' = S 2^w, and with them G_0', dWL', Q' times 2^w;
-//   vt' = vt 2^r and gz1_0' times 2^r (and -1/2 until column 0);  stored G_i times 2^-e[i], so that
+//   vt' = vt 2^r and gz1_0' times 2^r (over -2 e1 until column 0);  stored G_i times 2^-e[i], so that
 //   G_i (e1 zt_i 2^e[i])^T adds to dW2 like the other columns, and so
 //   GA_i' and gz1_i' carry 2^(r - e[i]).
 template <int XD, int H, int D1M, int D2M>
@@ -1392,7 +1401,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     float h2[NRB][4];
     {
       f4 Z0[NRB];
-      layer2_value<H, SM>(v, h1, sc.w, one, Z0);
+      layer2_value<H, SM>(v, h1, one, Z0);
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
@@ -1464,14 +1473,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         dw2_shared<H>(stgr, star, dW2);
     }
     // from here on layer 1 enters through h1 and e1 = 1 - h1^2, and the axes
-    // take layer 2 through p2 = h2 - h2^3 = -f2 / 2
+    // take layer 2 through p2 = -4 h2 (1 - h2^2) = 2 f2
     float e1[NRB][4], p2[NRB][4];
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         e1[rb][r] = fmaf(-h1[rb][r], h1[rb][r], 1.f);
-        p2[rb][r] = fmaf(-h2[rb][r] * h2[rb][r], h2[rb][r], h2[rb][r]);
+        p2[rb][r] = (-4.f * h2[rb][r]) * fmaf(-h2[rb][r], h2[rb][r], 1.f);
       }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -1499,15 +1508,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
           f4 Zi[NRB];
           frag_mul<H>(v.wt, asp, Zi);
           const float gq = (gur_b * ie_i) * (sc.iw * ie_i);   // Q' += gur_b Z_i^2 2^w
-          const float gm4 = -4.f * gq;                        // 2 gur_b f2 Z_i 2^-e[i]
           float Gi[NRB][4];
 #pragma unroll
           for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const float z = Zi[ob][r];
-              Q[ob][r] = fmaf(gq * z, z, Q[ob][r]);
-              Gi[ob][r] = gm4 * (p2[ob][r] * z);
+              const float z = Zi[ob][r], t = gq * z;
+              Q[ob][r] = fmaf(t, z, Q[ob][r]);
+              Gi[ob][r] = p2[ob][r] * t;                      // 2 gur_b f2 Z_i 2^-e[i]
             }
           gsp.set(Gi, one);
         }
@@ -1525,10 +1533,9 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
           for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const float p = (h1[rb][r] * e1[rb][r]) * v.zs[zrow + 16 * rb + r];   // -e2 zt_i 2^e[i] / 2
-              const float q = fmaf(gb4, p, ga * e1[rb][r]);
-              gzi[rb][r] = fmaf(vt[rb][r], q, e1[rb][r] * GA[rb][r]);
-              gz10[rb][r] = fmaf(p, GA[rb][r], gz10[rb][r]);
+              const float y = h1[rb][r] * v.zs[zrow + 16 * rb + r];   // -e2 zt_i 2^e[i] / (2 e1)
+              gzi[rb][r] = e1[rb][r] * fmaf(vt[rb][r], fmaf(gb4, y, ga), GA[rb][r]);
+              gz10[rb][r] = fmaf(y, GA[rb][r], gz10[rb][r]);
             }
         }
         tile_sync<O::PRIV>();
@@ -1558,12 +1565,11 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          // G_0 = f1 (gur_0 - 2 h2 S + (4 - 6 f1) Q), dWL = gur_0 h2 + f1 (S - 2 h2 Q)
           const float h = h2[ob][r];
-          const float f1 = fmaf(-h, h, 1.f);
-          const float f2 = -2.f * p2[ob][r];
-          const float f3 = f1 * fmaf(-6.f, f1, 4.f);
-          G0[ob][r] = fmaf(f3, Q[ob][r], fmaf(f2, Sx[ob][r], f1 * gur0));
-          vWL[ob][r] = fmaf(f2, Q[ob][r], fmaf(f1, Sx[ob][r], gur0 * h));
+          const float f1 = fmaf(-h, h, 1.f), m = -2.f * h;
+          G0[ob][r] = f1 * fmaf(m, Sx[ob][r], fmaf(fmaf(-6.f, f1, 4.f), Q[ob][r], gur0));
+          vWL[ob][r] = fmaf(f1, fmaf(m, Q[ob][r], Sx[ob][r]), gur0 * h);
         }
     }
     // ---- column 0: db2 += G_0, dW2 += G_0 h^T, W2~^T G_0 -> layer 1
@@ -1595,7 +1601,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) gz10[rb][r] = fmaf(-2.f, gz10[rb][r], e1[rb][r] * GA[rb][r]);
+        for (int r = 0; r < 4; ++r) gz10[rb][r] = e1[rb][r] * fmaf(-2.f, gz10[rb][r], GA[rb][r]);
     }
     // dW1[:, i] += gz1_0 xh_i (the gz1_i parts were added per axis)
     if constexpr (ACC) {
