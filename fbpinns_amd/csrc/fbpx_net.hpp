@@ -193,6 +193,11 @@ struct Scales {
 //   wr: (WL_k W2[k][16ob + pl]) 2^r, same k         (A of (diag(WL) W2)^T . g)
 // H = 16: one fragment, 4 hi then 4 lo halves per lane (k = 4g + ks).
 // Consecutive lanes read consecutive 16-byte slots: conflict-free.
+// The weights come from memory once, coalesced, through a padded f32 copy in
+// LDS (which may lie where the fragments go: they are written after the
+// barrier that follows the last read).  Gathered from memory in fragment
+// order, the staging of a chunk took 34,000 cycles at H = 64 and 17,700 at
+// H = 32.
 template <int H>
 struct W2Frags {
   static constexpr int NRB = H / 16;
@@ -200,21 +205,41 @@ struct W2Frags {
   static constexpr int NEL = H >= 32 ? 8 : 4;         // weights per item
   static constexpr int ITEMS = NQ * NRB * 64;
   static constexpr int IT = (ITEMS + 255) / 256;      // items per thread of a 256-thread workgroup
-  static constexpr int WORDS = H * H;                 // 32-bit words of one set (hi and lo)
-  float a[IT][NEL], c[IT][NEL];
+  static constexpr int LDW = H + 4;                   // row of the f32 copy: 16 rows start in 16 bank groups
+  static constexpr int TMP = H * LDW;
+  static constexpr int RAW = H * H / 256;
+  float raw[RAW], a[IT][NEL], c[IT][NEL];
   __device__ static int unit(int q, int g, int j) { return 32 * q + 16 * (j >> 2) + 4 * g + (j & 3); }
-  template <bool WT, bool WR>
-  __device__ void load(const float* w2, const float* wl) {
+  __device__ void load(const float* w2) {
+#pragma unroll
+    for (int j = 0; j < RAW; ++j) raw[j] = w2[(int)threadIdx.x + 256 * j];
+  }
+  __device__ void stash(float* tmp) const {
+#pragma unroll
+    for (int j = 0; j < RAW; ++j) {
+      const int i = (int)threadIdx.x + 256 * j;
+      tmp[(i / H) * LDW + i % H] = raw[j];
+    }
+  }
+  template <bool WR>
+  __device__ void read(const float* tmp, const float* wl) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
       const int t = (int)threadIdx.x + 256 * it, l = t & 63, g = l >> 4, pl = l & 15, f = t >> 6;
       const int q = f / NRB, ob = f % NRB;
       if (t >= ITEMS) continue;
 #pragma unroll
-      for (int j = 0; j < NEL; ++j) {
-        const int k = unit(q, g, j);
-        if (WT) a[it][j] = w2[(16 * ob + pl) * H + k];
-        if (WR) c[it][j] = w2[k * H + 16 * ob + pl] * wl[k];
+      for (int b = 0; b < NEL / 4; ++b) {
+        const f4 v = *reinterpret_cast<const f4*>(tmp + (16 * ob + pl) * LDW + unit(q, g, 4 * b));
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) a[it][4 * b + ks] = v[ks];
+      }
+      if (WR) {
+#pragma unroll
+        for (int j = 0; j < NEL; ++j) {
+          const int k = unit(q, g, j);
+          c[it][j] = tmp[k * LDW + 16 * ob + pl] * wl[k];
+        }
       }
     }
   }
@@ -271,14 +296,36 @@ __device__ inline float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
-// Largest of v over the wave, in every lane (v >= 0).
-__device__ inline float max_wave(float v) {
-  v = fmaxf(v, dpp<0x140>(v));
-  v = fmaxf(v, dpp<0x141>(v));
-  v = fmaxf(v, dpp<0x1B>(v));
-  v = fmaxf(v, dpp<0xB1>(v));
-  v = fmaxf(v, __shfl_xor(v, 16));
-  return fmaxf(v, __shfl_xor(v, 32));
+// One stage of a reduce-scatter of maxima over a DPP row (see split_stage).
+template <int N, int CTRL>
+__device__ inline void max_stage(float* v, bool upper) {
+#pragma unroll
+  for (int k = 0; k < N / 2; ++k) {
+    const float lo = v[k], hi = v[k + N / 2];
+    v[k] = fmaxf(upper ? hi : lo, dpp<CTRL>(upper ? lo : hi));
+  }
+}
+
+// Lane pl of every row gets the largest v[pl] over the wave (v >= 0), the 16
+// values together: 60 instructions, where a butterfly per value took 45 each.
+__device__ inline float max_wave16(float* v, int pl) {
+  max_stage<16, 0x140>(v, (pl >> 3) & 1);
+  max_stage<8, 0x141>(v, (pl >> 2) & 1);
+  max_stage<4, 0x1B>(v, (pl >> 1) & 1);
+  max_stage<2, 0xB1>(v, pl & 1);
+  float a = v[0], b = v[0];
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  a = b = fmaxf(a, b);
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return fmaxf(a, b);
+}
+
+// Sum of v over the 16 lanes of a row, in every lane of it.
+__device__ inline float sum_row(float v) {
+  v += dpp<0x140>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x1B>(v);
+  return v + dpp<0xB1>(v);
 }
 
 // One reduce-scatter stage over a DPP row: lanes whose stage bit is set keep
@@ -339,16 +386,16 @@ __device__ inline void half_mirror_stage(float* v) {
 #undef FBPX_DPP_PAIR
 
 // vals[rb][r] holds this lane's contribution for unit 16rb + 4g + r.  Sums
-// every entry over the 16 pair-lanes of the row and adds the total for unit
-// 16*(pl/4) + 4g + pl%4 into dst (lane pl owns that unit; no two lanes of a
-// wave share a destination).  Butterfly reduce-scatter: partners
+// every entry over the 16 pair-lanes of the row and returns the total for
+// unit 16*(pl/4) + 4g + pl%4 to lane pl < 4 NRB (lane pl owns that unit; no
+// two lanes of a wave own the same).  Butterfly reduce-scatter: partners
 // row_mirror (pl ^ 15), row_half_mirror (pl ^ 7), quad_perm[3,2,1,0]
 // (pl ^ 3), quad_perm[1,0,3,2] (pl ^ 1) flip bits 3, 2, 1, 0 of pl in turn
 // while sharing the bits above; with fewer than 16 values the top stages
 // are plain additions.  After the last stage lane pl holds the total of
-// value index pl & (V - 1), which is multiplied by post before it is added.
+// value index pl & (V - 1).
 template <int NRB>
-__device__ inline void reduce_units_to_lds(const float (*vals)[4], float* dst, int pl, int g, float post = 1.f) {
+__device__ inline float reduce_units(const float (*vals)[4], int pl) {
   constexpr int V = NRB * 4;
   float v[V];
 #pragma unroll
@@ -367,7 +414,18 @@ __device__ inline void reduce_units_to_lds(const float (*vals)[4], float* dst, i
   if constexpr (V >= 8) half_mirror_stage(v);
   split_stage<4, 0x1B>(v, (pl >> 1) & 1);
   split_stage<2, 0xB1>(v, pl & 1);
-  if (pl < V) dst[16 * (pl >> 2) + 4 * g + (pl & 3)] += v[0] * post;
+  return v[0];
+}
+
+// dst[the lane's unit of reduce_units] += v
+template <int NRB>
+__device__ inline void add_unit(float* dst, float v, int pl, int g) {
+  if (pl < 4 * NRB) dst[16 * (pl >> 2) + 4 * g + (pl & 3)] += v;
+}
+
+template <int NRB>
+__device__ inline void reduce_units_to_lds(const float (*vals)[4], float* dst, int pl, int g) {
+  add_unit<NRB>(dst, reduce_units<NRB>(vals, pl), pl, g);
 }
 
 // Hide the values of a register tile from the optimiser (an empty asm that
@@ -450,60 +508,85 @@ __device__ inline LaneLds lane_lds(const float* ss, const float* szt, const floa
   return v;
 }
 
+// The fragments of one 16-row block (all K-steps).  A pass takes its first
+// block's as an argument, so that the caller can issue those reads before the
+// vector work that forms the B operand: read inside the pass, every pass
+// began with an LDS round trip that the other wave of the SIMD did not cover.
+template <int H>
+struct FragRow {
+  static constexpr int NQ = W2Frags<H>::NQ;
+  h8v hi[NQ], lo[NQ];   // H = 16: hi[0] = 4 hi and 4 lo weights
+  __device__ void load(const float* frag, int ob) {
+    if constexpr (H >= 32) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        hi[q] = *reinterpret_cast<const h8v*>(frag + (q * (H / 16) + ob) * 512);
+        lo[q] = *reinterpret_cast<const h8v*>(frag + (q * (H / 16) + ob) * 512 + 256);
+      }
+    } else {
+      hi[0] = *reinterpret_cast<const h8v*>(frag);
+    }
+  }
+};
+
+// Block 0 of a fragment set, its reads pinned here.
+template <int H>
+__device__ inline FragRow<H> frag_head(const float* frag) {
+  FragRow<H> f;
+  f.load(frag, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  return f;
+}
+
 // Z[ob] += fragments (LDS, see W2Frags) times the split B operand.  The two
 // small products of every K-step are accumulated before the large ones, whose
 // rounding then happens once per K-step: 8.7e-8 relative error at H = 64
 // where one K-step after the other gives about 1e-7.
 template <int H>
-__device__ inline void frag_pass(const float* frag, const Split<H>& b, f4* Z) {
+__device__ inline void frag_pass(const float* frag, FragRow<H> f, const Split<H>& b, f4* Z) {
   using F = W2Frags<H>;
   constexpr int NRB = H / 16;
+  __builtin_amdgcn_sched_barrier(0);
   if constexpr (H >= 32) {
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ob = 0; ob < NRB; ++ob) {
-      h8v hi[F::NQ], lo[F::NQ];
+      FragRow<H> n;
+      if (ob + 1 < NRB) n.load(frag, ob + 1);
 #pragma unroll
       for (int q = 0; q < F::NQ; ++q) {
-        hi[q] = *reinterpret_cast<const h8v*>(frag + (q * NRB + ob) * 512);
-        lo[q] = *reinterpret_cast<const h8v*>(frag + (q * NRB + ob) * 512 + 256);
+        Z[ob] = mfma_k32(f.lo[q], b.b(b.hi, q), Z[ob]);
+        Z[ob] = mfma_k32(f.hi[q], b.b(b.lo, q), Z[ob]);
       }
 #pragma unroll
-      for (int q = 0; q < F::NQ; ++q) {
-        Z[ob] = mfma_k32(lo[q], b.b(b.hi, q), Z[ob]);
-        Z[ob] = mfma_k32(hi[q], b.b(b.lo, q), Z[ob]);
-      }
-#pragma unroll
-      for (int q = 0; q < F::NQ; ++q) Z[ob] = mfma_k32(hi[q], b.b(b.hi, q), Z[ob]);
+      for (int q = 0; q < F::NQ; ++q) Z[ob] = mfma_k32(f.hi[q], b.b(b.hi, q), Z[ob]);
+      if (ob + 1 < NRB) f = n;
     }
     // the reads of the next row block go between this block's MFMAs
     constexpr int NR = 2 * F::NQ, NM = 3 * F::NQ;
-    __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
 #pragma unroll
     for (int ob = 0; ob + 1 < NRB; ++ob) {
 #pragma unroll
       for (int j = 0; j < NR; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
     }
     __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
-    __builtin_amdgcn_sched_barrier(0);
   } else {
     // one K-step of 16: hi and lo weights side by side in a K of 32 against
     // lo twice (which adds the lo lo product) and hi twice
-    const h8v w = *reinterpret_cast<const h8v*>(frag);
-    Z[0] = mfma_k32(w, b.b(b.lo, 0), Z[0]);
-    Z[0] = mfma_k32(w, b.b(b.hi, 0), Z[0]);
+    Z[0] = mfma_k32(f.hi[0], b.b(b.lo, 0), Z[0]);
+    Z[0] = mfma_k32(f.hi[0], b.b(b.hi, 0), Z[0]);
   }
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 template <int H>
-__device__ inline void frag_mul(const float* frag, const Split<H>& b, f4* Z) {
+__device__ inline void frag_mul(const float* frag, const FragRow<H>& head, const Split<H>& b, f4* Z) {
 #pragma unroll
   for (int ob = 0; ob < H / 16; ++ob) Z[ob] = f4{0.f, 0.f, 0.f, 0.f};
-  frag_pass<H>(frag, b, Z);
+  frag_pass<H>(frag, head, b, Z);
 }
 
 // Layer 1 for this lane's units (rows 16rb + 4g + r): h = tanh(W1 xh + b1).
@@ -529,9 +612,10 @@ __device__ inline void layer2_value(const LaneLds& v, const float (*h1)[4], floa
     const float* b2 = v.vec + SM::B2 + 16 * ob;
     Z[ob] = f4{b2[0], b2[1], b2[2], b2[3]};
   }
+  const FragRow<H> head = frag_head<H>(v.wt);
   Split<H> b;
   b.set(h1, one);
-  frag_pass<H>(v.wt, b, Z);
+  frag_pass<H>(v.wt, head, b, Z);
 }
 
 // a[rb][r] zs[zrow + ...]: the B operand e1 zt_i 2^e[i] of axis i (zrow = i H).
@@ -583,9 +667,9 @@ __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const floa
 
 // Stages one subdomain of a two-hidden-layer network in LDS: the small
 // parameters, the tangent tables and the f16 fragments of W2 (and with WR of
-// diag(WL) W2), and forms the chunk's scales.  With BWD, gm[c] is this
-// thread's largest |upstream gradient| of jet column c over its share of the
-// chunk's pairs, and the gradients' scale k is chosen from a bound on every
+// diag(WL) W2), and forms the chunk's scales.  With BWD, grad_max() (called
+// once the weights' loads are issued) returns this thread's largest |upstream
+// gradient| per jet column over its share of the chunk's pairs, and the gradients' scale k is chosen from a bound on every
 // gradient value that enters a product: with R the largest absolute row sum
 // of W2, ZB_i = max_o sum_u |W2[o][u] zt_i[u]| >= |Z_i|, ZT_i = max |zt_i| and
 // g the bound on gur (window jets |w| <= 1, |w_i| <= 0.65 k_i, |w_ii| <= k_i^2
@@ -595,24 +679,31 @@ __device__ inline void pair_s(const LaneLds& v, const float (*h1)[4], const floa
 // Typical values lie 2^-8 to 2^-12 below the bound; the f16 pairs hold 22
 // bits down to 2^-17 below it and 2^-40 of the bound absolutely after that.
 // All threads of the workgroup; ends with a barrier.
-template <class S, int H, class SM, bool WR, bool BWD>
-__device__ inline void stage_two(const float* th, const Dom& d, const float* isd, const float* gm, float one,
+template <class S, int H, class SM, bool WR, bool BWD, class GradMax>
+__device__ inline void stage_two(const float* th, const Dom& d, const float* isd, GradMax grad_max, float one,
                                  float* ss, float* szt, float* swt, float* swr, float* red, Scales<S::XD>& sc) {
   constexpr int XD = S::XD, J = S::J;
   using L = Layout<XD, H, 2>;
   using F = W2Frags<H>;
-  constexpr int RW = 0, RR = 1, RS = 2, RZ = 3, RG = RZ + XD, NR = BWD ? RG + J : 2;
+  constexpr int RW = 0, RR = 1, RT = 2, RS = RT + XD, RZ = RS + 1, RG = RZ + XD, NR = BWD ? RG + J : RS;
+  static_assert(NR <= 16, "one row of lanes reduces them all");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   F f;
-  stage_small<XD, H, 2>(th, ss);
-  f.template load<true, WR>(th + L::W2, th + L::WL);
+  SmallStage<XD, H, 2> st;
+  st.load(th);
+  f.load(th + L::W2);
+  const float* gm = grad_max();
+  st.store(ss);
+  f.stash(swt);
   __syncthreads();
   stage_zt<XD, H, SM>(ss, isd, szt);
+  f.template read<WR>(swt, ss + SM::WL);
   __syncthreads();
-  float zmax[XD];
+  float m[16];
 #pragma unroll
-  for (int i = 0; i < XD; ++i) zmax[i] = max_wave(fabsf(szt[i * H + lane % H]));
-  float m[NR];
+  for (int i = 0; i < 16; ++i) m[i] = 0.f;
+#pragma unroll
+  for (int i = 0; i < XD; ++i) m[RT + i] = fabsf(szt[i * H + lane % H]);
   m[RW] = F::largest(f.a);
   m[RR] = WR ? F::largest(f.c) : 0.f;
   if constexpr (BWD) {
@@ -639,10 +730,9 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
 #pragma unroll
     for (int c = 0; c < J; ++c) m[RG + c] = gm[c];
   }
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const float v = max_wave(m[i]);
-    if (lane == 0) red[wave * 16 + i] = v;
+  {
+    const float v = max_wave16(m, lane & 15);
+    if (lane < 16) red[wave * 16 + lane] = v;
   }
   __syncthreads();
 #pragma unroll
@@ -654,7 +744,7 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
   sc.ir = pow2_inv(sc.r);
 #pragma unroll
   for (int i = 0; i < XD; ++i) {
-    sc.e[i] = uniform(pow2_scale(zmax[i], 2, 40));
+    sc.e[i] = pow2_scale(m[RT + i], 2, 40);
     sc.ie[i] = pow2_inv(sc.e[i]);
   }
   sc.k = sc.ik = 1.f;
@@ -667,9 +757,9 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
       const float k = kPi * fabsf(isd[i]);
       const float ga = m[RG + S::col1(i)], gb = S::has2(i) ? m[RG + S::col2(i)] : 0.f;
       g0 = fmaf(0.65f * k, ga, fmaf(k * k, gb, g0));
-      bS = fmaf(us * fmaf(1.3f * k, gb, ga), zmax[i], fmaf(0.77f * us * gb, zmax[i] * zmax[i], bS));
+      bS = fmaf(us * fmaf(1.3f * k, gb, ga), m[RT + i], fmaf(0.77f * us * gb, m[RT + i] * m[RT + i], bS));
       q = fmaf(2.f * us * gb, m[RZ + i] * m[RZ + i], q);
-      b = fmaxf(b, 0.77f * us * gb * m[RZ + i] * zmax[i]);
+      b = fmaxf(b, 0.77f * us * gb * m[RZ + i] * m[RT + i]);
     }
     b = fmaxf(fmaxf(b, bS), fmaf(us, g0, fmaf(0.77f * m[RS], bS, q)));
     sc.k = uniform(pow2_scale(b, 15, 100));
@@ -703,8 +793,9 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   constexpr int J = S::J, NRB = H / 16, NT = WAVE ? 4 : 1;
   __shared__ float ss_[NT][SM::N];
   __shared__ float szt_[NT][(NH == 2 ? 3 : 2) * XD * H];
-  __shared__ __attribute__((aligned(16))) float swt[NH == 2 ? H * H : 1];
-  __shared__ __attribute__((aligned(16))) float swr[NH == 2 && S::N1 > 0 ? H * H : 1];
+  // both fragment sets, or (the value alone) one, which the f32 copy outgrows
+  __shared__ __attribute__((aligned(16))) float swt[NH == 2 ? (S::N1 > 0 ? 2 * H * H : W2Frags<H>::TMP) : 1];
+  float* const swr = swt + (NH == 2 && S::N1 > 0 ? H * H : 0);
   __shared__ float red[64];
   float* const ss = ss_[T::index()];
   float* const szt = szt_[T::index()];
@@ -720,7 +811,7 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   // dependent global loads overlap the previous sub-tile's compute; with one
   // hidden layer the first sub-tile's pair index is loaded with the
   // parameter staging and its coordinates before the staging's LDS writes
-  // and barriers
+  // and barriers (with two, the registers they would hold spill others)
   float xn[XD];
   const int k0 = beg + wave * 16 + pl;
   if constexpr (NH == 1) {
@@ -746,7 +837,8 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
     stage_zt<XD, H, SM, WAVE>(ss, isd, szt);
     T::sync();
   } else {
-    stage_two<S, H, SM, (S::N1 > 0), false>(th, d, isd, nullptr, one, ss, szt, swt, swr, red, sc);
+    stage_two<S, H, SM, (S::N1 > 0), false>(th, d, isd, [] { return (const float*)nullptr; }, one, ss, szt, swt, swr,
+                                            red, sc);
   }
 
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
@@ -820,9 +912,10 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
       float e1[NRB][4], ve[NRB][4], w[NRB][4];
       if constexpr (S::N1 > 0) {
         f4 vt[NRB];
+        const FragRow<H> head = frag_head<H>(v.wr);
         Split<H> b;
         b.set(f1, one);
-        frag_mul<H>(v.wr, b, vt);
+        frag_mul<H>(v.wr, head, b, vt);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb)
@@ -849,9 +942,10 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
         }
         f4 Zi[NRB];
         {
+          const FragRow<H> head = frag_head<H>(v.wt);
           Split<H> b;
           tangent_split<H>(v, e1, i * H, one, b);
-          frag_mul<H>(v.wt, b, Zi);
+          frag_mul<H>(v.wt, head, b, Zi);
         }
         const float iz = sc.iw * sc.ie[i];
         float q1 = 0.f, q2 = 0.f, q3 = 0.f;
@@ -1258,18 +1352,36 @@ __device__ inline void store_tile(float* tl, const Split<H>& v) {
 }
 
 // This thread's largest |gseg| per jet column over its share of the chunk's
-// pairs (stage_two reduces them over the workgroup).
+// pairs (stage_two reduces them over the workgroup), in two halves so that the
+// other loads of the chunk's start go between them: indices() issues the loads
+// of the first FIRST segment indices, values() the rows'.
 template <int J>
-__device__ inline void gradient_max(const fbpx_worklist& wl, const float* gseg, int beg, int end, float* gm) {
+struct GradientMax {
+  static constexpr int FIRST = 4;
+  int seg[FIRST];
+  float m[J];
+  __device__ void indices(const fbpx_worklist& wl, int beg, int end) {
 #pragma unroll
-  for (int c = 0; c < J; ++c) gm[c] = 0.f;
-#pragma unroll 4
-  for (int k = beg + (int)threadIdx.x; k < end; k += 256) {
-    const int seg = wl.pair_seg[k];
-#pragma unroll
-    for (int c = 0; c < J; ++c) gm[c] = fmaxf(gm[c], fabsf(gseg[(size_t)seg * J + c]));
+    for (int j = 0; j < FIRST; ++j) {
+      const int k = beg + (int)threadIdx.x + 256 * j;
+      seg[j] = wl.pair_seg[k < end ? k : beg];   // a repeated pair does not change the maximum
+    }
   }
-}
+  __device__ void values(const fbpx_worklist& wl, const float* gseg, int beg, int end) {
+#pragma unroll
+    for (int c = 0; c < J; ++c) m[c] = 0.f;
+#pragma unroll
+    for (int j = 0; j < FIRST; ++j)
+#pragma unroll
+      for (int c = 0; c < J; ++c) m[c] = fmaxf(m[c], fabsf(gseg[(size_t)seg[j] * J + c]));
+#pragma unroll 4
+    for (int k = beg + (int)threadIdx.x + 256 * FIRST; k < end; k += 256) {
+      const int sk = wl.pair_seg[k];
+#pragma unroll
+      for (int c = 0; c < J; ++c) m[c] = fmaxf(m[c], fabsf(gseg[(size_t)sk * J + c]));
+    }
+  }
+};
 
 // [xd, h, h, 1]: hidden-to-hidden layer on MFMA, streamed one axis at a time.
 // Scales (all powers of two, Scales): everything linear in the upstream
@@ -1280,8 +1392,7 @@ __device__ inline void gradient_max(const fbpx_worklist& wl, const float* gseg, 
 //   GA_i' and gz1_i' carry 2^(r - e[i]).
 template <int XD, int H, int D1M, int D2M>
 __device__ inline void bwd_two(const float* theta, const float* dom, const float* x, const fbpx_worklist& wl,
-                               const float* gseg, float* partial, int chunk, float gs, const AdamFold& af,
-                               const float* bc) {
+                               const float* gseg, float* partial, int chunk, float gs) {
   using S = Schema<XD, D1M, D2M>;
   using L = Layout<XD, H, 2>;
   using SM = Small<XD, H, 2>;
@@ -1295,14 +1406,13 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   constexpr bool ACC = DW2Own<H>::PRIV && XD <= 2;
   constexpr int AXIS_UNROLL = H == 64 || ACC ? XD : 1;
   static_assert(H >= 16 && H <= 64, "hidden width 16, 32 or 64");
-  static_assert(2 * O::TSZ >= L::P, "the gradient row reuses the transpose buffers");
   __shared__ float ss[SM::N];
   __shared__ float szt[3 * XD * H];
-  __shared__ __attribute__((aligned(16))) float swt[H * H];
-  __shared__ __attribute__((aligned(16))) float swr[H * H];
+  __shared__ __attribute__((aligned(16))) float swt[2 * H * H];
+  float* const swr = swt + H * H;
   __shared__ __attribute__((aligned(16))) float strans[2 * O::TSZ];
   __shared__ float ssmall[4 * NS * H];
-  __shared__ float sbl[64];
+  __shared__ float sbl[4];
   __shared__ float red[64];
   float* sta = strans;            // a1 columns
   float* stg = strans + O::TSZ;   // G columns
@@ -1311,8 +1421,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   const int beg = wl.chunk_start[chunk];
   const int end = wl.chunk_start[chunk + 1];
   const float* th = theta + (size_t)model * L::P;
-  for (int i = threadIdx.x; i < 4 * NS * H; i += blockDim.x) ssmall[i] = 0.f;
-  if (threadIdx.x < 64) sbl[threadIdx.x] = 0.f;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int pl = lane & 15, g = lane >> 4;
+  // the index loads of the gradient maxima and of the first tile, ahead of
+  // everything that waits
+  GradientMax<J> gmax;
+  gmax.indices(wl, beg, end);
+  const int k0 = beg + wave * 16 + pl;
+  const int p0 = wl.pair_point[k0 < end ? k0 : beg], seg0 = wl.pair_seg[k0 < end ? k0 : beg];
   Dom d;
   load_dom(dom, model, d);
   float mu[XD], isd[XD];
@@ -1323,15 +1439,20 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   }
   const float one = opaque_one();
   Scales<XD> sc;
-  {
-    float gm[J];
-    gradient_max<J>(wl, gseg, beg, end, gm);
-    stage_two<S, H, SM, true, true>(th, d, isd, gm, one, ss, szt, swt, swr, red, sc);
-  }
+  float xn[XD], gUn[J];   // the next tile's point and upstream jets
+  stage_two<S, H, SM, true, true>(
+      th, d, isd,
+      [&]() -> const float* {
+#pragma unroll
+        for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
+#pragma unroll
+        for (int c = 0; c < J; ++c) gUn[c] = k0 < end ? gseg[(size_t)seg0 * J + c] : 0.f;
+        gmax.values(wl, gseg, beg, end);
+        return gmax.m;
+      },
+      one, ss, szt, swt, swr, red, sc);
   d.usd *= sc.k;
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int pl = lane & 15, g = lane >> 4;
   // WL of the unit a reduction leaves in this lane (for G_0')
   const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)] * sc.iw;
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
@@ -1356,6 +1477,10 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
   for (int j = 0; j < O::NOB; ++j) dW2[j] = f4{0.f, 0.f, 0.f, 0.f};
   float dbl = 0.f;
+  // !ACC: this lane's unit totals over the chunk (reduce_units), by kind
+  float small[NS];
+#pragma unroll
+  for (int j = 0; j < NS; ++j) small[j] = 0.f;
 
   // with shared dW2 blocks every wave runs the same number of tiles (barriers
   // below); with wave-private blocks (H <= 32) a wave runs only the tiles in
@@ -1365,17 +1490,6 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // each tile's point and upstream jets are fetched during the previous tile
   // (indices at the start of its column-0 phase, data before its last dW2
   // column), so the two dependent global loads do not stall the tile start
-  float xn[XD], gUn[J];
-  {
-    const int k = beg + wave * 16 + pl;
-    const int kk = k < end ? k : beg;
-    const int p = wl.pair_point[kk];
-    const int seg = wl.pair_seg[kk];
-#pragma unroll
-    for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p * XD + i];
-#pragma unroll
-    for (int c = 0; c < J; ++c) gUn[c] = k < end ? gseg[(size_t)seg * J + c] : 0.f;
-  }
   for (int t = 0; t < ntile; ++t) {
     float xv[XD], xh[XD];
 #pragma unroll
@@ -1435,13 +1549,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       float rv[NRB][4];
       Split<H> ssp, fsp;
       {
-        float sv[NRB][4];
-        pair_s<S, H>(v, h1, gur, sv, rv);
-        ssp.set(sv, one);
-      }
-      {
+        const FragRow<H> head = frag_head<H>(v.wt);
+        {
+          float sv[NRB][4];
+          pair_s<S, H>(v, h1, gur, sv, rv);
+          ssp.set(sv, one);
+        }
         f4 Sv[NRB];
-        frag_mul<H>(v.wt, ssp, Sv);
+        frag_mul<H>(v.wt, head, ssp, Sv);
 #pragma unroll
         for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
@@ -1450,6 +1565,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
             Q[ob][r] = 0.f;
           }
       }
+      const FragRow<H> head = frag_head<H>(v.wr);
       {
         float f1[NRB][4];
 #pragma unroll
@@ -1461,7 +1577,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       tile_sync<O::PRIV>();   // the previous tile's column has been consumed
       store_tile<H>(staw, ssp);
       store_tile<H>(stgw, fsp);
-      frag_mul<H>(v.wr, fsp, vt);
+      frag_mul<H>(v.wr, head, fsp, vt);
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
@@ -1503,10 +1619,12 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       float gzi[NRB][4];
       if (two) {
         Split<H> gsp, asp;
+        FragRow<H> head = frag_head<H>(v.wt);
         tangent_split<H>(v, e1, zrow, one, asp);
         {
           f4 Zi[NRB];
-          frag_mul<H>(v.wt, asp, Zi);
+          frag_mul<H>(v.wt, head, asp, Zi);
+          head = frag_head<H>(v.wr);
           const float gq = (gur_b * ie_i) * (sc.iw * ie_i);   // Q' += gur_b Z_i^2 2^w
           float Gi[NRB][4];
 #pragma unroll
@@ -1527,7 +1645,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         store_tile<H>(stgw, gsp);
         {
           f4 GA[NRB];
-          frag_mul<H>(v.wr, gsp, GA);
+          frag_mul<H>(v.wr, head, gsp, GA);
           const float gb4 = -4.f * gur_b * ie_i * ie_i, ga = gur_a * ie_i;
 #pragma unroll
           for (int rb = 0; rb < NRB; ++rb)
@@ -1556,7 +1674,11 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
           for (int r = 0; r < 4; ++r) aW1[i][rb][r] = fmaf(gzi[rb][r], post, aW1[i][rb][r]);
       } else {
-        reduce_units_to_lds<NRB>(gzi, mysmall + (K_W1 + i) * H, pl, g, post);
+        {
+          const float r = reduce_units<NRB>(gzi, pl) * post;
+#pragma unroll
+          for (int j = 0; j < XD; ++j) small[K_W1 + j] += j == i ? r : 0.f;
+        }
       }
     }
     if constexpr (S::N1 > 0) {
@@ -1583,10 +1705,11 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) aB2[ob][r] += G0[ob][r];
     } else {
-      reduce_units_to_lds<NRB>(G0, mysmall + K_B2 * H, pl, g, wl_red);
+      small[K_B2] = fmaf(reduce_units<NRB>(G0, pl), wl_red, small[K_B2]);
     }
     {
       Split<H> gsp, hsp;
+      const FragRow<H> head = frag_head<H>(v.wr);
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
@@ -1597,7 +1720,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       store_tile<H>(staw, hsp);
       store_tile<H>(stgw, gsp);
       f4 GA[NRB];
-      frag_mul<H>(v.wr, gsp, GA);
+      frag_mul<H>(v.wr, head, gsp, GA);
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
@@ -1624,10 +1747,10 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) vv[rb][r] = gz10[rb][r] * xh[i];
-        reduce_units_to_lds<NRB>(vv, mysmall + (K_W1 + i) * H, pl, g, sc.ir);
+        small[K_W1 + i] = fmaf(reduce_units<NRB>(vv, pl), sc.ir, small[K_W1 + i]);
       }
-      reduce_units_to_lds<NRB>(vWL, mysmall + K_WL * H, pl, g, sc.iw);
-      reduce_units_to_lds<NRB>(gz10, mysmall + K_B1 * H, pl, g, sc.ir);
+      small[K_WL] = fmaf(reduce_units<NRB>(vWL, pl), sc.iw, small[K_WL]);
+      small[K_B1] = fmaf(reduce_units<NRB>(gz10, pl), sc.ir, small[K_B1]);
     }
     // the next tile's point and upstream jets, in flight during the last dW2 column
     __builtin_amdgcn_sched_barrier(0);
@@ -1643,36 +1766,52 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     // (the next tile's first column has a barrier before its stores)
   }
 
-  // ---- end of chunk: the transpose buffers become the gradient row
+  // ---- end of chunk: the gradient row from the waves' sums
   if constexpr (ACC) {
 #pragma unroll
-    for (int i = 0; i < XD; ++i) reduce_units_to_lds<NRB>(aW1[i], mysmall + (K_W1 + i) * H, pl, g);
-    reduce_units_to_lds<NRB>(aWL, mysmall + K_WL * H, pl, g, sc.iw);
-    reduce_units_to_lds<NRB>(aB1, mysmall + K_B1 * H, pl, g, sc.ir);
-    reduce_units_to_lds<NRB>(aB2, mysmall + K_B2 * H, pl, g, wl_red);
+    for (int i = 0; i < XD; ++i) small[K_W1 + i] = reduce_units<NRB>(aW1[i], pl);
+    small[K_WL] = reduce_units<NRB>(aWL, pl) * sc.iw;
+    small[K_B1] = reduce_units<NRB>(aB1, pl) * sc.ir;
+    small[K_B2] = reduce_units<NRB>(aB2, pl) * wl_red;
   }
-  if (g == 0) sbl[wave * 16 + pl] = dbl;
-  __syncthreads();
-  float* sacc = strans;
-  for (int i = threadIdx.x; i < L::P; i += blockDim.x) sacc[i] = 0.f;
-  __syncthreads();
-  // H = 64: the waves hold disjoint dW2 blocks and write them at once;
-  // H <= 32: every wave holds every block over its own pairs, summed wave by
-  // wave in a fixed order
-  for (int w = 0; w < (O::PRIV ? nw : 1); ++w) {
-    if (!O::PRIV || wave == w) {
 #pragma unroll
-      for (int j = 0; j < O::NOB; ++j) {
-        const int ob = O::row_block(wave, j);
-        const int col = 16 * O::col_block(wave, j) + pl;
+  for (int j = 0; j < NS; ++j)
+    if (pl < 4 * NRB) mysmall[j * H + 16 * (pl >> 2) + 4 * g + (pl & 3)] = small[j];
+  dbl = sum_row(dbl);
+  if (lane == 0) sbl[wave] = dbl;
+  __syncthreads();   // every wave is done with the tiles
+  // H = 64: the waves hold disjoint dW2 blocks; H <= 32: every wave holds every
+  // block over its own pairs, one copy per wave, summed in wave order below
+  constexpr int NC = O::PRIV ? 4 : 1;
+  static_assert(NC * H * H <= 2 * O::TSZ, "the dW2 copies reuse the tile buffers");
+  {
+    float* const sw = strans + (O::PRIV ? wave * H * H : 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          sacc[L::W2 + (16 * ob + 4 * g + r) * H + col] += dW2[j][r] * v.vec[SM::WL + 16 * ob + r];
-      }
+    for (int j = 0; j < O::NOB; ++j) {
+      const int ob = O::row_block(wave, j);
+      const int col = 16 * O::col_block(wave, j) + pl;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sw[(16 * ob + 4 * g + r) * H + col] = dW2[j][r] * v.vec[SM::WL + 16 * ob + r];
     }
-    __syncthreads();
   }
-  finish_row<XD, H, 2>(sacc, ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs * sc.ik, af, model, bc);
+  __syncthreads();
+  float* const out = partial + (size_t)chunk * L::P;
+  const float post = gs * sc.ik;
+  for (int i = threadIdx.x; i < H * H; i += 256) {
+    float s = strans[i];
+#pragma unroll
+    for (int w = 1; w < NC; ++w) s += strans[w * H * H + i];
+    out[L::W2 + i] = s * post;
+  }
+  for (int t = threadIdx.x; t < NS * H; t += 256) {
+    const int kind = t / H, u = t % H;
+    const float s = (ssmall[t] + ssmall[NS * H + t]) + (ssmall[2 * NS * H + t] + ssmall[3 * NS * H + t]);
+    const int dst = kind == K_WL ? L::WL + u : kind == K_B1 ? L::B1 + u : kind == K_B2 ? L::B2 + u
+                                                                       : L::W1 + u * XD + (kind - K_W1);
+    out[dst] = s * post;
+  }
+  if (threadIdx.x == 0) out[L::BL] = ((sbl[0] + sbl[1]) + (sbl[2] + sbl[3])) * post;
 }
 
 // g_scale: NULL, or d L / d loss when gseg holds the segment gradients at
@@ -1707,7 +1846,7 @@ bwd_kernel(const float* __restrict__ theta, const float* __restrict__ dom, const
     if constexpr (NH == 1)
       bwd_one<XD, H, D1M, D2M, WAVE, ADAM>(theta, dom, x, wl, gseg, partial, chunk, gs, af, sbc, first);
     else
-      bwd_two<XD, H, D1M, D2M>(theta, dom, x, wl, gseg, partial, chunk, gs, af, sbc);
+      bwd_two<XD, H, D1M, D2M>(theta, dom, x, wl, gseg, partial, chunk, gs);
     first = false;
   }
   if constexpr (ADAM) {
