@@ -78,12 +78,11 @@ struct Team {
   }
 };
 
-// stage_small in two halves, so that a chunk's other first loads can be
-// issued between them: load() issues every global load of the team's share
-// (registers), store() writes them to LDS.  Teams of 64 or more threads (IT
-// covers a 64-thread team; wider teams leave later slots unused).  The
-// one-hidden-layer chunks use it; the two-hidden-layer ones keep the plain
-// loop, whose register schedule their main loops are tuned against.
+// The network's small parameters to LDS in two halves, so that a chunk's other
+// first loads can be issued between them: load() issues every global load of
+// the team's share (registers), store() writes them to LDS.  Teams of 64 or
+// more threads (IT covers a 64-thread team; wider teams leave later slots
+// unused).
 template <int XD, int H, int NH, bool WAVE = false>
 struct SmallStage {
   using L = Layout<XD, H, NH>;
@@ -105,14 +104,6 @@ struct SmallStage {
     }
   }
 };
-
-template <int XD, int H, int NH, bool WAVE = false>
-__device__ inline void stage_small(const float* th, float* ss) {
-  using L = Layout<XD, H, NH>;
-  using SM = Small<XD, H, NH>;
-  for (int i = Team<WAVE>::tid(); i < SM::N; i += Team<WAVE>::size())
-    ss[i] = th[i < SM::B2 ? i : (i < SM::WL ? L::B2 + (i - SM::B2) : L::WL + (i - SM::WL))];
-}
 
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
@@ -417,15 +408,12 @@ __device__ inline float reduce_units(const float (*vals)[4], int pl) {
   return v[0];
 }
 
-// dst[the lane's unit of reduce_units] += v
-template <int NRB>
-__device__ inline void add_unit(float* dst, float v, int pl, int g) {
-  if (pl < 4 * NRB) dst[16 * (pl >> 2) + 4 * g + (pl & 3)] += v;
-}
-
-template <int NRB>
-__device__ inline void reduce_units_to_lds(const float (*vals)[4], float* dst, int pl, int g) {
-  add_unit<NRB>(dst, reduce_units<NRB>(vals, pl), pl, g);
+// dst[kind * h + the lane's unit of reduce_units] = v[kind]
+template <int NRB, int NK>
+__device__ inline void store_units(float* dst, const float* v, int h, int pl, int g) {
+#pragma unroll
+  for (int j = 0; j < NK; ++j)
+    if (pl < 4 * NRB) dst[j * h + 16 * (pl >> 2) + 4 * g + (pl & 3)] = v[j];
 }
 
 // Hide the values of a register tile from the optimiser (an empty asm that
@@ -1041,55 +1029,53 @@ __device__ inline void pair_upstream(const float* gU, const float* xv, const Dom
   for (int c = 0; c < J; ++c) gur[c] *= d.usd;
 }
 
-// Chunk epilogue shared by both network depths: sums the per-wave small
-// gradients (ssmall[wave][kind][u]; kinds WL, B1, W1[:, i], B2) and the
-// per-lane output-bias partials (sbl) into sacc, then writes the row.
-template <int XD, int H, int NH, bool WAVE = false, bool ADAM = false>
-__device__ inline void finish_row(float* sacc, const float* ssmall, const float* sbl, int nw, float* out,
-                                  float gs, const AdamFold& af, int model, const float* bc) {
-  using L = Layout<XD, H, NH>;
+// Chunk epilogue of one hidden layer: the gradient row from the waves' unit
+// totals (ssmall[wave][kind][u]; kinds WL, B1, W1[:, i]) and output-bias sums
+// (sbl[wave]), written out, or with ADAM applied to the subdomain's row.
+template <int XD, int H, bool WAVE = false, bool ADAM = false>
+__device__ inline void finish_row(const float* ssmall, const float* sbl, int nw, float* out, float gs,
+                                  const AdamFold& af, int model, const float* bc) {
+  using L = Layout<XD, H, 1>;
   using T = Team<WAVE>;
-  constexpr int NS = (NH == 2 ? 3 : 2) + XD;
+  constexpr int NS = 2 + XD;
   constexpr int K_WL = 0, K_B1 = 1, K_W1 = 2;
-  for (int t = T::tid(); t < NS * H; t += T::size()) {
-    const int kind = t / H, u = t % H;
-    float s = 0.f;
-    for (int w = 0; w < nw; ++w) s += ssmall[(w * NS + kind) * H + u];
-    int dst;
-    if (kind == K_WL) dst = L::WL + u;
-    else if (kind == K_B1) dst = L::B1 + u;
-    else if (kind < K_W1 + XD) dst = L::W1 + u * XD + (kind - K_W1);
-    else dst = L::B2 + u;
-    sacc[dst] += s;
-  }
-  if (T::tid() == 0) {
-    float s = 0.f;
-    for (int q = 0; q < nw * 16; ++q) s += sbl[q];
-    sacc[L::BL] = s;
-  }
-  T::sync();
-  // gs: d L / d loss for a gseg at unit upstream gradient (the row is linear
-  // in gseg; 1 leaves it unchanged)
-  if constexpr (!ADAM) {
-    for (int i = T::tid(); i < L::P; i += T::size()) out[i] = sacc[i] * gs;
-    return;
-  }
-  // the row is its subdomain's whole gradient: Adam on it in place, as
-  // fbpx_adam_rows_partial updates a row from its one chunk row
   const size_t r0 = (size_t)model * L::P;
   for (int i = T::tid(); i < L::P; i += T::size()) {
-    const float row = sacc[i] * gs;
-    float gi = 0.f;
-    gi += row;
-    float p = af.theta[r0 + i], m = af.mu[r0 + i], v = af.nu[r0 + i];
-    adam_elem(p, m, v, gi, bc[0], bc[1], af.k);
-    af.theta[r0 + i] = p;
-    af.mu[r0 + i] = m;
-    af.nu[r0 + i] = v;
+    float row = 0.f;
+    if (i == L::BL) {
+      for (int w = 0; w < nw; ++w) row += sbl[w];
+    } else {
+      const int at = i < L::B1 ? (K_W1 + i % XD) * H + i / XD
+                               : i < L::WL ? K_B1 * H + (i - L::B1) : K_WL * H + (i - L::WL);
+      for (int w = 0; w < nw; ++w) row += ssmall[w * NS * H + at];
+    }
+    // gs: d L / d loss for a gseg at unit upstream gradient (the row is linear
+    // in gseg; 1 leaves it unchanged)
+    row *= gs;
+    if constexpr (!ADAM) {
+      out[i] = row;
+    } else {
+      // the row is its subdomain's whole gradient: Adam on it in place, as
+      // fbpx_adam_rows_partial updates a row from its one chunk row
+      float gi = 0.f;
+      gi += row;
+      float p = af.theta[r0 + i], m = af.mu[r0 + i], v = af.nu[r0 + i];
+      adam_elem(p, m, v, gi, bc[0], bc[1], af.k);
+      af.theta[r0 + i] = p;
+      af.mu[r0 + i] = m;
+      af.nu[r0 + i] = v;
+    }
   }
 }
 
 // [xd, h, 1]: no hidden-to-hidden layer; waves work independently.
+// Bound by latency: a chunk of a training step has one to three sub-tiles, so
+// the load chains and the chunk's ends weigh as much as the arithmetic.  The
+// unit gradients therefore stay in registers until the chunk's end (an LDS
+// read-modify-write per sub-tile and kind before), the output-bias sum is a
+// wave reduction (one thread's 16 reads per wave before), and the loads run
+// ahead (below): a 28-chunk step of 5,000 points 41.0 -> 37.5 us, 30 chunks of
+// 1,000 points 25.7 -> 24.4, 7,022 wave chunks of 20 pairs 51.5 -> 50.8.
 // WAVE: the chunk is one wave's (its own LDS copies, its slices of the
 // per-wave sums).
 // ADAM: bc holds the bias corrections, formed by the team's first lane in
@@ -1105,15 +1091,13 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   constexpr int J = S::J, NRB = H / 16, NS = 2 + XD, NT = WAVE ? 4 : 1;
   constexpr int K_WL = 0, K_B1 = 1, K_W1 = 2;
   __shared__ float ss_[NT][SM::N];
-  __shared__ float sacc_[NT][L::P];
   __shared__ float ssmall_[4 * NS * H];   // per wave (four teams of one wave with WAVE)
-  __shared__ float sbl_[64];
+  __shared__ float sbl_[4];
   __shared__ float szt_[NT][2 * XD * H];
   float* const ss = ss_[T::index()];
-  float* const sacc = sacc_[T::index()];
   float* const szt = szt_[T::index()];
   float* const ssmall = ssmall_ + T::index() * NS * H;
-  float* const sbl = sbl_ + T::index() * 16;
+  float* const sbl = sbl_ + T::index();
 
   const int model = wl.chunk_model[chunk];
   const int beg = wl.chunk_start[chunk];
@@ -1123,19 +1107,23 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   const float* th = theta + (size_t)model * L::P;
   const int lane = threadIdx.x & 63, wave = T::wave(), nw = T::nw();
   const int pl = lane & 15, g = lane >> 4;
-  // pair point and segment of this lane's pair in the next sub-tile: loaded
-  // one sub-tile ahead, the first with the parameter staging
+  // each sub-tile's pair indices are loaded two sub-tiles ahead and its point
+  // and upstream jets one ahead, so that a sub-tile waits on neither of the
+  // two dependent loads; the first ones are issued around the parameter
+  // staging (a chunk is often only one or two sub-tiles)
   int pn, sn;
-  {
-    const int k0 = beg + wave * 16 + pl;
-    const int kk = k0 < end ? k0 : beg;
-    pn = wl.pair_point[kk];
-    sn = wl.pair_seg[kk];
-  }
-  stage_small<XD, H, 1, WAVE>(th, ss);
-  for (int i = T::tid(); i < L::P; i += T::size()) sacc[i] = 0.f;
-  for (int i = T::tid(); i < T::nw() * NS * H; i += T::size()) ssmall[i] = 0.f;
-  if (T::tid() < T::nw() * 16) sbl[T::tid()] = 0.f;
+  const int k0 = beg + wave * 16 + pl, k1 = k0 + nw * 16;
+  const int p0 = wl.pair_point[k0 < end ? k0 : beg], s0 = wl.pair_seg[k0 < end ? k0 : beg];
+  pn = wl.pair_point[k1 < end ? k1 : beg];
+  sn = wl.pair_seg[k1 < end ? k1 : beg];
+  SmallStage<XD, H, 1, WAVE> st;
+  st.load(th);
+  float xn[XD], gUn[J];
+#pragma unroll
+  for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
+#pragma unroll
+  for (int c = 0; c < J; ++c) gUn[c] = k0 < end ? gseg[(size_t)s0 * J + c] : 0.f;
+  st.store(ss);
   Dom d;
   load_dom(dom, model, d);
   if constexpr (ADAM) {
@@ -1153,30 +1141,33 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
 
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, ss, ss, pl, g);
   float* mysmall = ssmall + wave * NS * H;
-  float dbl = 0.f;
+  float dbl = 0.f, small[NS];
+#pragma unroll
+  for (int j = 0; j < NS; ++j) small[j] = 0.f;
   for (int base = beg + wave * 16; base < end; base += nw * 16) {
     // one wave per chunk: the weights and window tangents are read from LDS
     // per sub-tile rather than held in registers across the loop (95 VGPRs
     // instead of 120 at [1, 32, 1]: five waves per SIMD instead of four)
     if constexpr (WAVE) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int k = base + pl;
-    const bool valid = k < end;   // else the pair at beg with a zero upstream gradient
-    const int p = pn, seg = sn;
-    {
-      const int kn = k + nw * 16;
-      const int kk = kn < end ? kn : beg;
-      pn = wl.pair_point[kk];
-      sn = wl.pair_seg[kk];
-    }
+    // lanes past the end run the pair at beg with a zero upstream gradient
     float xv[XD], xh[XD];
 #pragma unroll
     for (int i = 0; i < XD; ++i) {
-      xv[i] = x[(size_t)p * XD + i];
+      xv[i] = xn[i];
       xh[i] = (xv[i] - mu[i]) * isd[i];
     }
     float gur[J], gU[J];
 #pragma unroll
-    for (int c = 0; c < J; ++c) gU[c] = valid ? gseg[(size_t)seg * J + c] : 0.f;
+    for (int c = 0; c < J; ++c) gU[c] = gUn[c];
+    if (base + nw * 16 < end) {
+      const int kn = base + nw * 16 + pl, k2 = kn + nw * 16;
+#pragma unroll
+      for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
+#pragma unroll
+      for (int c = 0; c < J; ++c) gUn[c] = kn < end ? gseg[(size_t)sn * J + c] : 0.f;
+      pn = wl.pair_point[k2 < end ? k2 : beg];
+      sn = wl.pair_seg[k2 < end ? k2 : beg];
+    }
     pair_upstream<S>(gU, xv, d, gur);
     if (g == 0) dbl += gur[0];
     float h1[NRB][4];
@@ -1224,14 +1215,16 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
           }
           vv[rb][r] = t;
         }
-      reduce_units_to_lds<NRB>(vv, mysmall + (K_W1 + i) * H, pl, g);
+      small[K_W1 + i] += reduce_units<NRB>(vv, pl);
     }
-    reduce_units_to_lds<NRB>(vWL, mysmall + K_WL * H, pl, g);
-    reduce_units_to_lds<NRB>(gz10, mysmall + K_B1 * H, pl, g);
+    small[K_WL] += reduce_units<NRB>(vWL, pl);
+    small[K_B1] += reduce_units<NRB>(gz10, pl);
   }
-  if (g == 0) sbl[wave * 16 + pl] = dbl;
+  store_units<NRB, NS>(mysmall, small, H, pl, g);
+  dbl = sum_row(dbl);
+  if (lane == 0) sbl[wave] = dbl;
   T::sync();
-  finish_row<XD, H, 1, WAVE, ADAM>(sacc, ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs, af, model, bc);
+  finish_row<XD, H, WAVE, ADAM>(ssmall, sbl, nw, partial + (size_t)chunk * L::P, gs, af, model, bc);
 }
 
 // dW2 accumulation.  For each gradient column c the waves write the split
@@ -1774,9 +1767,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     small[K_B1] = reduce_units<NRB>(aB1, pl) * sc.ir;
     small[K_B2] = reduce_units<NRB>(aB2, pl) * wl_red;
   }
-#pragma unroll
-  for (int j = 0; j < NS; ++j)
-    if (pl < 4 * NRB) mysmall[j * H + 16 * (pl >> 2) + 4 * g + (pl & 3)] = small[j];
+  store_units<NRB, NS>(mysmall, small, H, pl, g);
   dbl = sum_row(dbl);
   if (lane == 0) sbl[wave] = dbl;
   __syncthreads();   // every wave is done with the tiles
