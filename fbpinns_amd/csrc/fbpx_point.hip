@@ -459,6 +459,23 @@ bool schema_supported(int xd, int d1, int d2) {
 //
 // (optax.adam's element update, AdamConst and adam_bias: fbpx_common.hpp)
 
+// Sum of element e of the chunk rows [c0, c1), in ascending order.  Bound by
+// latency: eight rows are read at once, the last one again past the end (the
+// Adam launch of 150 subdomains' 178,000 elements 5.2 -> 4.9 us against four).
+__device__ inline float chunk_rows_sum(const float* __restrict__ partial, int P, int e, int c0, int c1) {
+  constexpr int B = 8;
+  float g = 0.f;
+  for (int c = c0; c < c1; c += B) {
+    float t[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) t[j] = partial[(size_t)(c + j < c1 ? c + j : c1 - 1) * P + e];
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (c + j < c1) g += t[j];
+  }
+  return g;
+}
+
 __global__ void __launch_bounds__(256) reduce_rows_kernel(int P, const float* __restrict__ partial,
                                                           const int32_t* __restrict__ rows,
                                                           const int32_t* __restrict__ rcs, int n_rows,
@@ -466,12 +483,7 @@ __global__ void __launch_bounds__(256) reduce_rows_kernel(int P, const float* __
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)n_rows * P) return;
   const int row = (int)(idx / P), e = (int)(idx % P);
-  float g = 0.f;
-  // loads unrolled so several chunk rows are in flight; the sum stays in
-  // ascending chunk order
-#pragma unroll 4
-  for (int c = rcs[row]; c < rcs[row + 1]; ++c) g += partial[(size_t)c * P + e];
-  grad[(size_t)rows[row] * P + e] = g;
+  grad[(size_t)rows[row] * P + e] = chunk_rows_sum(partial, P, e, rcs[row], rcs[row + 1]);
 }
 
 // Each workgroup's thread 0 reads the step count once, at the start.  With
@@ -481,8 +493,14 @@ __global__ void __launch_bounds__(256) reduce_rows_kernel(int P, const float* __
 // launch.  Nothing else is ordered against the count, so no fence is needed.
 // Launches of at most this many workgroups finish their own reduction (or
 // the step count) in the last workgroup; larger ones use a second launch,
-// which costs less than a fence and an atomic per workgroup.
+// which costs less than an atomic per workgroup on one address (14 ns each).
 constexpr int kSingleLaunchBlocks = 256;
+// adam_rows_kernel advances the step count in its own launch up to this many
+// elements, in workgroups of 1,024 threads (a quarter of the counts): 303,360
+// elements 9.2 -> 7.6 us against a second one-thread launch, 178,000 9.2 ->
+// 4.9.  Past it (wave: 3.9 million) the counts would cost more than the 4 us of
+// the second launch, and 256 threads per workgroup are faster.
+constexpr int64_t kAdamFoldElems = 320 * 1024;
 
 __device__ inline void adam_count_step(int32_t* count, int32_t* count_done) {
   if (count_done != nullptr && threadIdx.x == 0 && atomicAdd(count_done, 1) == (int)gridDim.x - 1) {
@@ -494,20 +512,20 @@ __device__ inline void adam_count_step(int32_t* count, int32_t* count_done) {
 // PARTIAL false: the gradient rows grad; true: the per-chunk partial rows,
 // summed per listed row as fbpx_reduce_rows sums them (ascending chunks,
 // same unrolling), so that both forms give the same update bit for bit.
-// One element per thread: the launch covers n_rows * P (n_rows >= 1).  The
-// first wave forms the bias corrections while its first loads are in
-// flight, so that the count's round trip and the powf do not come before
-// them.
-template <bool PARTIAL>
-__global__ void __launch_bounds__(256) adam_rows_kernel(float* __restrict__ theta, float* __restrict__ mu,
-                                                        float* __restrict__ nu, int P,
-                                                        const float* __restrict__ grad,
-                                                        const float* __restrict__ partial,
-                                                        const int32_t* __restrict__ rcs,
-                                                        const int32_t* __restrict__ rows, int n_rows,
-                                                        int32_t* count, int32_t* count_done, AdamConst k) {
+// One element per thread: the launch of T-thread workgroups covers n_rows * P
+// (n_rows >= 1).  The first wave forms the bias corrections while its first
+// loads are in flight, so that the count's round trip and the powf do not
+// come before them.
+template <bool PARTIAL, int T>
+__global__ void __launch_bounds__(T) adam_rows_kernel(float* __restrict__ theta, float* __restrict__ mu,
+                                                      float* __restrict__ nu, int P,
+                                                      const float* __restrict__ grad,
+                                                      const float* __restrict__ partial,
+                                                      const int32_t* __restrict__ rcs,
+                                                      const int32_t* __restrict__ rows, int n_rows,
+                                                      int32_t* count, int32_t* count_done, AdamConst k) {
   __shared__ float sbc[2];
-  const int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);   // n_rows * P < 2^31 - 255
+  const int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);   // n_rows * P < 2^31 - T
   const bool on = idx < n_rows * P;
   // two dependent round trips: the row and its chunk range (past the end:
   // row 0's, unused), then the parameter, its moments and the gradient (or
@@ -529,12 +547,10 @@ __global__ void __launch_bounds__(256) adam_rows_kernel(float* __restrict__ thet
     p = theta[i];
     m = mu[i];
     v = nu[i];
-    if constexpr (!PARTIAL) {
+    if constexpr (!PARTIAL)
       gi = grad[i];
-    } else {
-#pragma unroll 4
-      for (int c = c0; c < c1; ++c) gi += partial[(size_t)c * P + e];
-    }
+    else
+      gi = chunk_rows_sum(partial, P, e, c0, c1);
   }
   __syncthreads();
   if (on) {
@@ -630,11 +646,52 @@ struct ResidualArgs {
 // Points per thread and loop trip: independent loads in flight per thread.
 constexpr int kResUnroll = 4;
 
+// Threads of a residual workgroup.  Bound by latency and, in the last
+// workgroup's sum, by the workgroups' counts on one address (14 ns each):
+// 262,144 points of three terms take 8.6 us in 256 workgroups of 256 threads,
+// 7.2 in 128 of 512, 7.8 in 64 of 1,024 (11.6 in 256 of 256 with a fence
+// before each count); 68,000 points of a set of two 9.0, 8.5, 9.5 (10.0).
+constexpr int kResThreads = 512;
+
 // The factor 1 of a term without a second (or any) column is read from here
 // at index 0, so that every factor is an unconditional load and all of a
 // point's loads are in flight at once (a load behind a branch on the term
 // count would be waited for before the next one is issued).
 __device__ float kResOne[1] = {1.f};
+
+// A workgroup's partials for the grid's last workgroup, without a fence: a
+// device-scope release writes the XCD's whole L2 back, and every workgroup
+// would wait for it.  put_partials (one thread) exchanges the n <= N values
+// in at device scope and waits for the exchanges to return, so that they have
+// been performed before the thread goes on to count its workgroup
+// (last_arrival); the last workgroup, whose own count came after every
+// other's, reads with device-scope loads (get_partial).
+template <int N>
+__device__ inline void put_partials(float* at, const float* v, int n = N) {
+  float old[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    old[j] = j < n ? __hip_atomic_exchange(at + j, v[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    asm volatile("" ::"v"(old[j]) : "memory");   // waits for the returned value; keeps the order
+}
+
+__device__ inline float get_partial(const float* at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Whether this workgroup is the last of the grid to count itself on done.
+// Every thread of every workgroup calls it, after thread 0 has put the
+// workgroup's partials.
+__device__ inline bool last_arrival(int32_t* done) {
+  __shared__ int last;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  __syncthreads();
+  return last;
+}
 
 // out[j] = scale * sum over the grid's workgroups b of scratch[b * ncol + j]
 // (plus out[j]'s value on entry when acc), computed by the last workgroup to
@@ -644,18 +701,10 @@ __device__ float kResOne[1] = {1.f};
 // has written the workgroup's partials.
 __device__ inline void last_block_sum(const float* scratch, int ncol, float scale, float* out, bool acc,
                                       int32_t* done, float* sm) {
-  __shared__ int last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();   // this workgroup's partials are visible before it is counted
-    last = atomicAdd(done, 1) == (int)gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();     // every other workgroup's partials are visible here
+  if (!last_arrival(done)) return;
   for (int j = 0; j < ncol; ++j) {
     float v = 0.f;
-    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) v += scratch[b * ncol + j];
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) v += get_partial(scratch + b * ncol + j);
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) out[j] = acc ? out[j] + scale * t : scale * t;
     __syncthreads();
@@ -808,11 +857,12 @@ __device__ inline float residual_block(int64_t n, const ResidualArgs& a, const f
 // loss[0] (scaled, added to it on entry when acc) by the last workgroup when
 // done is given, else by sum_columns_kernel.
 template <int NT, bool GRAD>
-__global__ void __launch_bounds__(256) residual_kernel(int64_t n, ResidualArgs a, const float* __restrict__ coef,
-                                                       float* __restrict__ r, float* scratch, float scale,
-                                                       float* __restrict__ loss, bool acc, int32_t* done,
-                                                       float w2n) {
-  __shared__ float sm[4];   // one partial per wave of the 256-thread block
+__global__ void __launch_bounds__(kResThreads) residual_kernel(int64_t n, ResidualArgs a,
+                                                               const float* __restrict__ coef,
+                                                               float* __restrict__ r, float* scratch, float scale,
+                                                               float* __restrict__ loss, bool acc, int32_t* done,
+                                                               float w2n) {
+  __shared__ float sm[kResThreads / 64];   // one partial per wave
   const float tot = residual_block<NT, GRAD>(n, a, coef, r, w2n, blockIdx.x, gridDim.x, sm);
   if (done && gridDim.x == 1) {
     // the only workgroup: its total is the sum that last_block_sum would
@@ -820,7 +870,12 @@ __global__ void __launch_bounds__(256) residual_kernel(int64_t n, ResidualArgs a
     if (threadIdx.x == 0) loss[0] = acc ? loss[0] + scale * tot : scale * tot;
     return;
   }
-  if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
+  if (threadIdx.x == 0) {
+    if (done)
+      put_partials<1>(scratch + blockIdx.x, &tot);
+    else
+      scratch[blockIdx.x] = tot;
+  }
   if (done) last_block_sum(scratch, 1, scale, loss, acc, done, sm);
 }
 
@@ -853,7 +908,7 @@ __device__ inline void residual_set_sum(const float* scratch, const ResidualSums
   float total = acc ? loss[0] : 0.f;
   for (int i = 0; i < q.n_res; ++i) {
     float v = 0.f;
-    for (int b = q.b0[i] + threadIdx.x; b < q.b0[i + 1]; b += blockDim.x) v += scratch[b];
+    for (int b = q.b0[i] + threadIdx.x; b < q.b0[i + 1]; b += blockDim.x) v += get_partial(scratch + b);
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) total = (i == 0 && !acc) ? q.scale[i] * t : total + q.scale[i] * t;
     __syncthreads();
@@ -864,10 +919,9 @@ __device__ inline void residual_set_sum(const float* scratch, const ResidualSums
 // NTMAX: the largest term count of the set (2, 4 or 8), so that a set of
 // short residuals is not compiled with the registers of eight-term ones.
 template <int NTMAX, bool GRAD>
-__global__ void __launch_bounds__(256) residual_set_kernel(ResidualSet s_arg, float* scratch,
+__global__ void __launch_bounds__(kResThreads) residual_set_kernel(ResidualSet s_arg, float* scratch,
                                                            float* __restrict__ loss, bool acc, int32_t* done) {
-  __shared__ float sm[4];   // one partial per wave of the 256-thread block
-  __shared__ int last;
+  __shared__ float sm[kResThreads / 64];   // one partial per wave
   // the set is read where the launch placed it (the first kernel argument,
   // at the start of the argument segment): indexed by the residual, a copy
   // of the argument would be made in per-lane stack memory
@@ -886,17 +940,13 @@ __global__ void __launch_bounds__(256) residual_set_kernel(ResidualSet s_arg, fl
     FBPX_SET_CASE(5) FBPX_SET_CASE(6) FBPX_SET_CASE(7) FBPX_SET_CASE(8)
   }
 #undef FBPX_SET_CASE
-  if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
-  if (!done) return;
-  // the last workgroup to finish sums the partials (as last_block_sum)
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();   // this workgroup's partial is visible before it is counted
-    last = atomicAdd(done, 1) == (int)gridDim.x - 1;
+  if (!done) {
+    if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
+    return;
   }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();     // every other workgroup's partial is visible here
+  // the last workgroup to finish sums the partials (as last_block_sum)
+  if (threadIdx.x == 0) put_partials<1>(scratch + blockIdx.x, &tot);
+  if (!last_arrival(done)) return;
   residual_set_sum(scratch, s.sums, loss, acc, sm);
   if (threadIdx.x == 0) atomicExch(done, 0);
 }
@@ -910,12 +960,13 @@ __global__ void __launch_bounds__(256) residual_set_sum_kernel(const float* __re
 // gcol[f][k] = s r[k] d r / d col_f, s = g_loss[0] * w2n; scratch[block *
 // NT + t] = sum over the block's points of s r term_t.
 template <int NT>
-__global__ void __launch_bounds__(256) residual_backward_kernel(int64_t n, ResidualArgs a,
-                                                                const float* __restrict__ coef,
-                                                                const float* __restrict__ r, float w2n,
-                                                                const float* __restrict__ g_loss, float* scratch,
-                                                                float* __restrict__ gcoef, int32_t* done) {
-  __shared__ float sm[4];   // one partial per wave of the 256-thread block
+__global__ void __launch_bounds__(kResThreads) residual_backward_kernel(int64_t n, ResidualArgs a,
+                                                                        const float* __restrict__ coef,
+                                                                        const float* __restrict__ r, float w2n,
+                                                                        const float* __restrict__ g_loss,
+                                                                        float* scratch, float* __restrict__ gcoef,
+                                                                        int32_t* done) {
+  __shared__ float sm[kResThreads / 64];   // one partial per wave
   const TermCols<NT> c = term_cols<NT>(a);
   const float sc = g_loss[0] * w2n;
   float cf[NT], acc[NT];
@@ -947,14 +998,17 @@ __global__ void __launch_bounds__(256) residual_backward_kernel(int64_t n, Resid
   const bool only = done && gridDim.x == 1;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const float tot = block_tree_sum(acc[t], sm);
-    if (threadIdx.x == 0) {
-      if (only)
-        gcoef[t] = tot;
-      else
-        scratch[blockIdx.x * NT + t] = tot;
-    }
+    acc[t] = block_tree_sum(acc[t], sm);
     __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    if (done && !only) {
+      put_partials<NT>(scratch + blockIdx.x * NT, acc);
+    } else {
+      float* const to = only ? gcoef : scratch + blockIdx.x * NT;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) to[t] = acc[t];
+    }
   }
   if (done && !only) last_block_sum(scratch, NT, 1.f, gcoef, false, done, sm);
 }
@@ -1045,7 +1099,7 @@ __device__ inline void pou_loss_total(const float* part, int nb, const PouLossAr
   float total = 0.f;   // thread 0's
   for (int i = 0; i < a.n_res; ++i) {
     float v = 0.f;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) v += part[b * a.n_res + i];
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) v += get_partial(part + b * a.n_res + i);
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) {
       const float term = a.scale[i] * t;
@@ -1196,18 +1250,16 @@ __global__ void __launch_bounds__(256) pou_loss_kernel(fbpx_worklist wl, const f
     }
     return;
   }
-  if (threadIdx.x == 0)
-    for (int i = 0; i < a.n_res; ++i) part[blockIdx.x * a.n_res + i] = tot[i];
-  if (done) {
-    __shared__ int last;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      __threadfence();   // this workgroup's partials are visible before it is counted
-      last = atomicAdd(done, 1) == (int)gridDim.x - 1;
+  if (threadIdx.x == 0) {
+    if (done) {
+      put_partials<NR>(part + blockIdx.x * a.n_res, tot, a.n_res);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        if (i < a.n_res) part[blockIdx.x * a.n_res + i] = tot[i];
     }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();     // every other workgroup's partials are visible here
+  }
+  if (done && last_arrival(done)) {
     pou_loss_total(part, gridDim.x, a, loss, acc, sm);
     if (threadIdx.x == 0) atomicExch(done, 0);
   }
@@ -1354,18 +1406,24 @@ static int adam_rows_launch(void* stream, float* theta, float* mu, float* nu, in
     set_error("adam_rows: null pointer");
     return FBPX_EINVAL;
   }
-  // the count is advanced in this launch (an atomic per workgroup) for a
-  // few workgroups, by a second one-thread launch otherwise
-  const int64_t total = (int64_t)n_rows * P, nb = (total + 255) / 256;
-  const bool fold = count_done && nb <= kSingleLaunchBlocks;
-  if (grad)
-    hipLaunchKernelGGL(adam_rows_kernel<false>, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)stream, theta, mu,
-                       nu, P, grad, partial, rcs, rows, n_rows, count, fold ? count_done : nullptr,
-                       adam_const(lr, b1, b2, eps));
+  const int64_t total = (int64_t)n_rows * P;
+  const bool small = total <= kAdamFoldElems, fold = count_done && small;
+  const int T = small ? 1024 : 256;
+  const unsigned nb = (unsigned)((total + T - 1) / T);
+  int32_t* const cd = fold ? count_done : nullptr;
+  const AdamConst k = adam_const(lr, b1, b2, eps);
+#define FBPX_ADAM_ROWS(PARTIAL, T)                                                                            \
+  hipLaunchKernelGGL((adam_rows_kernel<PARTIAL, T>), dim3(nb), dim3(T), 0, (hipStream_t)stream, theta, mu, nu, \
+                     P, grad, partial, rcs, rows, n_rows, count, cd, k)
+  if (grad && small)
+    FBPX_ADAM_ROWS(false, 1024);
+  else if (grad)
+    FBPX_ADAM_ROWS(false, 256);
+  else if (small)
+    FBPX_ADAM_ROWS(true, 1024);
   else
-    hipLaunchKernelGGL(adam_rows_kernel<true>, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)stream, theta, mu, nu,
-                       P, grad, partial, rcs, rows, n_rows, count, fold ? count_done : nullptr,
-                       adam_const(lr, b1, b2, eps));
+    FBPX_ADAM_ROWS(true, 256);
+#undef FBPX_ADAM_ROWS
   int rc = hip_check(hipGetLastError(), "adam_rows");
   if (rc == FBPX_OK && count_done && !fold) rc = fbpx_count_increment(stream, count);
   return rc;
@@ -1501,7 +1559,7 @@ int fbpx_affine_jets_backward(void* stream, const fbpx_net* net, int32_t n, int3
 }
 
 static int residual_blocks(int64_t n) {
-  const int64_t need = (n + 256 * kResUnroll - 1) / (256 * kResUnroll);
+  const int64_t need = (n + kResThreads * kResUnroll - 1) / (kResThreads * kResUnroll);
   return (int)(need < FBPX_RESIDUAL_BLOCKS ? need : FBPX_RESIDUAL_BLOCKS);
 }
 
@@ -1562,17 +1620,17 @@ static int residual_loss_launch(void* stream, int64_t n, int32_t n_cols, const f
   const float scale = weight / (float)n;
   const float w2n = 2.f * weight / (float)n;   // as in the transpose's launch
   const bool acc = accumulate != 0;
-  // the last-workgroup sum (a fence and an atomic per workgroup) pays off
+  // the last-workgroup sum (an atomic per workgroup on one address) pays off
   // against a second launch only for a few workgroups
   int32_t* const one = nb <= kSingleLaunchBlocks ? done : nullptr;
 #define FBPX_RES_CASE(NT)                                                                                     \
   case NT:                                                                                                    \
     if (gcol)                                                                                                 \
-      hipLaunchKernelGGL((residual_kernel<NT, true>), dim3(nb), dim3(256), 0, s, n, a, coef, r, scratch, scale, \
-                         loss, acc, one, w2n);                                                                \
+      hipLaunchKernelGGL((residual_kernel<NT, true>), dim3(nb), dim3(kResThreads), 0, s, n, a, coef, r,       \
+                         scratch, scale, loss, acc, one, w2n);                                                \
     else                                                                                                      \
-      hipLaunchKernelGGL((residual_kernel<NT, false>), dim3(nb), dim3(256), 0, s, n, a, coef, r, scratch,     \
-                         scale, loss, acc, one, w2n);                                                         \
+      hipLaunchKernelGGL((residual_kernel<NT, false>), dim3(nb), dim3(kResThreads), 0, s, n, a, coef, r,      \
+                         scratch, scale, loss, acc, one, w2n);                                                \
     break;
   switch (n_terms) {
     FBPX_RES_CASE(1) FBPX_RES_CASE(2) FBPX_RES_CASE(3) FBPX_RES_CASE(4)
@@ -1649,10 +1707,10 @@ int fbpx_residual_losses(void* stream, int32_t n_res, const fbpx_residual* res, 
   for (int i = 0; i < n_res; ++i) ntmax = s.nt[i] > ntmax ? s.nt[i] : ntmax;
 #define FBPX_SET_LAUNCH(NTMAX)                                                                                \
   if (grad)                                                                                                   \
-    hipLaunchKernelGGL((residual_set_kernel<NTMAX, true>), dim3(nb), dim3(256), 0, st, s, scratch, loss, acc, \
+    hipLaunchKernelGGL((residual_set_kernel<NTMAX, true>), dim3(nb), dim3(kResThreads), 0, st, s, scratch, loss, acc, \
                        one);                                                                                  \
   else                                                                                                        \
-    hipLaunchKernelGGL((residual_set_kernel<NTMAX, false>), dim3(nb), dim3(256), 0, st, s, scratch, loss, acc, \
+    hipLaunchKernelGGL((residual_set_kernel<NTMAX, false>), dim3(nb), dim3(kResThreads), 0, st, s, scratch, loss, acc, \
                        one);
   if (ntmax <= 2) {
     FBPX_SET_LAUNCH(2)
@@ -1683,7 +1741,7 @@ int fbpx_residual_loss_backward(void* stream, int64_t n, int32_t n_cols, const f
   const float w2n = 2.f * weight / (float)n;
 #define FBPX_RES_CASE(NT)                                                                                 \
   case NT:                                                                                                \
-    hipLaunchKernelGGL(residual_backward_kernel<NT>, dim3(nb), dim3(256), 0, s, n, a, coef, r, w2n, g_loss, \
+    hipLaunchKernelGGL(residual_backward_kernel<NT>, dim3(nb), dim3(kResThreads), 0, s, n, a, coef, r, w2n, g_loss, \
                        scratch, gcoef, one);                                                              \
     break;
   int32_t* const one = gcoef && nb <= kSingleLaunchBlocks ? done : nullptr;
