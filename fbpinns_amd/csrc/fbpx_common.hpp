@@ -110,17 +110,33 @@ __device__ inline void half_angle_cs(float phi, float& c, float& s) {
 // c = cos(phi), s = sin(phi) (half-angle identities, k = pi / sd):
 //   ((1 + cos theta) / 2)^2 = c^4,   d/dx = -2 k s c^3,
 //   d2/dx2 = k^2 (sin^2 theta - cos theta (1 + cos theta)) / 2 = k^2 c^2 (3 - 4 c^2).
+//
+// The per-axis constants of one subdomain's box are the caller's (WindowBox):
+// kept in scalar registers by the chunk kernels.
+template <int XD>
+struct WindowBox {
+  float mu[XD], hk[XD], n2k[XD], kk[XD];   // centre, k / 2, -2 k, k^2
+  __device__ inline explicit WindowBox(const Dom& d) {
+#pragma unroll
+    for (int i = 0; i < XD; ++i) {
+      const float sd = (d.xmax[i] - d.xmin[i]) * 0.5f;
+      const float k = kPi / sd;
+      mu[i] = (d.xmin[i] + d.xmax[i]) * 0.5f;
+      hk[i] = 0.5f * k;
+      n2k[i] = -2.f * k;
+      kk[i] = k * k;
+    }
+  }
+};
+
 template <class S>
-__device__ inline void window_jets(const float* x, const Dom& d, float* w) {
+__device__ inline void window_jets(const float* x, const WindowBox<S::XD>& b, float flag, float* w) {
   constexpr int XD = S::XD;
   float c[XD], c1[XD], c2[XD];
 #pragma unroll
   for (int i = 0; i < XD; ++i) {
-    const float mu = (d.xmin[i] + d.xmax[i]) * 0.5f;
-    const float sd = (d.xmax[i] - d.xmin[i]) * 0.5f;
-    const float k = kPi / sd;
     // clamped so that rounding at the box edge cannot leave the fitted range
-    const float phi = __builtin_amdgcn_fmed3f((x[i] - mu) * (0.5f * k), -0.5f * kPi, 0.5f * kPi);
+    const float phi = __builtin_amdgcn_fmed3f((x[i] - b.mu[i]) * b.hk[i], -0.5f * kPi, 0.5f * kPi);
     float co, si;
     half_angle_cs(phi, co, si);
     // 1 + cos(theta) = 2 c^2 rounds to 0 in the reference's float32 form once
@@ -129,22 +145,27 @@ __device__ inline void window_jets(const float* x, const Dom& d, float* w) {
     // trainers.py:166) as in the reference
     const float cc = fabsf(co) <= 0x1p-13f ? 0.f : co * co;
     c[i] = cc * cc;
-    c1[i] = (-2.f * k) * (si * (cc * co));
-    c2[i] = (k * k) * (cc * fmaf(-4.f, cc, 3.f));
+    c1[i] = b.n2k[i] * (si * (cc * co));
+    c2[i] = b.kk[i] * (cc * fmaf(-4.f, cc, 3.f));
   }
   float prod = 1.f;
 #pragma unroll
   for (int i = 0; i < XD; ++i) prod *= c[i];
-  w[0] = d.flag * prod + (1.f - d.flag);
+  w[0] = flag * prod + (1.f - flag);
 #pragma unroll
   for (int i = 0; i < XD; ++i) {
     float others = 1.f;
 #pragma unroll
     for (int j = 0; j < XD; ++j)
       if (j != i) others *= c[j];
-    if (S::has1(i)) w[S::col1(i)] = d.flag * c1[i] * others;
-    if (S::has2(i)) w[S::col2(i)] = d.flag * c2[i] * others;
+    if (S::has1(i)) w[S::col1(i)] = flag * c1[i] * others;
+    if (S::has2(i)) w[S::col2(i)] = flag * c2[i] * others;
   }
+}
+
+template <class S>
+__device__ inline void window_jets(const float* x, const Dom& d, float* w) {
+  window_jets<S>(x, WindowBox<S::XD>(d), d.flag, w);
 }
 
 // Leibniz product of two jets (uw = u * w), diagonal second order.

@@ -168,6 +168,24 @@ __device__ inline float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
+// A chunk's box: its window constants and 1 / sd, wave-uniform values that
+// every tile reads, in scalar registers (as results of vector arithmetic they
+// would hold four or five vector registers per axis across the tile loop).
+template <int XD>
+struct ChunkBox : WindowBox<XD> {
+  float isd[XD];
+  __device__ inline explicit ChunkBox(const Dom& d) : WindowBox<XD>(d) {
+#pragma unroll
+    for (int i = 0; i < XD; ++i) {
+      isd[i] = uniform(1.f / ((d.xmax[i] - d.xmin[i]) / 2.f));
+      this->mu[i] = uniform(this->mu[i]);
+      this->hk[i] = uniform(this->hk[i]);
+      this->n2k[i] = uniform(this->n2k[i]);
+      this->kk[i] = uniform(this->kk[i]);
+    }
+  }
+};
+
 // Powers of two of one chunk (all exact):
 //   W2 2^w and (diag(WL) W2) 2^r are at most 2^14 in LDS,
 //   zt_i 2^e[i] is at most 4 (table ztS),
@@ -452,10 +470,15 @@ template <int XD, int H, class SM, bool WAVE = false>
 __device__ inline void stage_zt(const float* ss, const float* isd, float* zt) {
   for (int t = Team<WAVE>::tid(); t < XD * H; t += Team<WAVE>::size()) {
     const int i = t / H, u = t % H;
-    float s = isd[0];
+    float s = 0.f;
 #pragma unroll
-    for (int j = 1; j < XD; ++j)
-      if (i == j) s = isd[j];
+    for (int j = 0; j < XD; ++j) {
+      // opaque: selects between the values, not between their addresses
+      // (which would put the array in memory)
+      float sj = isd[j];
+      asm("" : "+v"(sj));
+      s = i == j ? sj : s;
+    }
     const float z = ss[SM::W1 + u * XD + i] * s;
     zt[t] = z;
     zt[XD * H + t] = -2.f * z * z;
@@ -766,6 +789,21 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
   __syncthreads();
 }
 
+// What depends on a pair alone (its window jets, normalised point, upstream
+// gradient) would be formed by each of the four lane groups that share a
+// 16-pair sub-tile.  The two-layer kernels form it for four sub-tiles at once,
+// one pair per lane (lane group g: the g-th sub-tile), and keep it as rows of
+// ROW floats in LDS, per wave; a sub-tile reads its 16 rows back (a row stride
+// of 12 words: 16 four-word reads without a bank conflict).  Vector instructions
+// per sub-tile, backward: 1,962 -> 1,870 (3D, h = 64), 661 -> 625 (2D, h = 32, one
+// second derivative).  With the box constants in scalar registers, of 7.2 million
+// pairs (3D, h = 64): backward 3,360 -> 3,210 us, forward 1,195 -> 1,160; 412,000
+// pairs: 272 -> 249 and 105 -> 99.  2D, h = 32: forward 71.3 -> 69.2 us, backward 150 ->
+// 148.5 (946,000 pairs), 44.3 -> 43.0 and 68 -> 63.4 (614,000).
+struct PairRows {
+  static constexpr int ROW = 12, WAVE = 64 * ROW;
+};
+
 // ------------------------------------------------------------------ forward
 
 // One chunk of the forward (a run of pairs of one subdomain).
@@ -778,13 +816,14 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   using SM = Small<XD, H, NH>;
   using T = Team<WAVE>;
   static_assert(!WAVE || NH == 1, "one wave per chunk: one-hidden-layer networks");
+  using R = PairRows;
   constexpr int J = S::J, NRB = H / 16, NT = WAVE ? 4 : 1;
   __shared__ float ss_[NT][SM::N];
   __shared__ float szt_[NT][(NH == 2 ? 3 : 2) * XD * H];
   // both fragment sets, or (the value alone) one, which the f32 copy outgrows
   __shared__ __attribute__((aligned(16))) float swt[NH == 2 ? (S::N1 > 0 ? 2 * H * H : W2Frags<H>::TMP) : 1];
   float* const swr = swt + (NH == 2 && S::N1 > 0 ? H * H : 0);
-  __shared__ float red[64];
+  __shared__ __attribute__((aligned(16))) float srow[NH == 2 ? 4 * R::WAVE : 1];
   float* const ss = ss_[T::index()];
   float* const szt = szt_[T::index()];
 
@@ -794,12 +833,13 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   const float* th = theta + (size_t)model * L::P;
   const int lane = threadIdx.x & 63, wave = T::wave(), nw = T::nw();
   const int pl = lane & 15, g = lane >> 4;
-  // the point of each sub-tile is fetched one sub-tile ahead (pair index at
-  // the top of the previous sub-tile, coordinates in its middle), so the two
-  // dependent global loads overlap the previous sub-tile's compute; with one
-  // hidden layer the first sub-tile's pair index is loaded with the
-  // parameter staging and its coordinates before the staging's LDS writes
-  // and barriers (with two, the registers they would hold spill others)
+  // the points of each sub-tile (NH == 2: of each four, PairRows) are fetched
+  // one sub-tile ahead (pair index at the top of the previous sub-tile,
+  // coordinates in its middle), so the two dependent global loads overlap the
+  // previous sub-tile's compute; with one hidden layer the first sub-tile's
+  // pair index is loaded with the parameter staging and its coordinates before
+  // the staging's LDS writes and barriers (with two, the registers they would
+  // hold spill others)
   float xn[XD];
   const int k0 = beg + wave * 16 + pl;
   if constexpr (NH == 1) {
@@ -812,12 +852,9 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   }
   Dom d;
   load_dom(dom, model, d);
-  float mu[XD], isd[XD];
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    mu[i] = (d.xmax[i] + d.xmin[i]) / 2.f;
-    isd[i] = 1.f / ((d.xmax[i] - d.xmin[i]) / 2.f);
-  }
+  const ChunkBox<XD> box(d);
+  const float* const mu = box.mu;
+  const float* const isd = box.isd;
   const float one = opaque_one();
   Scales<XD> sc;
   if constexpr (NH == 1) {
@@ -826,26 +863,59 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
     T::sync();
   } else {
     stage_two<S, H, SM, (S::N1 > 0), false>(th, d, isd, [] { return (const float*)nullptr; }, one, ss, szt, swt, swr,
-                                            red, sc);
+                                            srow, sc);
   }
 
   const LaneLds v = lane_lds<XD, H, SM>(ss, szt, swt, swr, pl, g);
-  if constexpr (NH == 2) {
-    const int p0 = wl.pair_point[k0 < end ? k0 : beg];
+  // NH == 2: this lane's row (window jets, normalised point, slot) of the next
+  // four sub-tiles
+  static_assert(J + XD + 1 <= R::ROW, "a pair's row");
+  float* const rows = srow + (NH == 2 ? wave * R::WAVE : 0);
+  const auto put_row = [&](const float* xp, int slot) {
+    float wj[J];
+    window_jets<S>(xp, box, d.flag, wj);
+    float* const to = rows + lane * R::ROW;
 #pragma unroll
-    for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
+    for (int c = 0; c < J; ++c) to[c] = wj[c];
+#pragma unroll
+    for (int i = 0; i < XD; ++i) to[J + i] = (xp[i] - mu[i]) * isd[i];
+    to[J + XD] = __int_as_float(slot);
+    Team<true>::sync();
+  };
+  if constexpr (NH == 2) {
+    const int kq = beg + wave * 16 + g * 64 + pl;
+    const int pq = wl.pair_point[kq < end ? kq : beg], sq = wl.pair_slot[kq < end ? kq : beg];
+#pragma unroll
+    for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pq * XD + i];
+    put_row(xn, sq);
   }
-  for (int base = beg + wave * 16; base < end; base += nw * 16) {
+  int t = 0;   // sub-tile of this wave
+  for (int base = beg + wave * 16; base < end; base += nw * 16, ++t) {
     const int k = base + pl;
     const bool valid = k < end;
-    const int slot = wl.pair_slot[valid ? k : beg];
     const int kn = k + nw * 16;
-    const int pn = wl.pair_point[kn < end ? kn : beg];
     float xv[XD], xh[XD];
+    int pn, slot;
+    const float* const row = rows + (NH == 2 ? ((t & 3) * 16 + pl) * R::ROW : 0);
+    const int kq = kn + g * 64;
+    const bool refill = NH == 2 && (t & 3) == 3;
+    int slotn;
+    float xq[XD];
+    if constexpr (NH == 2) {
 #pragma unroll
-    for (int i = 0; i < XD; ++i) {
-      xv[i] = xn[i];
-      xh[i] = (xv[i] - mu[i]) * isd[i];
+      for (int i = 0; i < XD; ++i) xh[i] = row[J + i];
+      if (refill) {
+        pn = wl.pair_point[kq < end ? kq : beg];
+        slotn = wl.pair_slot[kq < end ? kq : beg];
+      }
+    } else {
+      slot = wl.pair_slot[valid ? k : beg];
+      pn = wl.pair_point[kn < end ? kn : beg];
+#pragma unroll
+      for (int i = 0; i < XD; ++i) {
+        xv[i] = xn[i];
+        xh[i] = (xv[i] - mu[i]) * isd[i];
+      }
     }
     float h1[NRB][4];
     layer1_stream<XD, H, SM>(v, xh, h1);
@@ -888,8 +958,10 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
           wd1[ob][r] = wlu * f1[ob][r];
           wd2[ob][r] = wd1[ob][r] * h;
         }
+      if (refill) {
 #pragma unroll
-      for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
+        for (int i = 0; i < XD; ++i) xq[i] = x[(size_t)pn * XD + i];
+      }
       __builtin_amdgcn_sched_barrier(0);
       // sum_o WL f1 Z_c = sum_u vt[u] a1_c[u] with vt = (diag(WL) W2)^T f1: one
       // transposed pass per sub-tile replaces the Z_ii passes of every axis and
@@ -962,12 +1034,24 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
 #pragma unroll
     for (int c = 1; c < J; ++c) uj[c] *= d.usd;
     float wj[J], uw[J];
-    window_jets<S>(xv, d, wj);
+    if constexpr (NH == 2) {
+#pragma unroll
+      for (int c = 0; c < J; ++c) wj[c] = row[c];
+      slot = __float_as_int(row[J + XD]);
+    } else {
+      window_jets<S>(xv, box, d.flag, wj);
+    }
     jet_mul<S>(uj, wj, uw);
     if (valid) {
 #pragma unroll
       for (int c = 0; c < J; ++c)
         if ((c & 3) == g) pairbuf[(size_t)slot * J + c] = uw[c];
+    }
+    if constexpr (NH == 2) {
+      if (refill) {
+        Team<true>::sync();   // this sub-tile's rows have been read
+        put_row(xq, slotn);
+      }
     }
   }
 }
@@ -1020,13 +1104,14 @@ fwd_kernel(const float* __restrict__ theta, const float* __restrict__ dom, const
 // Upstream gradient of one pair w.r.t. its network output jets:
 // gur = sd_u * (d uw / d u)^T gU, gU = gseg[seg] (zero for padding lanes).
 template <class S>
-__device__ inline void pair_upstream(const float* gU, const float* xv, const Dom& d, float* gur) {
+__device__ inline void pair_upstream(const float* gU, const float* xv, const WindowBox<S::XD>& box, float flag, float usd,
+                                     float* gur) {
   constexpr int J = S::J;
   float wj[J];
-  window_jets<S>(xv, d, wj);
+  window_jets<S>(xv, box, flag, wj);
   jet_mul_T<S>(gU, wj, gur);
 #pragma unroll
-  for (int c = 0; c < J; ++c) gur[c] *= d.usd;
+  for (int c = 0; c < J; ++c) gur[c] *= usd;
 }
 
 // Chunk epilogue of one hidden layer: the gradient row from the waves' unit
@@ -1129,12 +1214,9 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   if constexpr (ADAM) {
     if (first && T::tid() == 0) adam_bias_n(cnt, af.k, bc);
   }
-  float mu[XD], isd[XD];
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    mu[i] = (d.xmax[i] + d.xmin[i]) / 2.f;
-    isd[i] = 1.f / ((d.xmax[i] - d.xmin[i]) / 2.f);
-  }
+  const ChunkBox<XD> box(d);
+  const float* const mu = box.mu;
+  const float* const isd = box.isd;
   T::sync();
   stage_zt<XD, H, SM, WAVE>(ss, isd, szt);
   T::sync();
@@ -1168,7 +1250,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
       pn = wl.pair_point[k2 < end ? k2 : beg];
       sn = wl.pair_seg[k2 < end ? k2 : beg];
     }
-    pair_upstream<S>(gU, xv, d, gur);
+    pair_upstream<S>(gU, xv, box, d.flag, d.usd, gur);
     if (g == 0) dbl += gur[0];
     float h1[NRB][4];
     layer1_stream<XD, H, SM>(v, xh, h1);
@@ -1390,12 +1472,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   using L = Layout<XD, H, 2>;
   using SM = Small<XD, H, 2>;
   using O = DW2Own<H>;
+  using R = PairRows;
   constexpr int J = S::J, NRB = H / 16, NS = 3 + XD;
   constexpr int K_WL = 0, K_B1 = 1, K_W1 = 2, K_B2 = 2 + XD;
   // H <= 32 and XD <= 2 (wave-private dW2, registers to spare): the small
-  // per-unit gradients (dW1, dWL, db1, db2) are summed per lane over the
+  // per-unit gradients but dWL (dW1, db1, db2) are summed per lane over the
   // chunk's tiles and reduced over the pair lanes once per chunk instead of
-  // once per tile (with three axes the unrolled axis loop would spill)
+  // once per tile (with three axes the unrolled axis loop would spill; with
+  // dWL as well, 13 more spilled registers and 154 us against 148.5)
   constexpr bool ACC = DW2Own<H>::PRIV && XD <= 2;
   constexpr int AXIS_UNROLL = H == 64 || ACC ? XD : 1;
   static_assert(H >= 16 && H <= 64, "hidden width 16, 32 or 64");
@@ -1404,9 +1488,10 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   __shared__ __attribute__((aligned(16))) float swt[2 * H * H];
   float* const swr = swt + H * H;
   __shared__ __attribute__((aligned(16))) float strans[2 * O::TSZ];
-  __shared__ float ssmall[4 * NS * H];
+  // per wave: its pair rows, and at the chunk's end its unit totals
+  constexpr int SW = R::WAVE > NS * H ? R::WAVE : NS * H;
+  __shared__ __attribute__((aligned(16))) float srow[4 * SW];
   __shared__ float sbl[4];
-  __shared__ float red[64];
   float* sta = strans;            // a1 columns
   float* stg = strans + O::TSZ;   // G columns
 
@@ -1420,31 +1505,28 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // everything that waits
   GradientMax<J> gmax;
   gmax.indices(wl, beg, end);
-  const int k0 = beg + wave * 16 + pl;
+  const int k0 = beg + wave * 16 + g * 64 + pl;   // the pair of this lane's first row
   const int p0 = wl.pair_point[k0 < end ? k0 : beg], seg0 = wl.pair_seg[k0 < end ? k0 : beg];
   Dom d;
   load_dom(dom, model, d);
-  float mu[XD], isd[XD];
-#pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    mu[i] = (d.xmax[i] + d.xmin[i]) / 2.f;
-    isd[i] = 1.f / ((d.xmax[i] - d.xmin[i]) / 2.f);
-  }
+  const ChunkBox<XD> box(d);
+  const float* const mu = box.mu;
+  const float* const isd = box.isd;
   const float one = opaque_one();
   Scales<XD> sc;
-  float xn[XD], gUn[J];   // the next tile's point and upstream jets
+  float x0[XD], gU0[J];   // the first row's point and upstream jets
   stage_two<S, H, SM, true, true>(
       th, d, isd,
       [&]() -> const float* {
 #pragma unroll
-        for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
+        for (int i = 0; i < XD; ++i) x0[i] = x[(size_t)p0 * XD + i];
 #pragma unroll
-        for (int c = 0; c < J; ++c) gUn[c] = k0 < end ? gseg[(size_t)seg0 * J + c] : 0.f;
+        for (int c = 0; c < J; ++c) gU0[c] = k0 < end ? gseg[(size_t)seg0 * J + c] : 0.f;
         gmax.values(wl, gseg, beg, end);
         return gmax.m;
       },
-      one, ss, szt, swt, swr, red, sc);
-  d.usd *= sc.k;
+      one, ss, szt, swt, swr, srow, sc);
+  d.usd = uniform(d.usd * sc.k);
 
   // WL of the unit a reduction leaves in this lane (for G_0')
   const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)] * sc.iw;
@@ -1454,8 +1536,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // dW2 reads: this wave's own tiles (PRIV) or its quadrant's blocks
   const float* const star = sta + (O::PRIV ? wave * O::TILE : O::col_block(wave, 0) * O::BS) + O::at_tr(lane);
   const float* const stgr = stg + (O::PRIV ? wave * O::TILE : O::row_block(wave, 0) * O::BS) + O::at_tr(lane);
-  float* mysmall = ssmall + wave * NS * H;
-  float aW1[ACC ? XD : 1][NRB][4], aWL[NRB][4], aB1[NRB][4], aB2[NRB][4];
+  float aW1[ACC ? XD : 1][NRB][4], aB1[NRB][4], aB2[NRB][4];
   if constexpr (ACC) {
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb)
@@ -1463,7 +1544,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
         for (int i = 0; i < XD; ++i) aW1[i][rb][r] = 0.f;
-        aWL[rb][r] = aB1[rb][r] = aB2[rb][r] = 0.f;
+        aB1[rb][r] = aB2[rb][r] = 0.f;
       }
   }
   f4 dW2[O::NOB];
@@ -1479,26 +1560,34 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // below); with wave-private blocks (H <= 32) a wave runs only the tiles in
   // which its 16-pair sub-tile holds a pair of the chunk.  Lanes past the
   // chunk end carry zero upstream gradient and so contribute nothing.
-  const int ntile = O::PRIV ? (end - beg - 16 * wave + 63) >> 6 : (end - beg + 63) >> 6;
-  // each tile's point and upstream jets are fetched during the previous tile
-  // (indices at the start of its column-0 phase, data before its last dW2
-  // column), so the two dependent global loads do not stall the tile start
-  for (int t = 0; t < ntile; ++t) {
-    float xv[XD], xh[XD];
-#pragma unroll
-    for (int i = 0; i < XD; ++i) {
-      xv[i] = xn[i];
-      xh[i] = (xv[i] - mu[i]) * isd[i];
-    }
+  const int ntile =
+      O::PRIV ? __builtin_amdgcn_readfirstlane((end - beg - 16 * wave + 63) >> 6) : (end - beg + 63) >> 6;
+  // this lane's row (upstream gradient, normalised point) of the next four
+  // tiles.  Their points and upstream jets are fetched during the tile
+  // before (indices at the start of its column-0 phase, data before its last
+  // dW2 column), so the two dependent global loads do not stall a tile's start
+  static_assert(J + XD <= R::ROW, "a pair's row");
+  float* const rows = srow + wave * SW;
+  const auto put_row = [&](const float* xp, const float* gU) {
     float gur[J];
-    pair_upstream<S>(gUn, xv, d, gur);
-    // materialise the pair's values here, so that the prefetched data dies
-    // at the tile start instead of being carried into the axis phases
+    pair_upstream<S>(gU, xp, box, d.flag, d.usd, gur);
+    dbl += gur[0];
+    float* const to = rows + lane * R::ROW;
 #pragma unroll
-    for (int c = 0; c < J; ++c) asm volatile("" : "+v"(gur[c]));
+    for (int c = 0; c < J; ++c) to[c] = gur[c];
 #pragma unroll
-    for (int i = 0; i < XD; ++i) asm volatile("" : "+v"(xh[i]));
-    if (g == 0) dbl += gur[0];
+    for (int i = 0; i < XD; ++i) to[J + i] = (xp[i] - mu[i]) * isd[i];
+    Team<true>::sync();
+  };
+  put_row(x0, gU0);
+  for (int t = 0; t < ntile; ++t) {
+    const float* const row = rows + ((t & 3) * 16 + pl) * R::ROW;
+    float gur[J], xh[XD];
+#pragma unroll
+    for (int c = 0; c < J; ++c) gur[c] = row[c];
+#pragma unroll
+    for (int i = 0; i < XD; ++i) xh[i] = row[J + i];
+    const bool refill = (t & 3) == 3 && t + 1 < ntile;
 
     float h1[NRB][4];
     layer1_stream<XD, H, SM>(v, xh, h1);
@@ -1688,10 +1777,17 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         }
     }
     // ---- column 0: db2 += G_0, dW2 += G_0 h^T, W2~^T G_0 -> layer 1
-    const int kn = beg + (t + 1) * 64 + wave * 16 + pl;   // next tile's pair
+    // (h = 64 reads in every tile what the fourth uses: a branch here splits the
+    // tile's schedule, 78 -> 259 registers spilled, 3,360 -> 10,070 us; below it
+    // the branch is the cheaper form)
+    const int kn = beg + ((t | 3) + 1 + g) * 64 + wave * 16 + pl;   // the next row's pair
     const bool valid_n = kn < end;
-    const int pn = wl.pair_point[valid_n ? kn : beg];
-    const int segn = wl.pair_seg[valid_n ? kn : beg];
+    const bool fetch = !O::PRIV || refill;
+    int pn, segn;
+    if (fetch) {
+      pn = wl.pair_point[valid_n ? kn : beg];
+      segn = wl.pair_seg[valid_n ? kn : beg];
+    }
     if constexpr (ACC) {
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
@@ -1719,6 +1815,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) gz10[rb][r] = e1[rb][r] * fmaf(-2.f, gz10[rb][r], GA[rb][r]);
     }
+    small[K_WL] = fmaf(reduce_units<NRB>(vWL, pl), sc.iw, small[K_WL]);
     // dW1[:, i] += gz1_0 xh_i (the gz1_i parts were added per axis)
     if constexpr (ACC) {
       float xr[XD];
@@ -1730,7 +1827,6 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         for (int r = 0; r < 4; ++r) {
 #pragma unroll
           for (int i = 0; i < XD; ++i) aW1[i][rb][r] = fmaf(gz10[rb][r], xr[i], aW1[i][rb][r]);
-          aWL[rb][r] += vWL[rb][r];
           aB1[rb][r] += gz10[rb][r];
         }
     } else {
@@ -1742,33 +1838,35 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
           for (int r = 0; r < 4; ++r) vv[rb][r] = gz10[rb][r] * xh[i];
         small[K_W1 + i] = fmaf(reduce_units<NRB>(vv, pl), sc.ir, small[K_W1 + i]);
       }
-      small[K_WL] = fmaf(reduce_units<NRB>(vWL, pl), sc.iw, small[K_WL]);
       small[K_B1] = fmaf(reduce_units<NRB>(gz10, pl), sc.ir, small[K_B1]);
     }
-    // the next tile's point and upstream jets, in flight during the last dW2 column
+    // the next row's point and upstream jets, in flight during the last dW2 column
     __builtin_amdgcn_sched_barrier(0);
+    float xn[XD], gUn[J];
+    if (fetch) {
 #pragma unroll
-    for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
+      for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
 #pragma unroll
-    for (int c = 0; c < J; ++c) gUn[c] = valid_n ? gseg[(size_t)segn * J + c] : 0.f;
+      for (int c = 0; c < J; ++c) gUn[c] = valid_n ? gseg[(size_t)segn * J + c] : 0.f;
+    }
     tile_sync<O::PRIV>();
     if constexpr (O::PRIV)
       dw2_private<H>(stgr, star, dW2);
     else
       dw2_shared<H>(stgr, star, dW2);
     // (the next tile's first column has a barrier before its stores)
+    if (refill) put_row(xn, gUn);
   }
 
   // ---- end of chunk: the gradient row from the waves' sums
   if constexpr (ACC) {
 #pragma unroll
     for (int i = 0; i < XD; ++i) small[K_W1 + i] = reduce_units<NRB>(aW1[i], pl);
-    small[K_WL] = reduce_units<NRB>(aWL, pl) * sc.iw;
     small[K_B1] = reduce_units<NRB>(aB1, pl) * sc.ir;
     small[K_B2] = reduce_units<NRB>(aB2, pl) * wl_red;
   }
-  store_units<NRB, NS>(mysmall, small, H, pl, g);
-  dbl = sum_row(dbl);
+  store_units<NRB, NS>(rows, small, H, pl, g);   // after this wave's last row
+  dbl = sum_groups(sum_row(dbl));
   if (lane == 0) sbl[wave] = dbl;
   __syncthreads();   // every wave is done with the tiles
   // H = 64: the waves hold disjoint dW2 blocks; H <= 32: every wave holds every
@@ -1797,7 +1895,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   }
   for (int t = threadIdx.x; t < NS * H; t += 256) {
     const int kind = t / H, u = t % H;
-    const float s = (ssmall[t] + ssmall[NS * H + t]) + (ssmall[2 * NS * H + t] + ssmall[3 * NS * H + t]);
+    const float s = (srow[t] + srow[SW + t]) + (srow[2 * SW + t] + srow[3 * SW + t]);
     const int dst = kind == K_WL ? L::WL + u : kind == K_B1 ? L::B1 + u : kind == K_B2 ? L::B2 + u
                                                                        : L::W1 + u * XD + (kind - K_W1);
     out[dst] = s * post;
