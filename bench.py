@@ -29,7 +29,9 @@ sys.path.insert(0, ROOT)
 DEFAULT_STEPS = {"wave": (100, 10), "poisson": (2000, 100), "burgers": (5000, 200), "ho": (20000, 1000),
                  "inverse": (10000, 500)}
 
-PEAK_FP32_MFMA = 157.3   # TFLOP/s, MI355X dense FP32 matrix
+PEAK_FP32 = 157.3        # TFLOP/s, MI355X dense FP32 (one hidden layer: vector)
+PEAK_F16_MFMA = 2516.6   # TFLOP/s, MI355X dense f16 matrix
+PEAK_SPLIT = PEAK_F16_MFMA / 3   # float32 products as three f16 ones (two hidden layers)
 PEAK_HBM = 8000.0         # GB/s
 
 
@@ -215,8 +217,8 @@ def kernel_roofline(eng, cfgmod):
                 f_pair=f_pair, n_pairs=wl.n_pairs, trained_pairs=trained_pairs,
                 executed_mfma={"flop_per_pair_fwd": x_fwd, "flop_per_pair_bwd": x_bwd,
                                "tflops_fwd": tf(ex_fwd, t_fwd), "tflops_bwd": tf(ex_bwd, t_bwd),
-                               "frac_fwd": tf(ex_fwd, t_fwd) / PEAK_FP32_MFMA,
-                               "frac_bwd": tf(ex_bwd, t_bwd) / PEAK_FP32_MFMA})
+                               "frac_fwd": tf(ex_fwd, t_fwd) / PEAK_F16_MFMA,
+                               "frac_bwd": tf(ex_bwd, t_bwd) / PEAK_F16_MFMA})
 
 
 def host_threads():
@@ -422,6 +424,7 @@ def main():
         f"bwd {rl['t_bwd_ms']:.3f} ms ({rl['tflops_bwd']:.1f} TFLOP/s)")
     dom_is_bwd = rl["t_bwd_ms"] >= rl["t_fwd_ms"]
     ach = rl["tflops_bwd"] if dom_is_bwd else rl["tflops_fwd"]
+    peak = PEAK_SPLIT if eng.net.nh == 2 else PEAK_FP32
     dom_kernel = "bwd_kernel" if dom_is_bwd else "fwd_kernel"
     # the recorded counters hold for the configuration's own overlap and the
     # launch shape they were measured with
@@ -489,8 +492,8 @@ def main():
                    "launch": {"forward": f"{autotune.name(eng.launch[0])}, {wgf} workgroups",
                               "backward": f"{autotune.name(eng.launch[1])}, {wgb} workgroups"}},
         "collocation_pts_per_s": sps * n_pts,
-        "roofline": {"bound": "mfma", "achieved": ach, "peak": PEAK_FP32_MFMA, "unit": "TFLOP/s",
-                     "frac": ach / PEAK_FP32_MFMA, "traffic": traffic,
+        "roofline": {"bound": "mfma", "achieved": ach, "peak": peak, "unit": "TFLOP/s",
+                     "frac": ach / peak, "traffic": traffic,
                      "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated, "
                                      "recorded for this launch shape)",
                      "kernel": dom_kernel, "launch": launch_txt,

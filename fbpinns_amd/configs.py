@@ -147,8 +147,8 @@ def fwd_flops_per_pair(xd, h, nh, J):
 
 
 # matrix-core FLOPs the kernels execute per (point, subdomain) pair: the
-# layer-2 contractions run as passes of v_mfma_f32_16x16x4f32 over 16 pairs,
-# (h/16) x (h/4) instructions of 2 * 16 * 16 * 4 FLOPs per pass.  Forward: Z_0,
+# layer-2 contractions run as passes over 16 pairs, each product of 2 * h * h *
+# 16 FLOPs as three f16 products (hi hi, hi lo, lo hi).  Forward: Z_0,
 # the W2^T vector when any first derivative is carried, one Z_i per axis with
 # a second derivative.  Backward: Z_0; with first derivatives the s-vector
 # pass, its W2^T pass and its dW2 column; per second-derivative axis Z_i, its
@@ -157,7 +157,7 @@ def fwd_flops_per_pair(xd, h, nh, J):
 def mfma_flops_per_pair(h, nh, n1, n2):
     if nh != 2:
         return 0, 0
-    per_pass = (h // 16) * (h // 4) * 2 * 16 * 16 * 4 / 16
+    per_pass = 3 * 2 * h * h
     fwd = (1 + (n1 > 0) + n2) * per_pass
     bwd = (3 + 3 * (n1 > 0) + 3 * n2) * per_pass
     return fwd, bwd
