@@ -48,15 +48,16 @@ its sub-tiles; with many, the waves a short chunk leaves idle cost more.
 plan_chunk (the lists that nobody times: inference and FBPINNJets layers, and
 the small lists above): two chunks per CU, of 64 to 384 pairs.  Forward +
 backward us by chunk cap (none = one chunk per subdomain):
-  [2,64,64,1] 180,699 pairs, 56 subdomains: none 221 + 647, 128 40 + 143,
-    384 36 + 111, 512 43 + 136
-  [3,64,64,1] 13,647 pairs, 36 subdomains: none 81 + 245, 64 26 + 47, 128
-    25 + 53, 512 43 + 118
-  [2,32,32,1] 361,229 pairs, 196 subdomains: none 68 + 142, 256 33 + 110, 384
-    31 + 97, 512 37 + 114
-  [3,64,1] 206,094 pairs, 75 subdomains: none 120 + 205, 384 32 + 50
-  [3,64,64,1] values of 685,693 pairs, 864 subdomains: none 61, 256 53, 384
-    51, 512 55
+  [2,64,64,1] 180,699 pairs, 56 subdomains: none 201 + 555, 128 44 + 122,
+    256 37 + 117, 384 36 + 94, 512 42 + 114
+  [3,64,64,1] 13,647 pairs, 36 subdomains: none 71 + 198, 64 16 + 28, 128
+    17 + 34, 512 35 + 91
+  [2,32,32,1] 361,229 pairs, 196 subdomains: none 59 + 113, 256 31 + 92, 384
+    28 + 79, 512 34 + 92
+  [3,64,1] 206,094 pairs, 75 subdomains: none 113 + 189, 256 18 + 33, 384
+    20 + 36, 512 17 + 31
+  [3,64,64,1] values of 685,693 pairs, 864 subdomains: none 54, 256 54, 384
+    49, 512 52
 A few pairs per chunk cost a weight staging each; a whole subdomain per chunk
 leaves most of 256 CUs idle.
 """
