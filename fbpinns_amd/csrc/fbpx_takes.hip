@@ -40,9 +40,16 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kThreads * kScanItems;   // elements per scan workgroup
-constexpr int kTilePoints = 1024;                   // points per tile workgroup
+constexpr int kXcds = 8;                            // dies with an L2 each, workgroups dealt in turn
 constexpr int kSortWaves = 8;                       // waves of a tile workgroup
+constexpr int kSortAhead = 8;                       // 64-pair steps whose pairs are read at once
 constexpr int kSortModels = 1536;                   // models counted at a time (48 KB of LDS counters)
+// Points per tile workgroup: 512, or 1,024 where several windows of models are
+// counted (the counts, one per model and workgroup, are then the larger part).
+// 864 models, 524,288 points, 3.6 M pairs: count and place 9.4 + 102 us with
+// 2,048 or 1,024 points, 8.8 + 61.6 with 512; a build with 6,400 models and
+// 200,000 points 1,320 us with 1,024, 1,340 with 512.
+constexpr int tile_points(int m) { return m <= kSortModels ? 512 : 1024; }
 constexpr int kUsedLds = 32768;                     // models flagged in LDS
 constexpr int64_t kUsedPairs = 4096;                // pairs per "used" workgroup
 constexpr int kMaxPou = 32;
@@ -331,18 +338,21 @@ __global__ void __launch_bounds__(kThreads) seg_fill_kernel(int64_t s, const int
 }
 
 // Stable counting sort of the point-major pairs by model position, one
-// workgroup per block of kTilePoints points, wave w over kTilePoints /
-// kSortWaves consecutive points of it, kSortModels models at a time.
+// workgroup per block of tile_points(m) points, wave w over its share of them
+// in order, kSortModels models at a time.
 // FILL = false: blkcnt[k * nblk + b] = the block's pairs of model position k
 // (0 for k >= n_used).  FILL = true: blkcnt holds the scanned bases; each
 // wave turns its counts into its own bases and places its pairs 64 at a time,
 // a pair's place being its model's base plus its rank among the 64 lanes
 // (equal models found by one ballot per bit of the position), so pairs of a
-// model stay in point-major order.  LDS and memory latency bound: pairs are
-// read twice and written once.  (Testing every point of a block against
-// every box and searching each pair's twin in its point's list took 1.35 +
-// 1.85 ms on 524,288 points, 864 boxes and 3.6 M pairs; this takes 12 + 131
-// us.)
+// model stay in point-major order.  Bound by partial-line writes: a block's run
+// of a model is a few pairs, and its neighbours in memory come from the next
+// blocks.  Workgroups are dealt to the dies in turn, so each die takes a run of
+// consecutive blocks (and blocks are small enough to be in flight together):
+// the lines fill in its L2 before they leave it.  Placing 3.6 M pairs of 864
+// models took 131 us with blocks dealt in order, 102 with this mapping, 61.6
+// with 512 points per block as well.  (Testing every point of a block against
+// every box and searching each pair's twin in its point's list took 1.85 ms.)
 template <bool FILL>
 __global__ void __launch_bounds__(64 * kSortWaves) tile_sort_kernel(
     int n, int nblk, int m, int win, const int64_t* __restrict__ off, const int32_t* __restrict__ info,
@@ -350,18 +360,25 @@ __global__ void __launch_bounds__(64 * kSortWaves) tile_sort_kernel(
     const int32_t* __restrict__ slot_pm, int32_t* __restrict__ blkcnt, int32_t* __restrict__ pair_point,
     int32_t* __restrict__ pair_seg, int32_t* __restrict__ pair_slot) {
   extern __shared__ int32_t sort_cnt[];   // [kSortWaves][win]
-  constexpr int kWavePoints = kTilePoints / kSortWaves;
-  const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int tp = tile_points(m), wave_points = tp / kSortWaves;
+  const int per = gridDim.x / kXcds;   // the grid is kXcds times as many as a die's blocks
+  const int b = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (b >= nblk) return;
   int32_t* cnt = sort_cnt + w * win;
   const int n_used = info[kInfoUsed];
-  const int p0 = min(n, b * kTilePoints + w * kWavePoints), p1 = min(n, p0 + kWavePoints);
+  const int p0 = (int)min((int64_t)n, (int64_t)b * tp + w * wave_points), p1 = min(n, p0 + wave_points);
   const int64_t q0 = off[p0], q1 = off[p1];
   for (int k0 = 0; k0 < (FILL ? n_used : m); k0 += win) {
     for (int k = lane; k < win; k += 64) cnt[k] = 0;
     if (k0 < n_used) {
-      for (int64_t q = q0 + lane; q < q1; q += 64) {
-        const int k = m_take[q] - k0;
-        if (k >= 0 && k < win) atomicAdd(&cnt[k], 1);
+      for (int64_t q = q0 + lane; q < q1; q += 64 * kSortAhead) {
+        int k[kSortAhead];
+#pragma unroll
+        for (int j = 0; j < kSortAhead; ++j) k[j] = m_take[min(q + 64 * j, q1 - 1)] - k0;
+#pragma unroll
+        for (int j = 0; j < kSortAhead; ++j)
+          if (q + 64 * j < q1 && k[j] >= 0 && k[j] < win) atomicAdd(&cnt[k[j]], 1);
       }
     }
     __syncthreads();
@@ -377,29 +394,41 @@ __global__ void __launch_bounds__(64 * kSortWaves) tile_sort_kernel(
     }
     __syncthreads();
     if (FILL) {
-      for (int64_t q = q0; q < q1; q += 64) {   // wave-uniform trip count
-        const bool live = q + lane < q1;
-        const int k = live ? m_take[q + lane] - k0 : -1;
-        const bool in = k >= 0 && k < win;
-        uint64_t same = __ballot(in);
-        if (same == 0) continue;
+      // kSortAhead steps' pairs are read at once
+      for (int64_t qb = q0; qb < q1; qb += 64 * kSortAhead) {   // wave-uniform trip count
+        int ka[kSortAhead], pp[kSortAhead], ps[kSortAhead], pt[kSortAhead];
 #pragma unroll
-        for (int bit = 0; bit < 11; ++bit) {
-          const bool one = (k >> bit) & 1;
-          const uint64_t v = __ballot(one);
-          same &= one ? v : ~v;
+        for (int j = 0; j < kSortAhead; ++j) {
+          const int64_t q = min(qb + 64 * j + lane, q1 - 1);
+          ka[j] = m_take[q];
+          pp[j] = n_take[q];
+          ps[j] = p_take[q];
+          pt[j] = slot_pm[q];
         }
-        if (in) {
-          const int64_t t = cnt[k] + __popcll(same & ((1ull << lane) - 1));
-          // the model's highest lane moves its base past the 64 pairs, after
-          // every lane has read it (a wave's LDS operations are in order)
+#pragma unroll
+        for (int j = 0; j < kSortAhead; ++j) {
+          const int k = qb + 64 * j + lane < q1 ? ka[j] - k0 : -1;
+          const bool in = k >= 0 && k < win;
+          uint64_t same = __ballot(in);
+          if (same == 0) continue;
+#pragma unroll
+          for (int bit = 0; bit < 11; ++bit) {
+            const bool one = (k >> bit) & 1;
+            const uint64_t v = __ballot(one);
+            same &= one ? v : ~v;
+          }
+          if (in) {
+            const int64_t t = cnt[k] + __popcll(same & ((1ull << lane) - 1));
+            // the model's highest lane moves its base past the 64 pairs, after
+            // every lane has read it (a wave's LDS operations are in order)
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if ((same >> lane) == 1) cnt[k] += __popcll(same);
+            pair_point[t] = pp[j];
+            pair_seg[t] = ps[j];
+            pair_slot[t] = pt[j];
+          }
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          if ((same >> lane) == 1) cnt[k] += __popcll(same);
-          pair_point[t] = n_take[q + lane];
-          pair_seg[t] = p_take[q + lane];
-          pair_slot[t] = slot_pm[q + lane];
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       }
       __syncthreads();
     }
@@ -524,7 +553,7 @@ struct Carve {
   }
 };
 
-int64_t nblocks(int n) { return (n + kTilePoints - 1) / kTilePoints; }
+int64_t nblocks(int n, int m) { return ((int64_t)n + tile_points(m) - 1) / tile_points(m); }
 
 struct Work {
   int32_t* counts;
@@ -546,7 +575,7 @@ struct Work {
 Work carve(void* base, int n, int xd, int m, int64_t s, int fbins, int bbins, size_t* bytes) {
   Carve c{static_cast<char*>(base), 0, 0};
   Work w;
-  const int64_t nb = nblocks(n);
+  const int64_t nb = nblocks(n, m);
   const int64_t nmax = std::max<int64_t>(std::max<int64_t>(n, s + 1), (int64_t)m * nb + 1);
   w.counts = c.take<int32_t>(n);
   w.tsum = c.take<int64_t>(scan_tiles(nmax) + 1);
@@ -570,7 +599,8 @@ void launch_tiles(hipStream_t st, bool fill_pass, int n, int nblk, int m, const 
                   const fbpx_takes_out& o) {
   const int win = std::min(m, kSortModels);
   const size_t lds = sizeof(int32_t) * kSortWaves * win;
-  hipLaunchKernelGGL(fill_pass ? tile_sort_kernel<true> : tile_sort_kernel<false>, dim3((unsigned)nblk),
+  const unsigned grid = (unsigned)((nblk + kXcds - 1) / kXcds * kXcds);
+  hipLaunchKernelGGL(fill_pass ? tile_sort_kernel<true> : tile_sort_kernel<false>, dim3(grid),
                      dim3(64 * kSortWaves), lds, st, n, nblk, m, win, off, w.info, o.m_take, o.n_take, o.p_take,
                      w.slot_pm, w.blkcnt, o.pair_point, o.pair_seg, o.pair_slot);
 }
@@ -665,7 +695,7 @@ int fbpx_build_worklist(void* stream, const float* x, int32_t n, int32_t xd, con
   }
   hipStream_t st = (hipStream_t)stream;
   Work w = carve(work, n, xd, m, s, fbins, bbins, &need);
-  const int64_t nblk = nblocks(n);
+  const int64_t nblk = nblocks(n, m);
 
   // point-major pairs and the models they use
   fill<uint8_t>(st, w.used, m, 0);
