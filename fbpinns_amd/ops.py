@@ -38,7 +38,10 @@ def _p(t, dtype=None, name="tensor"):
         raise FbpxError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise FbpxError(f"{name} must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    ptr = t.data_ptr()
+    if not ptr and t.numel():
+        raise FbpxError(f"{name} has no memory")   # a zero tensor of autograd's
+    return ctypes.c_void_p(ptr)
 
 
 class NetSpec:
@@ -146,8 +149,12 @@ def _wl_struct(ts: List[torch.Tensor], ns: List[int]):
 # ------------------------------------------------------------------ custom ops
 
 def _is_plain(v):
-    """A tensor whose data pointer the body may use as it is."""
-    return type(v) is torch.Tensor and not (v.requires_grad and torch.is_grad_enabled()) and not v.is_inference()
+    """A tensor whose data pointer the body may use as it is (an upstream
+    gradient may come as a negative view: _neg_view, the imaginary part of a
+    conjugate).  int32 tensors have neither negative views nor gradients."""
+    if type(v) is not torch.Tensor or v.is_inference():
+        return False
+    return v.dtype is torch.int32 or not (v.is_neg() or (v.requires_grad and torch.is_grad_enabled()))
 
 
 def _op(name, mutates_args):
