@@ -163,9 +163,11 @@ def _op(name, mutates_args):
     counts the mutated tensors' versions as the dispatcher would; the
     dispatcher's own share of a call was about 35 us of host time, three to
     four times the body's.  Whatever interposes on operators sees the custom
-    op as before: compilation, tracing, dispatch and function modes, functorch
-    transforms, forward-mode levels, inference mode, tensor subclasses and
-    arguments that require a gradient."""
+    op as before: compilation, tracing, profiling, dispatch and function modes,
+    functorch transforms, forward-mode levels, inference mode, tensor
+    subclasses and arguments that require a gradient.  (An
+    ExecutionTraceObserver outside a profiler cannot be asked for and does not
+    see direct calls.)"""
     def deco(fn):
         op = torch.library.custom_op(name, fn, mutates_args=mutates_args)
         params = list(inspect.signature(fn).parameters.values())
@@ -179,7 +181,8 @@ def _op(name, mutates_args):
             if kwargs or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() \
                     or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None \
                     or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0 \
-                    or torch.is_inference_mode_enabled() or len(args) > len(params):
+                    or torch.is_inference_mode_enabled() or torch._C._autograd._profiler_enabled() \
+                    or len(args) > len(params):
                 return op(*args, **kwargs)
             for i, k in tensors:
                 if i >= len(args):

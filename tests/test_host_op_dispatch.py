@@ -117,6 +117,16 @@ class _Seen(TorchDispatchMode):
         return func(*args, **(kwargs or {}))
 
 
+def test_profiler_sees_the_operator():
+    args = _args()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as p:
+        axpy(*args)
+    assert any(e.key == "fbpx_test::axpy" for e in p.key_averages())
+    with torch.autograd.profiler.profile() as p:
+        axpy(*args)
+    assert any(e.key == "fbpx_test::axpy" for e in p.key_averages())
+
+
 def test_modes_functions_and_subclasses_see_the_operator():
     with _Seen() as seen:
         axpy(*_args())
