@@ -157,6 +157,13 @@ def _is_plain(v):
     return v.dtype is torch.int32 or not (v.is_neg() or (v.requires_grad and torch.is_grad_enabled()))
 
 
+# an argument's kind by its annotation; scalars: their own type
+_TENSOR, _OPTIONAL, _TENSORS, _INTS = "tensor", "optional", "tensors", "ints"
+_KINDS = {torch.Tensor: _TENSOR, Optional[torch.Tensor]: _OPTIONAL, List[torch.Tensor]: _TENSORS, List[int]: _INTS,
+          int: int, float: float, bool: bool}
+_INT_ONLY = frozenset((int,))
+
+
 def _op(name, mutates_args):
     """Registers the function as the torch custom op `name` and returns a
     callable for it that, in plain eager mode, runs the function directly and
@@ -165,15 +172,15 @@ def _op(name, mutates_args):
     four times the body's.  Whatever interposes on operators sees the custom
     op as before: compilation, tracing, profiling, dispatch and function modes,
     functorch transforms, forward-mode levels, inference mode, tensor
-    subclasses and arguments that require a gradient.  (An
+    subclasses, arguments that require a gradient and arguments that the
+    schema converts or refuses.  (An
     ExecutionTraceObserver outside a profiler cannot be asked for and does not
     see direct calls.)"""
     def deco(fn):
         op = torch.library.custom_op(name, fn, mutates_args=mutates_args)
         params = list(inspect.signature(fn).parameters.values())
-        kinds = [{torch.Tensor: 1, Optional[torch.Tensor]: 2, List[torch.Tensor]: 3}.get(p.annotation, 0)
-                 for p in params]
-        tensors = [(i, k) for i, k in enumerate(kinds) if k]
+        required = sum(p.default is inspect.Parameter.empty for p in params)
+        kinds = [_KINDS[p.annotation] for p in params]
         mutated = [i for i, p in enumerate(params) if p.name in mutates_args]
 
         @functools.wraps(fn)
@@ -182,16 +189,19 @@ def _op(name, mutates_args):
                     or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None \
                     or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0 \
                     or torch.is_inference_mode_enabled() or torch._C._autograd._profiler_enabled() \
-                    or len(args) > len(params):
+                    or not required <= len(args) <= len(params):
                 return op(*args, **kwargs)
-            for i, k in tensors:
-                if i >= len(args):
-                    break
-                v = args[i]
-                if k == 3:
+            for k, v in zip(kinds, args):
+                if k is _TENSOR or k is _OPTIONAL:
+                    if not _is_plain(v) and not (k is _OPTIONAL and v is None):
+                        return op(*args)
+                elif k is _TENSORS:
                     if type(v) is not list or not all(_is_plain(t) for t in v):
                         return op(*args)
-                elif not _is_plain(v) and not (k == 2 and v is None):
+                elif k is _INTS:
+                    if type(v) is not list or not _INT_ONLY.issuperset(map(type, v)):
+                        return op(*args)
+                elif type(v) is not k:
                     return op(*args)
             fn(*args)
             for i in mutated:

@@ -199,6 +199,32 @@ def test_inference_tensors_outside_inference_mode():
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("at,value", [(2, [1, 2.5]), (2, (1, 2)), (2, ["a"]), (3, 1.5), (3, "a"), (3, True), (4, 2),
+                                      (4, "a"), (4, np.float64(2.0)), (5, 1), (0, None), (1, [None]), (7, 1.0)])
+def test_schema(at, value):
+    """Arguments of another type are converted or refused as the custom op does."""
+    results = []
+    for call in (axpy, axpy.custom_op):
+        args = _args()
+        args[at] = value
+        try:
+            call(*args)
+            results.append((None, args[6].tolist()))
+        except Exception as e:
+            results.append((type(e), args[6].tolist()))
+    assert results[0] == results[1], results
+
+
+@pytest.mark.parametrize("n", [0, 3, 6])
+def test_missing_arguments(n):
+    kinds = []
+    for call in (axpy, axpy.custom_op):
+        with pytest.raises(Exception) as e:
+            call(*_args()[:n])
+        kinds.append(e.type)
+    assert kinds[0] is kinds[1]
+
+
 def test_versions():
     args = _args()
     axpy(*args)
