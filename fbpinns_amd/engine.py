@@ -436,12 +436,22 @@ class FusedEngine:
                         self.m), takes
 
     def model_jets(self, x, active=None, schema=(0, 0)):
-        """Jets of u~ (before constraining_fn) at points x; returns (J, n)."""
+        """Jets of u~ (before constraining_fn) at points x; returns (J, n).
+
+        The plan of the last call is kept and used again while x is the same
+        memory, unchanged since by the tensor's version (a buffer refilled in
+        place with new points gets a new plan; after a write that PyTorch does
+        not count, through x.data or a raw pointer, pass x.clone()).  Tensors
+        without a version (inference mode) always get a new plan."""
         x = x.to(self.device, torch.float32).contiguous()
-        key = (x.data_ptr(), x.shape[0], None if active is None else tuple(np.asarray(active).tolist()), schema)
-        if key not in self._test_cache:
-            self._test_cache = {key: (x, self.make_plan(x, active, schema)[0])}
-        x, plan = self._test_cache[key]
+        if x.is_inference():
+            plan = self.make_plan(x, active, schema)[0]
+        else:
+            key = (x.data_ptr(), tuple(x.shape), x._version,
+                   None if active is None else tuple(np.asarray(active).tolist()), schema)
+            if key not in self._test_cache:
+                self._test_cache = {key: (x, self.make_plan(x, active, schema)[0])}
+            x, plan = self._test_cache[key]
         with torch.no_grad():
             return FBPINNJets.apply(self.theta, plan)
 
