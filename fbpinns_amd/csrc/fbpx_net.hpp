@@ -773,7 +773,9 @@ __device__ inline void stage_two(const float* th, const Dom& d, const float* isd
       b = fmaxf(b, 0.77f * us * gb * m[RZ + i] * m[RT + i]);
     }
     b = fmaxf(fmaxf(b, bS), fmaf(us, g0, fmaf(0.77f * m[RS], bS, q)));
-    sc.k = uniform(pow2_scale(b, 15, 100));
+    // (with the unnormalising factor in the bound, us 2^k stays below 2^100, so
+    // that gradients of zero stay zero: 0 times an infinite factor is NaN)
+    sc.k = uniform(pow2_scale(fmaxf(b, us * 0x1p-85f), 15, 100));
     sc.ik = pow2_inv(sc.k);
   }
   for (int t = threadIdx.x; t < XD * H; t += blockDim.x) {

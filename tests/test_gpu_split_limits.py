@@ -1,0 +1,49 @@
+"""The split-f16 hidden-layer products at the ends of float32's range, where the
+powers of two that scale their operands meet it, against the float64 oracle.
+Tolerances: those of tests/test_gpu_jets.py (1e-5 per column, 1e-4 per layer
+tensor of the gradient)."""
+
+import numpy as np
+import pytest
+import torch
+
+from fbpinns_amd.engine import FusedEngine
+from fbpinns_amd.networks import FCN
+from fbpinns_amd.ops import FBPINNJets
+from fbpinns_amd.problems import Problem
+
+import setups
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(ls, nsub, unnorm=(0.1, 1.3), n=333):
+    lo, hi = (-1.0,) * ls[0], (1.0,) * ls[0]
+    dec_cls, ap = setups.build(nsub, lo, hi, 1.9, ls, seed=1, unnorm=unnorm)
+    return dec_cls, ap, setups.uniform_points(n, lo, hi, seed=5)
+
+
+def _engine(dec_cls, ap):
+    return FusedEngine(Problem, dec_cls, FCN, ap, device="cuda:0", graph=False)
+
+
+@pytest.mark.parametrize("sd", [1e6, 1e9, 1e20])
+@pytest.mark.parametrize("ls,nsub,d", [([1, 16, 16, 1], (5,), (1, 1)), ([2, 32, 32, 1], (3, 2), (3, 1)),
+                                       ([3, 64, 64, 1], (2, 2, 2), (7, 7)), ([2, 64, 64, 1], (2, 2), (0, 0))])
+def test_zero_gradients_of_a_large_output_scale(ls, nsub, d, sd):
+    """Outputs unnormalised by sd, upstream gradients zero on one half of the
+    domain: its subdomains' gradients are exactly zero, the others' finite."""
+    print(f"[limits] {ls} {d} sd={sd}", flush=True)
+    dec_cls, ap, x = _setup(ls, nsub, unnorm=(0.1, sd))
+    eng = _engine(dec_cls, ap)
+    plan, _ = eng.make_plan(x.cuda(), schema=d)
+    th = eng.theta.detach().requires_grad_(True)
+    u = FBPINNJets.apply(th, plan)
+    r = torch.randn(u.shape, generator=torch.Generator().manual_seed(0)).cuda()
+    g, = torch.autograd.grad(u, th, torch.zeros_like(r))
+    assert (g == 0).all()
+    r[:, x[:, 0].cuda() < 0] = 0
+    g, = torch.autograd.grad(FBPINNJets.apply(th, plan), th, r / sd)
+    assert torch.isfinite(g).all()
+    right = ap["static"]["decomposition"]["subdomain"]["params"][1][:, 0].cuda() > 0   # reaches x > 0
+    assert (g[~right] == 0).all() and (g[right].abs().amax(1) > 0).all()
