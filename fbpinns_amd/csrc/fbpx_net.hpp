@@ -153,11 +153,12 @@ struct Split {
 __device__ inline f4 mfma_k32(h8v a, h8v b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
 // 2^e with m 2^e <= 2^top (within a factor of two below it), e within
-// [-100, lim]: the clamp keeps the inverse and products of factors finite and
-// is what m = 0 and m = inf take.
+// [-126, lim]: every finite m is reached (top >= 2), and so are finite values
+// under a bound m that overflowed to infinity; the clamps keep the factor and
+// its inverse finite.
 __device__ inline float pow2_scale(float m, int top, int lim) {
   int e = top + 126 - (int)((__builtin_bit_cast(uint32_t, m) >> 23) & 255u);
-  e = e < -100 ? -100 : (e > lim ? lim : e);
+  e = e < -126 ? -126 : (e > lim ? lim : e);
   return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
 }
 __device__ inline float pow2_inv(float s) {   // 1 / s for s = 2^e, |e| < 127
@@ -1902,21 +1903,20 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   }
   __syncthreads();
   float* const out = partial + (size_t)chunk * L::P;
-  const float post = gs * sc.ik;
   for (int i = threadIdx.x; i < H * H; i += 256) {
     float s = strans[i];
 #pragma unroll
     for (int w = 1; w < NC; ++w) s += strans[w * H * H + i];
-    out[L::W2 + i] = s * post;
+    out[L::W2 + i] = s * sc.ik * gs;   // in this order: sc.ik gs alone may overflow
   }
   for (int t = threadIdx.x; t < NS * H; t += 256) {
     const int kind = t / H, u = t % H;
     const float s = (srow[t] + srow[SW + t]) + (srow[2 * SW + t] + srow[3 * SW + t]);
     const int dst = kind == K_WL ? L::WL + u : kind == K_B1 ? L::B1 + u : kind == K_B2 ? L::B2 + u
                                                                        : L::W1 + u * XD + (kind - K_W1);
-    out[dst] = s * post;
+    out[dst] = s * sc.ik * gs;
   }
-  if (threadIdx.x == 0) out[L::BL] = ((sbl[0] + sbl[1]) + (sbl[2] + sbl[3])) * post;
+  if (threadIdx.x == 0) out[L::BL] = ((sbl[0] + sbl[1]) + (sbl[2] + sbl[3])) * sc.ik * gs;
 }
 
 // g_scale: NULL, or d L / d loss when gseg holds the segment gradients at

@@ -13,6 +13,7 @@ from fbpinns_amd.ops import FBPINNJets
 from fbpinns_amd.problems import Problem
 
 import setups
+from oracle import model as om
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,49 @@ def test_zero_gradients_of_a_large_output_scale(ls, nsub, d, sd):
     assert torch.isfinite(g).all()
     right = ap["static"]["decomposition"]["subdomain"]["params"][1][:, 0].cuda() > 0   # reaches x > 0
     assert (g[~right] == 0).all() and (g[right].abs().amax(1) > 0).all()
+
+
+def _compare(eng, ap, x, xd, d, gscale):
+    """Columns of the jets and every layer's gradient against the oracle."""
+    plan, _ = eng.make_plan(x.cuda(), schema=d)
+    th = eng.theta.detach().requires_grad_(True)
+    u = FBPINNJets.apply(th, plan)
+    r = torch.randn(u.shape, generator=torch.Generator().manual_seed(0)) * gscale
+    g, = torch.autograd.grad(u, th, r.cuda())
+    ref, _, _ = setups.oracle_jets(ap, x, xd, *d)
+    assert (setups.col_rel_err(u, ref) <= 1e-5).all()
+    takes, all_ims, layers, dom, _ = setups.oracle_view(ap, x)
+    layers = [(W.requires_grad_(True), b.requires_grad_(True)) for W, b in layers]
+    ujs = om.fbpinn_forward(layers, dom, x.double(), takes, om.identity_constraint,
+                            om.get_jmaps(setups.schema_request(xd, *d)))
+    og = torch.autograd.grad((torch.cat(ujs, 1).T * r.double()).sum(), [t for W, b in layers for t in (W, b)])
+    got, off = g.detach().cpu().double()[all_ims], 0
+    assert torch.isfinite(got).all()
+    for t in og:
+        a, b = got[:, off:off + t[0].numel()], t.reshape(len(all_ims), -1)
+        off += t[0].numel()
+        e = ((a - b).abs().max() / b.abs().max().clamp_min(1e-300)).item()
+        print(f"  {tuple(t.shape)} rel err {e:.2e}", flush=True)
+        assert e <= 1e-4
+
+
+@pytest.mark.parametrize("ls,nsub", [([1, 16, 16, 1], (5,)), ([2, 32, 32, 1], (3, 2)), ([3, 64, 64, 1], (2, 2, 2))])
+def test_largest_weights(ls, nsub):
+    """Hidden weights up to 2^120, which saturate every unit: values and
+    gradients of the value."""
+    print(f"[limits] {ls} weights", flush=True)
+    dec_cls, ap, x = _setup(ls, nsub)
+    layers = ap["trainable"]["network"]["subdomain"]["layers"]
+    W = layers[1][0]
+    layers[1] = (W * (2.0 ** 120 / W.abs().max()), layers[1][1])
+    _compare(_engine(dec_cls, ap), ap, x, ls[0], (0, 0), 1.0)
+
+
+@pytest.mark.parametrize("ls,nsub,d", [([1, 16, 16, 1], (5,), (1, 1)), ([2, 32, 32, 1], (3, 2), (3, 1)),
+                                       ([3, 64, 64, 1], (2, 2, 2), (7, 7)), ([3, 64, 64, 1], (2, 2, 2), (0, 0))])
+def test_largest_gradients(ls, nsub, d):
+    """Upstream gradients of 1e33: the bound the scale is chosen from comes near
+    or passes float32's largest value, the gradients do not."""
+    print(f"[limits] {ls} {d} gradients", flush=True)
+    dec_cls, ap, x = _setup(ls, nsub)
+    _compare(_engine(dec_cls, ap), ap, x, ls[0], d, 1e33)
