@@ -1477,7 +1477,7 @@ struct GradientMax {
 
 // [xd, h, h, 1]: hidden-to-hidden layer on MFMA, streamed one axis at a time.
 // Scales (all powers of two, Scales): everything linear in the upstream
-// gradient is carried times 2^k; on top of it (marked ' below)
+// gradient is carried times 2^k and the tile's sign; on top of it (marked ' below)
 //   Z_i' = Z_i 2^(w + e[i]),  S' = S 2^w, and with them G_0', dWL', Q' times 2^w;
 //   vt' = vt 2^r and gz1_0' times 2^r (over -2 e1 until column 0);  stored G_i times 2^-e[i], so that
 //   G_i (e1 zt_i 2^e[i])^T adds to dW2 like the other columns, and so
@@ -1544,6 +1544,18 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       },
       one, ss, szt, swt, swr, srow, sc);
   d.usd = uniform(d.usd * sc.k);
+  // The f16 matrix instructions align their products by cutting them off
+  // towards minus infinity: a product of split operands comes out about 5e-9 of
+  // its typical size too small, always on the same side (the float32
+  // instruction: none).  Added over a subdomain's pairs, whose upstream
+  // gradients differ in sign, that offset grows with their number N and the
+  // gradient with its root: 2.4e-7 of it at N = 3,600.  Everything linear in the
+  // upstream gradient is therefore carried with the other sign in every second
+  // tile (and every second chunk starts with it), and the signs are taken off
+  // where the tiles are added up.  Of the tile's cost only the dW2 accumulators'
+  // change of sign is new: wave backward and Burgers slab step as before, Poisson
+  // step 247.7 -> 250.7 us.
+  const float lane_sign = ((g + chunk) & 1) ? -1.f : 1.f;   // of this lane's rows: tiles g, g + 4, ...
 
   // WL of the unit a reduction leaves in this lane (for G_0')
   const float wl_red = ss[SM::WL + 16 * (pl >> 2) + 4 * g + (pl & 3)] * sc.iw;
@@ -1587,7 +1599,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   float* const rows = srow + wave * SW;
   const auto put_row = [&](const float* xp, const float* gU) {
     float gur[J];
-    pair_upstream<S>(gU, xp, box, d.flag, d.usd, gur);
+    pair_upstream<S>(gU, xp, box, d.flag, d.usd * lane_sign, gur);
     dbl += gur[0];
     float* const to = rows + lane * R::ROW;
 #pragma unroll
@@ -1598,6 +1610,9 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   };
   put_row(x0, gU0);
   for (int t = 0; t < ntile; ++t) {
+    const float sign = ((t + chunk) & 1) ? -1.f : 1.f;
+#pragma unroll
+    for (int j = 0; j < O::NOB; ++j) dW2[j] = -dW2[j];
     const float* const row = rows + ((t & 3) * 16 + pl) * R::ROW;
     float gur[J], xh[XD];
 #pragma unroll
@@ -1713,7 +1728,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
       const float gur_b = two ? pick<J>(gur, S::col2(i)) : 0.f;
       const float e_i = pick<XD>(sc.e, i), ie_i = pick<XD>(sc.ie, i);
       // gz1_i' = gz1_i 2^(r - e[i]) (r alone without a second derivative)
-      const float post = pick<XD>(isd, i) * sc.ir * (two ? e_i : 1.f);
+      const float post = pick<XD>(isd, i) * (sc.ir * sign) * (two ? e_i : 1.f);
       const int zrow = i * H;
       float gzi[NRB][4];
       if (two) {
@@ -1809,9 +1824,9 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
       for (int ob = 0; ob < NRB; ++ob)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) aB2[ob][r] += G0[ob][r];
+        for (int r = 0; r < 4; ++r) aB2[ob][r] = fmaf(G0[ob][r], sign, aB2[ob][r]);
     } else {
-      small[K_B2] = fmaf(reduce_units<NRB>(G0, pl), wl_red, small[K_B2]);
+      small[K_B2] = fmaf(reduce_units<NRB>(G0, pl), wl_red * sign, small[K_B2]);
     }
     {
       Split<H> gsp, hsp;
@@ -1832,19 +1847,19 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
 #pragma unroll
         for (int r = 0; r < 4; ++r) gz10[rb][r] = e1[rb][r] * fmaf(-2.f, gz10[rb][r], GA[rb][r]);
     }
-    small[K_WL] = fmaf(reduce_units<NRB>(vWL, pl), sc.iw, small[K_WL]);
+    small[K_WL] = fmaf(reduce_units<NRB>(vWL, pl), sc.iw * sign, small[K_WL]);
     // dW1[:, i] += gz1_0 xh_i (the gz1_i parts were added per axis)
     if constexpr (ACC) {
       float xr[XD];
 #pragma unroll
-      for (int i = 0; i < XD; ++i) xr[i] = xh[i] * sc.ir;
+      for (int i = 0; i < XD; ++i) xr[i] = xh[i] * (sc.ir * sign);
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
 #pragma unroll
           for (int i = 0; i < XD; ++i) aW1[i][rb][r] = fmaf(gz10[rb][r], xr[i], aW1[i][rb][r]);
-          aB1[rb][r] += gz10[rb][r];
+          aB1[rb][r] = fmaf(gz10[rb][r], sign, aB1[rb][r]);
         }
     } else {
 #pragma unroll
@@ -1853,9 +1868,9 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
         for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) vv[rb][r] = gz10[rb][r] * xh[i];
-        small[K_W1 + i] = fmaf(reduce_units<NRB>(vv, pl), sc.ir, small[K_W1 + i]);
+        small[K_W1 + i] = fmaf(reduce_units<NRB>(vv, pl), sc.ir * sign, small[K_W1 + i]);
       }
-      small[K_B1] = fmaf(reduce_units<NRB>(gz10, pl), sc.ir, small[K_B1]);
+      small[K_B1] = fmaf(reduce_units<NRB>(gz10, pl), sc.ir * sign, small[K_B1]);
     }
     // the next row's point and upstream jets, in flight during the last dW2 column
     __builtin_amdgcn_sched_barrier(0);
@@ -1883,7 +1898,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     small[K_B2] = reduce_units<NRB>(aB2, pl) * wl_red;
   }
   store_units<NRB, NS>(rows, small, H, pl, g);   // after this wave's last row
-  dbl = sum_groups(sum_row(dbl));
+  dbl = sum_groups(sum_row(dbl * lane_sign));
   if (lane == 0) sbl[wave] = dbl;
   __syncthreads();   // every wave is done with the tiles
   // H = 64: the waves hold disjoint dW2 blocks; H <= 32: every wave holds every
@@ -1892,13 +1907,14 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   static_assert(NC * H * H <= 2 * O::TSZ, "the dW2 copies reuse the tile buffers");
   {
     float* const sw = strans + (O::PRIV ? wave * H * H : 0);
+    const float last_sign = ((ntile - 1 + chunk) & 1) ? -1.f : 1.f;
 #pragma unroll
     for (int j = 0; j < O::NOB; ++j) {
       const int ob = O::row_block(wave, j);
       const int col = 16 * O::col_block(wave, j) + pl;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sw[(16 * ob + 4 * g + r) * H + col] = dW2[j][r] * v.vec[SM::WL + 16 * ob + r];
+        sw[(16 * ob + 4 * g + r) * H + col] = dW2[j][r] * (v.vec[SM::WL + 16 * ob + r] * last_sign);
     }
   }
   __syncthreads();
