@@ -94,3 +94,29 @@ def test_largest_gradients(ls, nsub, d):
     print(f"[limits] {ls} {d} gradients", flush=True)
     dec_cls, ap, x = _setup(ls, nsub)
     _compare(_engine(dec_cls, ap), ap, x, ls[0], d, 1e33)
+
+
+@pytest.mark.parametrize("h", [16, 32, 64])
+def test_bits_of_a_weight(h):
+    """The first layer's bias gradient where it is one weight per unit: at x = 0
+    with zero biases every tanh is 0 and its derivative 1, and with output
+    weights of 1 and one hidden weight per column the gradient of u for unit u
+    is that weight.  Three f16 pieces (h = 16) hold a float32 whole, two hold it
+    to 2^-23 of itself."""
+    dec_cls, ap = setups.build((1,), (-1.0,), (1.0,), 1.0, [1, h, h, 1], seed=4)
+    gen = torch.Generator().manual_seed(h)
+    w = torch.rand(h, generator=gen) + 0.5
+    W = torch.zeros(1, h, h)
+    W[0, torch.randperm(h, generator=gen), torch.arange(h)] = w
+    layers = ap["trainable"]["network"]["subdomain"]["layers"]
+    zero = [torch.zeros_like(b) for _, b in layers]
+    layers[0], layers[1] = (layers[0][0], zero[0]), (W, zero[1])
+    layers[2] = (torch.ones_like(layers[2][0]), zero[2])
+    eng = _engine(dec_cls, ap)
+    plan, _ = eng.make_plan(torch.zeros(1, 1).cuda(), schema=(0, 0))
+    th = eng.theta.detach().requires_grad_(True)
+    g, = torch.autograd.grad(FBPINNJets.apply(th, plan), th, torch.ones(1, 1).cuda())
+    got = g[0, h:2 * h].cpu()
+    err = ((got.double() - w.double()) / w.double()).abs().max().item()
+    print(f"[limits] h={h} weight error {err:.2e}", flush=True)
+    assert err <= (0.0 if h == 16 else 2.0 ** -23)
