@@ -59,7 +59,13 @@ backward us by chunk cap (none = one chunk per subdomain):
   [3,64,64,1] values of 685,693 pairs, 864 subdomains: none 54, 256 54, 384
     49, 512 52
 A few pairs per chunk cost a weight staging each; a whole subdomain per chunk
-leaves most of 256 CUs idle.
+leaves most of 256 CUs idle.  Larger lists, forward + backward us by cap (bins:
+one per resident workgroup):
+  [3,64,64,1] 6,861,409 pairs, 864 subdomains: none 1,381 + 4,987, 384 1,194 +
+    3,377, 1,536 1,117 + 3,369, bins 1,112 + 3,446; values: none 456, 384 415,
+    1,536 364, bins 384
+  [2,32,32,1] 3,610,262 pairs, 256 subdomains: none 393 + 782, 384 232 + 629,
+    1,536 218 + 551, bins 216 + 524
 """
 
 import math

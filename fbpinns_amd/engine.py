@@ -323,6 +323,7 @@ class FusedEngine:
         self.plan = ops.Plan(self.net, self.dom, x, plan.wl, wsum, plan.chunk_train, plan.rows,
                              plan.row_chunk_start, self.m)
         self.plan.keep_gradient_buffer(self.net.P)
+        self.plan.partial   # allocated here: the first step runs on the capture's stream
         # the step's Adam inside the backward's launch (fbpx_backward_adam):
         # one hidden layer, no trainable problem leaves, and every trained
         # row exactly one chunk (so each chunk's row is its whole gradient)

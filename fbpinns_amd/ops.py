@@ -874,7 +874,7 @@ class Plan:
         self.net, self.dom, self.x, self.wl, self.wsum = net, dom, x, wl, wsum
         self.chunk_train, self.rows, self.row_chunk_start, self.m = chunk_train, rows, row_chunk_start, m
         self.pairbuf = torch.empty((max(wl.n_pairs, 1), net.J), dtype=torch.float32, device=x.device)
-        self.partial = torch.empty((max(wl.n_chunks, 1), net.P), dtype=torch.float32, device=x.device)
+        self._partial = None
         self.gseg = torch.empty((max(wl.n_segs, 1), net.J), dtype=torch.float32, device=x.device)
         # set by the engine for its step plan: the backward returns this one
         # [m][P] buffer every time (untrained rows stay 0, so no zero fill per
@@ -889,6 +889,17 @@ class Plan:
         # (backward_adam); adam_folded records that it did, this step
         self.adam_fold = None
         self.adam_folded = False
+
+    @property
+    def partial(self):
+        """[n_chunks][P] gradient rows, allocated at the first backward: with a
+        subdomain cut into many chunks they are the plan's largest array, and a
+        plan for values never needs them (6.9 million pairs of 864 [3,64,64,1]
+        subdomains: 18,256 rows, 327 MB; 15 MB at one row per subdomain)."""
+        if self._partial is None:
+            self._partial = torch.empty((max(self.wl.n_chunks, 1), self.net.P), dtype=torch.float32,
+                                        device=self.x.device)
+        return self._partial
 
     def keep_gradient_buffer(self, P):
         self.g_theta = torch.zeros((self.m, P), dtype=torch.float32, device=self.x.device)
