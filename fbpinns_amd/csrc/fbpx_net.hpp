@@ -59,6 +59,10 @@ struct Small {
   static constexpr int N = BL + 1;
 };
 
+// Pair indices are unsigned: loads run up to 1,024 pairs ahead of the chunk's
+// end before they are compared with it, which passes int32 for lists near its
+// end.
+
 // The threads that run one chunk: the workgroup, or with WAVE one wave (a
 // workgroup's four waves then run four chunks of their own).  A wave's LDS
 // operations are performed in order, so a wavefront-scope fence orders its
@@ -851,8 +855,7 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   float* const szt = szt_[T::index()];
 
   const int model = wl.chunk_model[chunk];
-  const int beg = wl.chunk_start[chunk];
-  const int end = wl.chunk_start[chunk + 1];
+  const uint32_t beg = wl.chunk_start[chunk], end = wl.chunk_start[chunk + 1];
   const float* th = theta + (size_t)model * L::P;
   const int lane = threadIdx.x & 63, wave = T::wave(), nw = T::nw();
   const int pl = lane & 15, g = lane >> 4;
@@ -864,7 +867,7 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
   // the staging's LDS writes and barriers (with two, the registers they would
   // hold spill others)
   float xn[XD];
-  const int k0 = beg + wave * 16 + pl;
+  const uint32_t k0 = beg + wave * 16 + pl;
   if constexpr (NH == 1) {
     const int p0 = wl.pair_point[k0 < end ? k0 : beg];
     SmallStage<XD, H, NH, WAVE> st;
@@ -906,21 +909,21 @@ __device__ inline void fwd_chunk(const float* __restrict__ theta, const float* _
     Team<true>::sync();
   };
   if constexpr (NH == 2) {
-    const int kq = beg + wave * 16 + g * 64 + pl;
+    const uint32_t kq = beg + wave * 16 + g * 64 + pl;
     const int pq = wl.pair_point[kq < end ? kq : beg], sq = wl.pair_slot[kq < end ? kq : beg];
 #pragma unroll
     for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pq * XD + i];
     put_row(xn, sq);
   }
   int t = 0;   // sub-tile of this wave
-  for (int base = beg + wave * 16; base < end; base += nw * 16, ++t) {
-    const int k = base + pl;
+  for (uint32_t base = beg + wave * 16; base < end; base += nw * 16, ++t) {
+    const uint32_t k = base + pl;
     const bool valid = k < end;
-    const int kn = k + nw * 16;
+    const uint32_t kn = k + nw * 16;
     float xv[XD], xh[XD];
     int pn, slot;
     const float* const row = rows + (NH == 2 ? ((t & 3) * 16 + pl) * R::ROW : 0);
-    const int kq = kn + g * 64;
+    const uint32_t kq = kn + g * 64;
     const bool refill = NH == 2 && (t & 3) == 3;
     int slotn;
     float xq[XD];
@@ -1213,8 +1216,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   float* const sbl = sbl_ + T::index();
 
   const int model = wl.chunk_model[chunk];
-  const int beg = wl.chunk_start[chunk];
-  const int end = wl.chunk_start[chunk + 1];
+  const uint32_t beg = wl.chunk_start[chunk], end = wl.chunk_start[chunk + 1];
   int32_t cnt = 0;
   if constexpr (ADAM) cnt = af.count[0];   // issued with the chunk's first loads
   const float* th = theta + (size_t)model * L::P;
@@ -1223,12 +1225,15 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   // each sub-tile's pair indices are loaded two sub-tiles ahead and its point
   // and upstream jets one ahead, so that a sub-tile waits on neither of the
   // two dependent loads; the first ones are issued around the parameter
-  // staging (a chunk is often only one or two sub-tiles)
+  // staging (a chunk is often only one or two sub-tiles).  The selected index
+  // is an int again: as unsigned it took five more registers with one wave per
+  // chunk, [1, 32, 1] (96 -> 101: four waves per SIMD instead of five, inverse step
+  // 51.3 -> 52.1 us)
   int pn, sn;
-  const int k0 = beg + wave * 16 + pl, k1 = k0 + nw * 16;
-  const int p0 = wl.pair_point[k0 < end ? k0 : beg], s0 = wl.pair_seg[k0 < end ? k0 : beg];
-  pn = wl.pair_point[k1 < end ? k1 : beg];
-  sn = wl.pair_seg[k1 < end ? k1 : beg];
+  const uint32_t k0 = beg + wave * 16 + pl, k1 = k0 + nw * 16;
+  const int p0 = wl.pair_point[(int)(k0 < end ? k0 : beg)], s0 = wl.pair_seg[(int)(k0 < end ? k0 : beg)];
+  pn = wl.pair_point[(int)(k1 < end ? k1 : beg)];
+  sn = wl.pair_seg[(int)(k1 < end ? k1 : beg)];
   SmallStage<XD, H, 1, WAVE> st;
   st.load(th);
   float xn[XD], gUn[J];
@@ -1263,7 +1268,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   float dbl = 0.f, small[NS];
 #pragma unroll
   for (int j = 0; j < NS; ++j) small[j] = 0.f;
-  for (int base = beg + wave * 16; base < end; base += nw * 16) {
+  for (uint32_t base = beg + wave * 16; base < end; base += nw * 16) {
     // one wave per chunk: the weights and window tangents are read from LDS
     // per sub-tile rather than held in registers across the loop (95 VGPRs
     // instead of 120 at [1, 32, 1]: five waves per SIMD instead of four)
@@ -1279,13 +1284,13 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
 #pragma unroll
     for (int c = 0; c < J; ++c) gU[c] = gUn[c];
     if (base + nw * 16 < end) {
-      const int kn = base + nw * 16 + pl, k2 = kn + nw * 16;
+      const uint32_t kn = base + nw * 16 + pl, k2 = kn + nw * 16;
 #pragma unroll
       for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
 #pragma unroll
       for (int c = 0; c < J; ++c) gUn[c] = kn < end ? gseg[(size_t)sn * J + c] : 0.f;
-      pn = wl.pair_point[k2 < end ? k2 : beg];
-      sn = wl.pair_seg[k2 < end ? k2 : beg];
+      pn = wl.pair_point[(int)(k2 < end ? k2 : beg)];
+      sn = wl.pair_seg[(int)(k2 < end ? k2 : beg)];
     }
     pair_upstream<S>(gU, xv, box, d.flag, d.usd, gur);
     if (g == 0) dbl += gur[0];
@@ -1472,14 +1477,14 @@ struct GradientMax {
   static constexpr int FIRST = 4;
   int seg[FIRST];
   float m[J];
-  __device__ void indices(const fbpx_worklist& wl, int beg, int end) {
+  __device__ void indices(const fbpx_worklist& wl, uint32_t beg, uint32_t end) {
 #pragma unroll
     for (int j = 0; j < FIRST; ++j) {
-      const int k = beg + (int)threadIdx.x + 256 * j;
+      const uint32_t k = beg + threadIdx.x + 256 * j;
       seg[j] = wl.pair_seg[k < end ? k : beg];   // a repeated pair does not change the maximum
     }
   }
-  __device__ void values(const fbpx_worklist& wl, const float* gseg, int beg, int end) {
+  __device__ void values(const fbpx_worklist& wl, const float* gseg, uint32_t beg, uint32_t end) {
 #pragma unroll
     for (int c = 0; c < J; ++c) m[c] = 0.f;
 #pragma unroll
@@ -1487,7 +1492,7 @@ struct GradientMax {
 #pragma unroll
       for (int c = 0; c < J; ++c) m[c] = fmaxf(m[c], fabsf(gseg[(size_t)seg[j] * J + c]));
 #pragma unroll 4
-    for (int k = beg + (int)threadIdx.x + 256 * FIRST; k < end; k += 256) {
+    for (uint32_t k = beg + threadIdx.x + 256 * FIRST; k < end; k += 256) {
       const int sk = wl.pair_seg[k];
 #pragma unroll
       for (int c = 0; c < J; ++c) m[c] = fmaxf(m[c], fabsf(gseg[(size_t)sk * J + c]));
@@ -1533,8 +1538,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   float* stg = strans + O::TSZ;   // G columns
 
   const int model = wl.chunk_model[chunk];
-  const int beg = wl.chunk_start[chunk];
-  const int end = wl.chunk_start[chunk + 1];
+  const uint32_t beg = wl.chunk_start[chunk], end = wl.chunk_start[chunk + 1];
   const float* th = theta + (size_t)model * L::P;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int pl = lane & 15, g = lane >> 4;
@@ -1542,7 +1546,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // everything that waits
   GradientMax<J> gmax;
   gmax.indices(wl, beg, end);
-  const int k0 = beg + wave * 16 + g * 64 + pl;   // the pair of this lane's first row
+  const uint32_t k0 = beg + wave * 16 + g * 64 + pl;   // the pair of this lane's first row
   const int p0 = wl.pair_point[k0 < end ? k0 : beg], seg0 = wl.pair_seg[k0 < end ? k0 : beg];
   Dom d;
   load_dom(dom, model, d);
@@ -1610,7 +1614,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
   // which its 16-pair sub-tile holds a pair of the chunk.  Lanes past the
   // chunk end carry zero upstream gradient and so contribute nothing.
   const int ntile =
-      O::PRIV ? __builtin_amdgcn_readfirstlane((end - beg - 16 * wave + 63) >> 6) : (end - beg + 63) >> 6;
+      (int)(O::PRIV ? __builtin_amdgcn_readfirstlane((end - beg + (63 - 16 * wave)) >> 6) : (end - beg + 63) >> 6);
   // this lane's row (upstream gradient, normalised point) of the next four
   // tiles.  Their points and upstream jets are fetched during the tile
   // before (indices at the start of its column-0 phase, data before its last
@@ -1832,7 +1836,7 @@ __device__ inline void bwd_two(const float* theta, const float* dom, const float
     // (h = 64 reads in every tile what the fourth uses: a branch here splits the
     // tile's schedule, 78 -> 259 registers spilled, 3,360 -> 10,070 us; below it
     // the branch is the cheaper form)
-    const int kn = beg + ((t | 3) + 1 + g) * 64 + wave * 16 + pl;   // the next row's pair
+    const uint32_t kn = beg + ((uint32_t)(t | 3) + 1 + g) * 64 + wave * 16 + pl;   // the next row's pair
     const bool valid_n = kn < end;
     const bool fetch = !O::PRIV || refill;
     int pn, segn;

@@ -134,8 +134,8 @@ int inside_fill_checked(hipStream_t s, const float* x, int n, int xd, const floa
 __global__ void __launch_bounds__(256) slot_models_kernel(fbpx_worklist wl, int32_t* __restrict__ slot_model) {
   const int chunk = blockIdx.x;
   const int model = wl.chunk_model[chunk];
-  const int beg = wl.chunk_start[chunk], end = wl.chunk_start[chunk + 1];
-  for (int k = beg + threadIdx.x; k < end; k += blockDim.x) slot_model[wl.pair_slot[k]] = model;
+  const uint32_t beg = wl.chunk_start[chunk], end = wl.chunk_start[chunk + 1];
+  for (uint32_t k = beg + threadIdx.x; k < end; k += blockDim.x) slot_model[wl.pair_slot[k]] = model;
 }
 
 // Window jets summed per segment, one thread per point: a segment's pairs are
@@ -277,8 +277,9 @@ __device__ inline void pou_point(const fbpx_worklist& wl, const float* __restric
       U[c] = 0.f;
       W[c] = wsum[(size_t)seg * J + c];
     }
-    const int j0 = wl.seg_pair_start[seg], j1 = wl.seg_pair_start[seg + 1];
-    for (int j = j0; j < j1; j += B) {
+    // unsigned: the last trip passes the end, which may be near int32's
+    const uint32_t j0 = wl.seg_pair_start[seg], j1 = wl.seg_pair_start[seg + 1];
+    for (uint32_t j = j0; j < j1; j += B) {
       float t[B][J];
 #pragma unroll
       for (int b = 0; b < B; ++b) {

@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(64 * kSortWaves) tile_sort_kernel(
   if (b >= nblk) return;
   int32_t* cnt = sort_cnt + w * win;
   const int n_used = info[kInfoUsed];
-  const int p0 = (int)min((int64_t)n, (int64_t)b * tp + w * wave_points), p1 = min(n, p0 + wave_points);
+  const int p0 = (int)min((int64_t)n, (int64_t)b * tp + w * wave_points), p1 = (int)min((int64_t)n, (int64_t)p0 + wave_points);
   const int64_t q0 = off[p0], q1 = off[p1];
   for (int k0 = 0; k0 < (FILL ? n_used : m); k0 += win) {
     for (int k = lane; k < win; k += 64) cnt[k] = 0;
