@@ -669,10 +669,11 @@ struct ResidualArgs {
 constexpr int kResUnroll = 4;
 
 // Threads of a residual workgroup.  Bound by latency and, in the last
-// workgroup's sum, by the workgroups' counts on one address (14 ns each):
-// 262,144 points of three terms take 8.6 us in 256 workgroups of 256 threads,
-// 7.2 in 128 of 512, 7.8 in 64 of 1,024 (11.6 in 256 of 256 with a fence
-// before each count); 68,000 points of a set of two 9.0, 8.5, 9.5 (10.0).
+// workgroup's sum, by the workgroups' counts on one address (14 ns each): with a
+// count that orders nothing, 262,144 points of three terms take 8.6 us in 256
+// workgroups of 256 threads, 7.2 in 128 of 512, 7.8 in 64 of 1,024 (11.6 in 256 of
+// 256 with a fence before each count); 68,000 points of a set of two 9.0, 8.5, 9.5
+// (10.0).  last_arrival's order costs 0.8 us of the 512-thread form.
 constexpr int kResThreads = 512;
 
 // The factor 1 of a term without a second (or any) column is read from here
@@ -681,36 +682,17 @@ constexpr int kResThreads = 512;
 // count would be waited for before the next one is issued).
 __device__ float kResOne[1] = {1.f};
 
-// A workgroup's partials for the grid's last workgroup, without a fence: a
-// device-scope release writes the XCD's whole L2 back, and every workgroup
-// would wait for it.  put_partials (one thread) exchanges the n <= N values
-// in at device scope and waits for the exchanges to return, so that they have
-// been performed before the thread goes on to count its workgroup
-// (last_arrival); the last workgroup, whose own count came after every
-// other's, reads with device-scope loads (get_partial).
-template <int N>
-__device__ inline void put_partials(float* at, const float* v, int n = N) {
-  float old[N];
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-    old[j] = j < n ? __hip_atomic_exchange(at + j, v[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-    asm volatile("" ::"v"(old[j]) : "memory");   // waits for the returned value; keeps the order
-}
-
-__device__ inline float get_partial(const float* at) {
-  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Whether this workgroup is the last of the grid to count itself on done.
-// Every thread of every workgroup calls it, after thread 0 has put the
-// workgroup's partials.
+// Every thread of every workgroup calls it, after thread 0 has written the
+// workgroup's partials: its count releases them and acquires those of the
+// workgroups counted before, and the barrier after it hands them to the last
+// workgroup's other threads.  The ordering lies in the one count; fences around
+// it by the whole workgroup cost 3 us of the 11.6 us Poisson residual.
 __device__ inline bool last_arrival(int32_t* done) {
   __shared__ int last;
   __syncthreads();
   if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
   __syncthreads();
   return last;
 }
@@ -726,7 +708,7 @@ __device__ inline void last_block_sum(const float* scratch, int ncol, float scal
   if (!last_arrival(done)) return;
   for (int j = 0; j < ncol; ++j) {
     float v = 0.f;
-    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) v += get_partial(scratch + b * ncol + j);
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) v += scratch[b * ncol + j];
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) out[j] = acc ? out[j] + scale * t : scale * t;
     __syncthreads();
@@ -892,12 +874,7 @@ __global__ void __launch_bounds__(kResThreads) residual_kernel(int64_t n, Residu
     if (threadIdx.x == 0) loss[0] = acc ? loss[0] + scale * tot : scale * tot;
     return;
   }
-  if (threadIdx.x == 0) {
-    if (done)
-      put_partials<1>(scratch + blockIdx.x, &tot);
-    else
-      scratch[blockIdx.x] = tot;
-  }
+  if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
   if (done) last_block_sum(scratch, 1, scale, loss, acc, done, sm);
 }
 
@@ -930,7 +907,7 @@ __device__ inline void residual_set_sum(const float* scratch, const ResidualSums
   float total = acc ? loss[0] : 0.f;
   for (int i = 0; i < q.n_res; ++i) {
     float v = 0.f;
-    for (int b = q.b0[i] + threadIdx.x; b < q.b0[i + 1]; b += blockDim.x) v += get_partial(scratch + b);
+    for (int b = q.b0[i] + threadIdx.x; b < q.b0[i + 1]; b += blockDim.x) v += scratch[b];
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) total = (i == 0 && !acc) ? q.scale[i] * t : total + q.scale[i] * t;
     __syncthreads();
@@ -962,13 +939,9 @@ __global__ void __launch_bounds__(kResThreads) residual_set_kernel(ResidualSet s
     FBPX_SET_CASE(5) FBPX_SET_CASE(6) FBPX_SET_CASE(7) FBPX_SET_CASE(8)
   }
 #undef FBPX_SET_CASE
-  if (!done) {
-    if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
-    return;
-  }
+  if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
   // the last workgroup to finish sums the partials (as last_block_sum)
-  if (threadIdx.x == 0) put_partials<1>(scratch + blockIdx.x, &tot);
-  if (!last_arrival(done)) return;
+  if (!done || !last_arrival(done)) return;
   residual_set_sum(scratch, s.sums, loss, acc, sm);
   if (threadIdx.x == 0) atomicExch(done, 0);
 }
@@ -1024,13 +997,9 @@ __global__ void __launch_bounds__(kResThreads) residual_backward_kernel(int64_t 
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    if (done && !only) {
-      put_partials<NT>(scratch + blockIdx.x * NT, acc);
-    } else {
-      float* const to = only ? gcoef : scratch + blockIdx.x * NT;
+    float* const to = only ? gcoef : scratch + blockIdx.x * NT;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) to[t] = acc[t];
-    }
+    for (int t = 0; t < NT; ++t) to[t] = acc[t];
   }
   if (done && !only) last_block_sum(scratch, NT, 1.f, gcoef, false, done, sm);
 }
@@ -1121,7 +1090,7 @@ __device__ inline void pou_loss_total(const float* part, int nb, const PouLossAr
   float total = 0.f;   // thread 0's
   for (int i = 0; i < a.n_res; ++i) {
     float v = 0.f;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) v += get_partial(part + b * a.n_res + i);
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) v += part[b * a.n_res + i];
     const float t = block_tree_sum(v, sm);
     if (threadIdx.x == 0) {
       const float term = a.scale[i] * t;
@@ -1273,13 +1242,9 @@ __global__ void __launch_bounds__(256) pou_loss_kernel(fbpx_worklist wl, const f
     return;
   }
   if (threadIdx.x == 0) {
-    if (done) {
-      put_partials<NR>(part + blockIdx.x * a.n_res, tot, a.n_res);
-    } else {
 #pragma unroll
-      for (int i = 0; i < NR; ++i)
-        if (i < a.n_res) part[blockIdx.x * a.n_res + i] = tot[i];
-    }
+    for (int i = 0; i < NR; ++i)
+      if (i < a.n_res) part[blockIdx.x * a.n_res + i] = tot[i];
   }
   if (done && last_arrival(done)) {
     pou_loss_total(part, gridDim.x, a, loss, acc, sm);
