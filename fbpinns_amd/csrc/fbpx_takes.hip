@@ -21,15 +21,16 @@
 //            gives each pair its slot.
 //   tiles    pairs grouped by model position, ascending point within: a
 //            stable counting sort of the point-major pairs by model position.
-//            Each workgroup takes the pairs of 1024 points, counts them per
-//            model in LDS, one exclusive scan in (model, block) order gives
+//            Each workgroup takes the pairs of tile_points(m) points, counts
+//            them per model in LDS, one exclusive scan in (model, block) order gives
 //            every block's place in every model, and a fill pass writes the
 //            pairs there in order (tile_sort_kernel).
 //   chunks   cut flags at every model start, every `chunk` pairs inside a
 //            model and at both kernels' bin edges (round(linspace) over the
 //            pairs, numpy's half-to-even rounding), compacted by a scan.
-// All sums are exclusive scans with a fixed order; no atomics except the
-// idempotent "used" flags, so the result is a function of the input alone.
+// All sums are exclusive scans with a fixed order; the only atomics are
+// order-independent (the "used" flags, the sort's integer counts in LDS), so the
+// result is a function of the input alone.
 #include <algorithm>
 
 #include "fbpx_common.hpp"
