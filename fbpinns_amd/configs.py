@@ -146,18 +146,23 @@ def fwd_flops_per_pair(xd, h, nh, J):
     return f
 
 
-# matrix-core FLOPs the kernels execute per (point, subdomain) pair: the
-# layer-2 contractions run as passes over 16 pairs, each product of 2 * h * h *
-# 16 FLOPs as three f16 products (hi hi, hi lo, lo hi).  Forward: Z_0,
-# the W2^T vector when any first derivative is carried, one Z_i per axis with
-# a second derivative.  Backward: Z_0; with first derivatives the s-vector
-# pass, its W2^T pass and its dW2 column; per second-derivative axis Z_i, its
-# W2^T pass and dW2 column; W2^T G_0 and the G_0 column.  One hidden layer:
-# no matrix-core work.
+# matrix-core FLOPs the kernels execute per (point, subdomain) pair.  A
+# contraction of 2 h h FLOPs per pair runs as several f16 ones:
+#   passes over the weights (frag_pass): hi hi, hi lo and lo hi; at h = 16 three
+#     instructions of twice the contraction (hi and lo weights side by side
+#     against lo and against hi, the weights' rests against hi and zeros): six;
+#   dW2 columns: hi hi, hi lo and lo hi at h = 64; below it two instructions of
+#     twice the contraction (dw2_private): four.
+# Forward: Z_0, the W2^T vector when any first derivative is carried, one Z_i
+# per axis with a second derivative.  Backward: Z_0, W2^T G_0 and the G_0 column;
+# with first derivatives the s-vector pass, its W2^T pass and its dW2 column;
+# per second-derivative axis Z_i, its W2^T pass and dW2 column.  One hidden
+# layer: no matrix-core work.
 def mfma_flops_per_pair(h, nh, n1, n2):
     if nh != 2:
         return 0, 0
-    per_pass = 3 * 2 * h * h
-    fwd = (1 + (n1 > 0) + n2) * per_pass
-    bwd = (3 + 3 * (n1 > 0) + 3 * n2) * per_pass
+    product = 2 * h * h
+    frag, dw2 = (6 if h == 16 else 3) * product, (3 if h == 64 else 4) * product
+    fwd = (1 + (n1 > 0) + n2) * frag
+    bwd = (1 + (n1 > 0) + n2) * (2 * frag + dw2)
     return fwd, bwd
