@@ -1309,6 +1309,17 @@ int fbpx_pou_prepare(void* stream, const fbpx_net* net, const float* dom, const 
                      float* pair_scratch, float* wsum) {
   int J, rc;
   if ((rc = check_net_schema(net, &J)) || (rc = check_wl(wl))) return rc;
+  // the sums run per point over its segments: without them nothing would be
+  // written, or a null pointer read on the device
+  if (wl->n_segs > 0 && (wl->n_points == 0 || !dom || !x || !pair_scratch || !wsum || !wl->point_seg_start ||
+                         !wl->seg_pair_start)) {
+    set_error("pou_prepare: %d segments of %d points, or a null pointer", wl->n_segs, wl->n_points);
+    return FBPX_EINVAL;
+  }
+  if (wl->n_chunks > 0 && (!pair_scratch || !wl->chunk_model || !wl->chunk_start || !wl->pair_slot)) {
+    set_error("pou_prepare: null chunk or slot array");
+    return FBPX_EINVAL;
+  }
   hipStream_t s = (hipStream_t)stream;
   int32_t* slot_model = reinterpret_cast<int32_t*>(pair_scratch);
   if (wl->n_chunks > 0)
