@@ -172,8 +172,8 @@ def _op(name, mutates_args):
     four times the body's.  Whatever interposes on operators sees the custom
     op as before: compilation, tracing, profiling, dispatch and function modes,
     functorch transforms, forward-mode levels, inference mode, tensor
-    subclasses, arguments that require a gradient and arguments that the
-    schema converts or refuses.  (An
+    subclasses, arguments that require a gradient, arguments that the schema
+    converts or refuses, and whatever is registered on it.  (An
     ExecutionTraceObserver outside a profiler cannot be asked for and does not
     see direct calls.)"""
     def deco(fn):
@@ -182,10 +182,11 @@ def _op(name, mutates_args):
         required = sum(p.default is inspect.Parameter.empty for p in params)
         kinds = [_KINDS[p.annotation] for p in params]
         mutated = [i for i, p in enumerate(params) if p.name in mutates_args]
+        registered = []   # what a program registers on the operator itself
 
         @functools.wraps(fn)
         def call(*args, **kwargs):
-            if kwargs or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() \
+            if kwargs or registered or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() \
                     or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None \
                     or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0 \
                     or torch.is_inference_mode_enabled() or torch._C._autograd._profiler_enabled() \
@@ -206,6 +207,14 @@ def _op(name, mutates_args):
             fn(*args)
             for i in mutated:
                 torch.autograd.graph.increment_version(args[i])
+        def through(method):
+            def register(*args, **kwargs):
+                registered.append(method)   # direct calls would pass it by
+                return getattr(op, method)(*args, **kwargs)
+            return register
+        for m in dir(op):
+            if not m.startswith("_"):   # register_kernel, register_autograd, set_kernel_enabled, ...
+                setattr(call, m, through(m))
         call.custom_op = op
         return call
     return deco

@@ -229,3 +229,22 @@ def test_versions():
     args = _args()
     axpy(*args)
     assert args[6]._version == 1
+
+
+def test_registrations():
+    """The operator's own methods are there, and what they register is used."""
+    @ops._op("fbpx_test::fill", mutates_args=("out",))
+    def fill(out: torch.Tensor) -> None:
+        out.fill_(1.0)
+    out = torch.zeros(2)
+    fill(out)
+    assert out.tolist() == [1.0, 1.0]
+
+    @fill.register_kernel("cpu")
+    def _(out):
+        out.fill_(2.0)
+    fill(out)
+    assert out.tolist() == [2.0, 2.0]
+    with fill.set_kernel_enabled("cpu", False):
+        fill(out)
+    assert out.tolist() == [1.0, 1.0]
