@@ -14,6 +14,7 @@ kernel (activation recompute) + deterministic per-subdomain row reduction.
 import ctypes
 import functools
 import inspect
+import operator
 from typing import List, Optional
 
 import torch
@@ -161,7 +162,16 @@ def _is_plain(v):
 _TENSOR, _OPTIONAL, _TENSORS, _INTS = "tensor", "optional", "tensors", "ints"
 _KINDS = {torch.Tensor: _TENSOR, Optional[torch.Tensor]: _OPTIONAL, List[torch.Tensor]: _TENSORS, List[int]: _INTS,
           int: int, float: float, bool: bool}
-_INT_ONLY = frozenset((int,))
+_INT_ONLY, _TENSOR_ONLY, _INT32_ONLY = frozenset((int,)), frozenset((torch.Tensor,)), frozenset((torch.int32,))
+_dtype = operator.attrgetter("dtype")
+
+
+def _are_plain(v, mutated):
+    """_is_plain of a list's tensors; int32 tensors that are only read (work
+    lists) may be inference tensors too."""
+    if type(v) is not list or not _TENSOR_ONLY.issuperset(map(type, v)):
+        return False
+    return not mutated and _INT32_ONLY.issuperset(map(_dtype, v)) or all(map(_is_plain, v))
 
 
 def _op(name, mutates_args):
@@ -180,7 +190,7 @@ def _op(name, mutates_args):
         op = torch.library.custom_op(name, fn, mutates_args=mutates_args)
         params = list(inspect.signature(fn).parameters.values())
         required = sum(p.default is inspect.Parameter.empty for p in params)
-        kinds = [_KINDS[p.annotation] for p in params]
+        kinds = [(_KINDS[p.annotation], p.name in mutates_args) for p in params]
         mutated = [i for i, p in enumerate(params) if p.name in mutates_args]
         registered = []   # what a program registers on the operator itself
 
@@ -192,15 +202,18 @@ def _op(name, mutates_args):
                     or torch.is_inference_mode_enabled() or torch._C._autograd._profiler_enabled() \
                     or not required <= len(args) <= len(params):
                 return op(*args, **kwargs)
-            for k, v in zip(kinds, args):
-                if k is _TENSOR or k is _OPTIONAL:
-                    if not _is_plain(v) and not (k is _OPTIONAL and v is None):
-                        return op(*args)
-                elif k is _TENSORS:
-                    if type(v) is not list or not all(_is_plain(t) for t in v):
+            for (k, written), v in zip(kinds, args):
+                if k is _TENSOR:
+                    if not _is_plain(v):
                         return op(*args)
                 elif k is _INTS:
                     if type(v) is not list or not _INT_ONLY.issuperset(map(type, v)):
+                        return op(*args)
+                elif k is _TENSORS:
+                    if not _are_plain(v, written):
+                        return op(*args)
+                elif k is _OPTIONAL:
+                    if v is not None and not _is_plain(v):
                         return op(*args)
                 elif type(v) is not k:
                     return op(*args)
