@@ -1206,6 +1206,11 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   using T = Team<WAVE>;
   constexpr int J = S::J, NRB = H / 16, NS = 2 + XD, NT = WAVE ? 4 : 1;
   constexpr int K_WL = 0, K_B1 = 1, K_W1 = 2;
+  // (with 64 units and six or seven jets in a workgroup the values ahead spill
+  // inside the loop: point and jets are then read where they are used, pair
+  // indices one sub-tile ahead.  [3,64,1], 3.4 million pairs: seven jets 854 ->
+  // 681 us, six 652 -> 534; 690 and 577 before either)
+  constexpr bool AHEAD = H < 64 || J < 6 || WAVE;
   __shared__ float ss_[NT][SM::N];
   __shared__ float ssmall_[4 * NS * H];   // per wave (four teams of one wave with WAVE)
   __shared__ float sbl_[4];
@@ -1232,15 +1237,22 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
   int pn, sn;
   const uint32_t k0 = beg + wave * 16 + pl, k1 = k0 + nw * 16;
   const int p0 = wl.pair_point[(int)(k0 < end ? k0 : beg)], s0 = wl.pair_seg[(int)(k0 < end ? k0 : beg)];
-  pn = wl.pair_point[(int)(k1 < end ? k1 : beg)];
-  sn = wl.pair_seg[(int)(k1 < end ? k1 : beg)];
+  if constexpr (AHEAD) {
+    pn = wl.pair_point[(int)(k1 < end ? k1 : beg)];
+    sn = wl.pair_seg[(int)(k1 < end ? k1 : beg)];
+  } else {
+    pn = p0;
+    sn = s0;
+  }
   SmallStage<XD, H, 1, WAVE> st;
   st.load(th);
   float xn[XD], gUn[J];
+  if constexpr (AHEAD) {
 #pragma unroll
-  for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
+    for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)p0 * XD + i];
 #pragma unroll
-  for (int c = 0; c < J; ++c) gUn[c] = k0 < end ? gseg[(size_t)s0 * J + c] : 0.f;
+    for (int c = 0; c < J; ++c) gUn[c] = k0 < end ? gseg[(size_t)s0 * J + c] : 0.f;
+  }
   st.store(ss);
   // the row's first T::size() parameters for the update at the chunk's end
   // (one round trip less in a step of 200 points: 21.75 -> 21.5 us)
@@ -1274,6 +1286,15 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
     // instead of 120 at [1, 32, 1]: five waves per SIMD instead of four)
     if constexpr (WAVE) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     // lanes past the end run the pair at beg with a zero upstream gradient
+    if constexpr (!AHEAD) {
+      const uint32_t k = base + pl, k1 = k + nw * 16;
+#pragma unroll
+      for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];
+#pragma unroll
+      for (int c = 0; c < J; ++c) gUn[c] = k < end ? gseg[(size_t)sn * J + c] : 0.f;
+      pn = wl.pair_point[(int)(k1 < end ? k1 : beg)];
+      sn = wl.pair_seg[(int)(k1 < end ? k1 : beg)];
+    }
     float xv[XD], xh[XD];
 #pragma unroll
     for (int i = 0; i < XD; ++i) {
@@ -1283,7 +1304,7 @@ __device__ inline void bwd_one(const float* theta, const float* dom, const float
     float gur[J], gU[J];
 #pragma unroll
     for (int c = 0; c < J; ++c) gU[c] = gUn[c];
-    if (base + nw * 16 < end) {
+    if (AHEAD && base + nw * 16 < end) {
       const uint32_t kn = base + nw * 16 + pl, k2 = kn + nw * 16;
 #pragma unroll
       for (int i = 0; i < XD; ++i) xn[i] = x[(size_t)pn * XD + i];

@@ -1,4 +1,4 @@
-"""The two-layer kernels against the float64 oracle with chunks of many tiles, so
+"""The jet kernels against the float64 oracle with chunks of many tiles, so
 that what a wave carries from tile to tile is checked too: the pair rows and
 their refills, the loads ahead, the sums of dW2 and of the per-unit and bias
 gradients and their changes of sign.  Point counts leave a last tile of every
@@ -18,7 +18,10 @@ pytestmark = pytest.mark.gpu
 
 NETS = [([1, 16, 16, 1], (1, 1)), ([2, 16, 16, 1], (3, 1)), ([3, 16, 16, 1], (7, 7)), ([2, 32, 32, 1], (3, 3)),
         ([3, 32, 32, 1], (7, 3)), ([2, 32, 32, 1], (0, 0)), ([2, 64, 64, 1], (3, 1)), ([3, 64, 64, 1], (7, 7)),
-        ([3, 64, 64, 1], (7, 0)), ([2, 64, 64, 1], (0, 0))]
+        ([3, 64, 64, 1], (7, 0)), ([2, 64, 64, 1], (0, 0)),
+        # one hidden layer: loads one sub-tile ahead, or (64 units, six or seven jets) where they are used
+        ([1, 16, 1], (1, 1)), ([2, 32, 1], (3, 3)), ([2, 64, 1], (3, 3)), ([3, 64, 1], (7, 0)), ([3, 64, 1], (7, 3)),
+        ([3, 64, 1], (7, 7))]
 
 
 @pytest.mark.parametrize("n", [450, 577, 1100])
