@@ -248,3 +248,21 @@ def test_registrations():
     with fill.set_kernel_enabled("cpu", False):
         fill(out)
     assert out.tolist() == [1.0, 1.0]
+
+
+def test_compilation_sees_the_operator():
+    graphs = []
+
+    def backend(gm, example_inputs):
+        graphs.append(gm.code)
+        return gm.forward
+
+    def f(x, out):
+        axpy(x, [x], [1], 2, 1.5, False, out)
+        return out + 1
+    x, out = torch.ones(3), torch.zeros(3)
+    got = torch.compile(f, backend=backend, fullgraph=True)(x, out)
+    assert len(graphs) == 1 and "axpy" in graphs[0]
+    want = torch.zeros(3)
+    axpy.custom_op(x, [x], [1], 2, 1.5, False, want)
+    assert torch.equal(got, want + 1)
